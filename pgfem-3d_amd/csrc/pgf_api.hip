@@ -251,8 +251,13 @@ struct pgf_handle_s {
   GraphKey gkey{};
   int32_t glaunches = 0;
   // linear solve
-  int32_t *d_Ap = nullptr, *d_Ai = nullptr;
+  int32_t *d_Ai = nullptr;
+  int4 *d_rows = nullptr;  // the linear solve's row groups (pgf::RowGroups)
+  int32_t *d_row_range = nullptr;
+  int n_ranges = 0;
   double *d_solve_work = nullptr;
+  pgf::SolveStatus *solve_status = nullptr;  // pinned host memory
+  hipEvent_t solve_ev[2] = {nullptr, nullptr};
   // interface elements
   std::vector<pgf::CohBlock> cblocks;
   int32_t n_ccolors = 0;
@@ -1032,8 +1037,36 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
   if ((rc = pgf::upload(&h->d_dofid, dofid.data(), dofid.size()))) return fail(rc);
   if ((rc = pgf::upload(&h->d_row_start, row_start.data(), row_start.size()))) return fail(rc);
   if ((rc = pgf::upload(&h->d_rowlen, rowlen.data(), rowlen.size()))) return fail(rc);
-  if ((rc = pgf::upload(&h->d_Ap, Ap, size_t(ndof) + 1))) return fail(rc);
   if ((rc = pgf::upload(&h->d_Ai, Ai, size_t(h->nnz)))) return fail(rc);
+  {  // row groups of the linear solve, in row order
+    std::vector<uint8_t> cnt(size_t(ndof), 1);
+    for (int64_t n = 0; n < m.n_nodes; ++n) {
+      int64_t first = -1;
+      uint8_t k = 0;
+      for (int j = 0; j < 3; ++j)
+        if (dofid[n * 3 + j] > 0) {
+          if (first < 0) first = dofid[n * 3 + j] - 1;
+          ++k;
+        }
+      if (first >= 0) cnt[first] = k;
+    }
+    std::vector<int4> rows;
+    std::vector<int32_t> range;
+    rows.reserve(size_t(m.n_nodes));
+    for (int64_t d = 0; d < ndof;) {
+      const int64_t end = d + cnt[d];
+      while (d < end) {  // a node's rows; a range's end cuts them
+        const int64_t cut = std::min(end, (d / pgf::kRowRange + 1) * pgf::kRowRange);
+        if (d % pgf::kRowRange == 0) range.push_back(int32_t(rows.size()));
+        rows.push_back(make_int4(int(d), int(cut - d), Ap[d], Ap[d + 1] - Ap[d]));
+        d = cut;
+      }
+    }
+    h->n_ranges = int(range.size());
+    range.push_back(int32_t(rows.size()));
+    if ((rc = pgf::upload(&h->d_rows, rows.data(), rows.size()))) return fail(rc);
+    if ((rc = pgf::upload(&h->d_row_range, range.data(), range.size()))) return fail(rc);
+  }
   for (size_t bi = 0; bi < h->blocks.size(); ++bi) {
     Block &b = h->blocks[bi];
     std::vector<int32_t> mat(b.ne);
@@ -1142,9 +1175,13 @@ int pgf_destroy(pgf_handle h) {
   hipFree(h->d_tf);
   hipFree(h->d_tfbuf);
   if (h->gexec) hipGraphExecDestroy(h->gexec);
-  hipFree(h->d_Ap);
   hipFree(h->d_Ai);
+  hipFree(h->d_rows);
+  hipFree(h->d_row_range);
   hipFree(h->d_solve_work);
+  if (h->solve_status) hipHostFree(h->solve_status);
+  for (hipEvent_t e : h->solve_ev)
+    if (e) hipEventDestroy(e);
   hipFree(h->d_cprops);
   hipFree(h->d_cpmat);
   hipFree(h->d_grains);
@@ -1780,15 +1817,22 @@ int pgf_solve(pgf_handle h, const double *vals, const double *b, double *x, doub
               int32_t *iters, double *relres) {
   if (!h || !vals || !b || !x || !(tol > 0.0) || maxit < 1) return PGF_EINVAL;
   const int64_t n = h->ndof;
+  if (!h->solve_status &&
+      hipHostMalloc(reinterpret_cast<void **>(&h->solve_status), sizeof(pgf::SolveStatus)) != hipSuccess) {
+    h->solve_status = nullptr;
+    return PGF_ENOMEM;
+  }
+  for (hipEvent_t &e : h->solve_ev)
+    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return PGF_EHIP;
   if (!h->d_solve_work) {
-    int rc = pgf::dalloc(&h->d_solve_work, size_t(9 * n + 1025));
+    int rc = pgf::dalloc(&h->d_solve_work, size_t(pgf::solve_work_doubles(n)));
     if (rc) return rc;
   }
   int it = 0;
   double rr = 0.0;
-  if (pgf::bicgstab(h->stream, h->d_Ap, h->d_Ai, vals, b, x, n, tol, maxit, &it, &rr, h->d_solve_work))
+  if (pgf::bicgstab(h->stream, {h->d_rows, h->d_row_range, h->n_ranges}, h->d_Ai, vals, b, x, n, tol, maxit, &it, &rr,
+                    h->d_solve_work, h->solve_status, h->solve_ev))
     return PGF_EHIP;
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
   if (iters) *iters = it;
   if (relres) *relres = rr;
   return (rr <= tol) ? PGF_OK : 1;  // 1 = not converged within maxit

@@ -280,9 +280,24 @@ int gather_waves(int32_t maxlen);
 // waves: nodes per workgroup (capped by the LDS each node needs); batch: staging blocks each
 // half-wave keeps in flight (2, 4 or 8)
 void launch_gather(int mode, const GatherArgs &g, int waves, int batch, hipStream_t s);
-// Jacobi-preconditioned BiCGStab on a CSR matrix; work holds 9 n + 1025 doubles.
-int bicgstab(hipStream_t s, const int32_t *Ap, const int32_t *Ai, const double *vals, const double *b, double *x,
-             int64_t n, double tol, int maxit, int *iters, double *relres, double *work);
+// The CSR rows in groups of up to three with the same columns (a node's free DOFs), cut at
+// multiples of 256 rows: group g is rows [x, x + y) from entry z on, w columns each; rows
+// [256 k, 256 (k + 1)) are groups [range[k], range[k + 1]).
+struct RowGroups {
+  const int4 *groups;
+  const int32_t *range;
+  int n_ranges;
+};
+constexpr int kRowRange = 256;
+struct SolveStatus {  // pinned host memory, written by the kernel that decides the stop
+  volatile int32_t done, it;
+  volatile double res;
+};
+// Jacobi-preconditioned BiCGStab; work holds solve_work_doubles(n), ev two events.
+int64_t solve_work_doubles(int64_t n);
+int bicgstab(hipStream_t s, const RowGroups &rows, const int32_t *Ai, const double *vals, const double *b, double *x,
+             int64_t n, double tol, int maxit, int *iters, double *relres, double *work, SolveStatus *status,
+             hipEvent_t *ev);
 
 void launch_tf_update(int nne, const TfArgs &t, hipStream_t s);
 void launch_tf_initial(int nne, const TfArgs &t, hipStream_t s);
