@@ -118,10 +118,6 @@ void make_grain(const double *R, double C11, double C12, double C44, DevGrain &g
     }
     for (int i = 0; i < 3; ++i)
       for (int j = 0; j < 3; ++j) g.P[a][i * 3 + j] = s[i] * m[j];
-    for (int i = 0; i < 3; ++i) {
-      g.s[a][i] = s[i];
-      g.m[a / 3][i] = m[i];  // the same for the plane's three systems
-    }
   }
   auto L0 = [&](int i, int j, int k, int l) {
     double v = 0.0;
@@ -130,9 +126,6 @@ void make_grain(const double *R, double C11, double C12, double C44, DevGrain &g
     return v;
   };
   for (int i = 0; i < 9; ++i) g.R[i] = R[i];
-  g.cub[0] = C11 - C12;
-  g.cub[1] = C12;
-  g.cub[2] = 2.0 * C44;
   static const int vi[6] = {0, 1, 2, 0, 1, 0}, vj[6] = {0, 1, 2, 1, 2, 2};
   for (int I = 0; I < 6; ++I)
     for (int J = 0; J < 6; ++J) {
@@ -231,6 +224,7 @@ struct pgf_handle_s {
   const double *warm = nullptr;
   double cp_g0 = 0.0, dt = 1.0;
   int32_t cp_law = 0;  // elastic law of the crystal-plasticity material (pgf_material.cp_elastic)
+  int32_t cp_flow = 0;  // what its flow and hardening rule need pow for (pgf::CPArgs::flow)
   int64_t cp_nq = 0;         // crystal-plasticity QPs: device QPs [0, cp_nq)
   int64_t cp_chunk = 256;    // QPs per wave range of the local-Newton work queue (autotuned; 1:
                              // every wave draws from one global queue)
@@ -344,6 +338,7 @@ pgf::CPArgs cp_args(pgf_handle h, const Block &b, const pgf_nodal_input *in) {
   c.qpbuf = h->d_qpbuf;  // indexed by device QP (pgf::qrec)
   c.err = h->d_err;
   c.law = h->cp_law;
+  c.flow = h->cp_flow;
   if (h->tf && b.ne > 0 && b.model == PGF_MODEL_CRYSTAL_PLASTICITY) {  // CM3F: the kinematics scales F
     c.tf_V = h->d_tf + b.e_base;
     c.tf_dV = h->d_tf + 6 * h->n_elem + b.e_base;
@@ -1102,6 +1097,9 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     c.w = cpm.w_sat;
     c.tol = cpm.tol_M > 0.0 ? cpm.tol_M : 1.0e-10;
     c.maxit = cpm.max_itr_M > 0 ? cpm.max_itr_M : 50;
+    c.c11m12 = cpm.C11 - cpm.C12;
+    c.c12 = cpm.C12;
+    c.c44x2 = 2.0 * cpm.C44;
     c.m10 = cpm.m10;
     c.kappa = cpm.E / (3.0 * (1.0 - 2.0 * cpm.nu));
     c.law = cpm.cp_elastic;
@@ -1109,10 +1107,13 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     {
       // the flow rule's exponent, evaluated as the kernels do
       const double e = 1.0 / c.m - 1.0;
+      c.expo = e;
+      c.gd0_m = c.gd0 / c.m;
       c.ipow = (e >= 0.0 && e <= 64.0 && e == std::floor(e)) ? int32_t(e) : -1;
     }
     h->cp_g0 = cpm.g0;
     h->cp_law = cpm.cp_elastic;
+    h->cp_flow = c.ipow < 0 ? 0 : (c.w != 0.0 ? 1 : 2);
     h->cp_mat_host = {cpm.C11, cpm.C12, cpm.C44};
     if ((rc = pgf::upload(&h->d_cpmat, &c, 1))) return fail(rc);
     for (int t = 0; t < 2; ++t) {

@@ -18,14 +18,14 @@
 // below tol.  The 11x11 system is
 // solved through the Schur complement of its (M, M) block: with the bordered structure
 //   [A b c; d^T 0 0; e^T 0 f]
-// one 9x9 LU (register-resident, pivoting by predicated row swaps so nothing is indexed at
-// run time) serves the two right-hand sides of a Newton step and the nine of the tangent.
+// one 9x9 elimination (in registers, unpivoted; the rare matrix that needs pivoting is solved
+// again in scratch memory) serves the two right-hand sides of a Newton step, and a 6x6 one the
+// nine columns of the tangent.  All of it runs in the crystal frame (see below).
 //
 // Kernels:
 //   cp_kinematics  F(n+1) at every QP of a block (gather of the element nodes)
 //   cp_start_kernel  the starting points (and the choice of a caller's start), one per lane
-//   cp_newton      persistent: each wave owns a QP range; a lane that converges takes the
-//                  next QP of its wave at once, so uneven iteration counts do not idle lanes
+//   cp_newton      persistent: each wave works through a QP range, 64 QPs at a time
 //   cp_tangent     at the converged state: S, tau, gdot and dMe/dF (Me = pF(n+1)^-1), for the
 //                  element kernel (qpbuf)
 //   cp_elem        coloured element rows: the reference contraction (compute_stiffness_matrix,
@@ -37,6 +37,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "pgf_device.h"
 #include "pgf_math.h"
@@ -64,6 +65,12 @@ __device__ __forceinline__ void mtm3(const double *A, const double *B, double *C
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) C[i * 3 + j] = A[i] * B[j] + A[3 + i] * B[3 + j] + A[6 + i] * B[6 + j];
+}
+__device__ __forceinline__ void mmt3(const double *A, const double *B, double *C) {  // A B^T
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) C[i * 3 + j] = A[i * 3] * B[j * 3] + A[i * 3 + 1] * B[j * 3 + 1] + A[i * 3 + 2] * B[j * 3 + 2];
 }
 // S (Voigt tensor comps) = Lv : E, E symmetric 3x3 given as full 3x3
 __device__ __forceinline__ void lv_dot(const double *Lv, const double *E9, double *S6) {
@@ -184,348 +191,487 @@ __device__ __forceinline__ void he_dot(const HeTan &t, const double *X9, double 
   }
 }
 
-// A pointer whose value the compiler cannot see through: loads from it are not hoisted out of
-// loops or merged with earlier loads from the same address, so the data is read from cache
-// where it is used instead of being held in registers across a long stretch of code.
-__device__ __forceinline__ const double *opaque(const double *p) {
-  asm volatile("" : "+v"(p));
-  return p;
+// The stages of the local solve each fit the registers, their overlap does not.  pin makes a
+// stage's results due at its end (in program order with the other asm), end_stage keeps the
+// scheduler from mixing stages, and reload gives the lane's LDS slots under an index the
+// compiler cannot see through, so that what is read after it is read from LDS, not kept.
+__device__ __forceinline__ void end_stage() { __builtin_amdgcn_sched_barrier(0); }
+template <int N>
+__device__ __forceinline__ void pin(double (&x)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+}
+__device__ __forceinline__ double *reload(double *slots, int lane) {
+  asm volatile("" : "+v"(lane));
+  return slots + lane;
 }
 
-// Elastic PK2 from eF and Ce = eF^T eF: law 0 is S = Lv : (Ce - I)/2 with the grain's cubic
-// stiffness; law 1 is he_law, which also fills the tangent coefficients.
-template <bool HE>
-__device__ __forceinline__ void el_stress(const CPMaterial &cm, const DevGrain &gr, const double *eF,
-                                          const double *Ce, double *S6, HeTan &t) {
-  if constexpr (HE) {
-    he_law(cm, eF, Ce, S6, t);
-  } else {
-    double E[9];
+// ------------------------------------------------------------------- the local solve
+// The return map runs in the crystal frame: M, A = F pF(n)^-1 and the stress are rotated once per
+// point (X' = R^T X R), and every quantity of the residual but the frame is rotation invariant.
+// There the twelve Schmid tensors are P_a = kR6 s_a (x) n_k with entries of s and n in {0, +1, -1},
+// so contractions with them are sums, and the cubic stiffness is three constants; nothing of the
+// grain but R is read.  In the sample frame a system took about 260 operations of a Newton
+// iteration's Jacobian, here about 60, and the slip directions, plane normals and the stiffness's
+// frame were 72 doubles of the register file.
+constexpr double kR6 = 0.40824829046386301637;  // 1 / sqrt(6)
+// plane k's normal (1, 1, 1), with component k - 1 negative for k = 1, 2, 3
+__device__ constexpr int n_sign(int k, int j) { return k == j + 1 ? -1 : 1; }
+// slip direction of system a: the order of make_grain's table
+__device__ constexpr int s_sign(int a, int i) {
+  constexpr int t[12][3] = {{0, 1, -1}, {-1, 0, 1}, {1, -1, 0}, {0, 1, -1}, {1, 0, 1}, {1, 1, 0},
+                            {0, 1, 1},  {1, 0, -1}, {1, 1, 0},  {0, 1, 1},  {1, 0, 1}, {1, -1, 0}};
+  return t[a][i];
+}
+// +v, -v by a sign known at compile time (folds into the add that uses it)
+__device__ __forceinline__ double pm(int s, double v) { return s > 0 ? v : -v; }
+// s_a . x: the two components of system a's direction
+__device__ __forceinline__ double s_dot(int a, const double *x) {
+  return a % 3 == 0   ? x[1] + pm(s_sign(a, 2), x[2])
+         : a % 3 == 1 ? pm(s_sign(a, 0), x[0]) + pm(s_sign(a, 2), x[2])
+                      : x[0] + pm(s_sign(a, 1), x[1]);
+}
+__device__ __forceinline__ double n_dot(int k, double x0, double x1, double x2) {
+  return (pm(n_sign(k, 0), x0) + pm(n_sign(k, 1), x1)) + pm(n_sign(k, 2), x2);
+}
+// y += s_a v (y of three, v known per system)
+__device__ __forceinline__ void s_add(int a, double v, double *y) {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) E[i] = 0.5 * (Ce[i] - ((i % 4 == 0) ? 1.0 : 0.0));
-    cubic_dot(gr.R, gr.cub, E, S6);
-  }
-}
-// L : X at the state el_stress was evaluated at
-template <bool HE>
-__device__ __forceinline__ void el_dot(const DevGrain &gr, const HeTan &t, const double *X9, double *out6) {
-  if constexpr (HE) he_dot(t, X9, out6);
-  else lv_dot(gr.Lv, X9, out6);
-}
-
-// |r|^e of the power-law flow rule, e = 1/m - 1.  When e is a whole number (ie >= 0; the rate
-// sensitivity m = 0.05 gives 19) it is formed by binary powering, a handful of multiplies where
-// pow takes about 130 FP64 operations; the two agree to a few ulps.  ie is the same for every
-// lane, so the branch does not diverge.
-__device__ __forceinline__ double flow_pow(double x, double e, int ie) {
-  if (ie >= 0) {
-    double r = 1.0, b = x;
-    for (int k = ie; k; k >>= 1) {
-      if (k & 1) r *= b;
-      b *= b;
-    }
-    return r;
-  }
-  return pow(x, e);
+  for (int i = 0; i < 3; ++i)
+    if (s_sign(a, i) != 0) y[i] += pm(s_sign(a, i), v);
 }
 
-// The resolved shear stress X : P_a with the Schmid tensor in its factored form P_a = s_a (x) m_a:
-// s_a . (X m_a).  The kernels of the local solve keep the 6 numbers of each system's s and m
-// rather than the 9 of P_a: 72 doubles of the grain instead of 108 in the registers.
-__device__ __forceinline__ double resolved(const DevGrain &gr, int a, const double *X) {
-  const double *s = gr.s[a], *m = gr.m[a / 3];
-  double t = 0.0;
+// 3x3 products and inverse with explicit multiply-adds: what a residual pass and a fused pass
+// both compute has the same bits in either kernel.
+__device__ __forceinline__ void mul_ab(const double *A, const double *B, double *C) {
 #pragma unroll
-  for (int i = 0; i < 3; ++i) t += s[i] * (X[i * 3 + 0] * m[0] + X[i * 3 + 1] * m[1] + X[i * 3 + 2] * m[2]);
-  return t;
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) C[i * 3 + j] = fma3(A[i * 3], B[j], A[i * 3 + 1], B[3 + j], A[i * 3 + 2], B[6 + j]);
 }
-
-// 9x9 LU with partial pivoting; row swaps are predicated so every index is static.
-__device__ __forceinline__ bool lu9(double (&A)[81], int (&piv)[9]) {
+__device__ __forceinline__ void mul_atb(const double *A, const double *B, double *C) {
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    int p = k;
-    double amax = fabs(A[k * 9 + k]);
+  for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int i = k + 1; i < 9; ++i) {
-      const double v = fabs(A[i * 9 + k]);
-      if (v > amax) {
-        amax = v;
-        p = i;
-      }
-    }
-    if (!(amax > 0.0)) return false;
-    piv[k] = p;
-#pragma unroll
-    for (int i = k + 1; i < 9; ++i) {
-      const bool sw = (i == p);
-#pragma unroll
-      for (int j = 0; j < 9; ++j) {
-        const double t = A[k * 9 + j];
-        A[k * 9 + j] = sw ? A[i * 9 + j] : t;
-        A[i * 9 + j] = sw ? t : A[i * 9 + j];
-      }
-    }
-    const double r = 1.0 / A[k * 9 + k];
-#pragma unroll
-    for (int i = k + 1; i < 9; ++i) {
-      const double l = A[i * 9 + k] * r;
-      A[i * 9 + k] = l;
-#pragma unroll
-      for (int j = k + 1; j < 9; ++j) A[i * 9 + j] -= l * A[k * 9 + j];
-    }
-  }
-  return true;
+    for (int j = 0; j < 3; ++j) C[i * 3 + j] = fma3(A[i], B[j], A[3 + i], B[3 + j], A[6 + i], B[6 + j]);
 }
-__device__ __forceinline__ void lu9_solve(const double (&A)[81], const int (&piv)[9], double (&b)[9]) {
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-#pragma unroll
-    for (int i = k + 1; i < 9; ++i) {
-      const bool sw = (i == piv[k]);
-      const double t = b[k];
-      b[k] = sw ? b[i] : t;
-      b[i] = sw ? t : b[i];
-    }
-#pragma unroll
-  for (int k = 0; k < 9; ++k)
-#pragma unroll
-    for (int i = k + 1; i < 9; ++i) b[i] -= A[i * 9 + k] * b[k];
-#pragma unroll
-  for (int i = 8; i >= 0; --i) {
-    double s = b[i];
-#pragma unroll
-    for (int j = i + 1; j < 9; ++j) s -= A[i * 9 + j] * b[j];
-    b[i] = s / A[i * 9 + i];
-  }
-}
-
-// Material-point evaluation at x = (M, lambda, g).  Returns false outside the domain.
-struct CPPoint {
-  double Mi[9], pJ, eF[9], Ce[9], S[6], Sig[9], tau[12], gdot[12], dgdt[12], dgdg[12];
-  double gsum, gs, dgs, R[11];
-  HeTan he;  // law 1: tangent coefficients at Ce
-};
-
-template <bool HE>
-__device__ __forceinline__ bool cp_point(const CPMaterial &cm, const DevGrain &gr, const double *A,
-                                         double det_pFn, double g_n, double dt, const double *x,
-                                         CPPoint &p) {
-  const double *M = x;
-  const double lam = x[9], g = x[10];
-  if (!(g > 0.0)) return false;
-  const double dM = det3(M);
-  if (!(dM > 0.0)) return false;
-  if (!inv3(M, p.Mi)) return false;
-  p.pJ = det_pFn / dM;
-  mm3(A, M, p.eF);
-  mtm3(p.eF, p.eF, p.Ce);
-  el_stress<HE>(cm, gr, p.eF, p.Ce, p.S, p.he);
-  double S9[9];
-  v6_to_9(p.S, S9);
-  mm3(p.Ce, S9, p.Sig);
-  const double expo = 1.0 / cm.m - 1.0;
-  // one reciprocal of g for the twelve systems (the divisions are software sequences)
-  const double rg = 1.0 / g, cdg = cm.gd0 * rg / cm.m;
-  p.gsum = 0.0;
-#pragma unroll
-  for (int a = 0; a < 12; ++a) {
-    const double t = resolved(gr, a, p.Sig);
-    p.tau[a] = t;
-    const double r = t * rg;
-    const double pw = flow_pow(fabs(r), expo, cm.ipow);
-    p.gdot[a] = cm.gd0 * r * pw;
-    p.dgdt[a] = cdg * pw;
-    p.dgdg[a] = -p.dgdt[a] * r;
-    p.gsum += fabs(p.gdot[a]);
-  }
-  if (cm.w == 0.0) {
-    p.gs = cm.gs0;
-    p.dgs = 0.0;
-  } else if (p.gsum / cm.gds > 1.0e-15) {
-    p.gs = cm.gs0 * pow(p.gsum / cm.gds, cm.w);
-    p.dgs = cm.w * p.gs / p.gsum;
-  } else {
-    p.gs = 0.0;
-    p.dgs = 0.0;
-  }
-  double sl[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // sum_a gdot_a s_a (x) m_a, in system order
-#pragma unroll
-  for (int a = 0; a < 12; ++a)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const double c = p.gdot[a] * gr.s[a][i];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) sl[i * 3 + j] += c * gr.m[a / 3][j];
-    }
+__device__ __forceinline__ void mul_abt(const double *A, const double *B, double *C) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j)
-      p.R[i * 3 + j] = M[i * 3 + j] - ((i == j) ? 1.0 : 0.0) + dt * sl[i * 3 + j] - dt * lam * p.pJ * p.Mi[j * 3 + i];
-  p.R[9] = p.pJ - 1.0;
-  p.R[10] = g * (p.gs - cm.g0 + dt * cm.h0 * p.gsum) - (p.gs - cm.g0) * g_n - dt * cm.h0 * p.gs * p.gsum;
-  return true;
+      C[i * 3 + j] = fma3(A[i * 3], B[j * 3], A[i * 3 + 1], B[j * 3 + 1], A[i * 3 + 2], B[j * 3 + 2]);
+}
+__device__ __forceinline__ double det2(double a, double b, double c, double d) {  // a b - c d
+#pragma clang fp contract(off)
+  return __builtin_fma(a, b, -(c * d));
+}
+// the inverse and determinant of m; false below the singularity threshold of inv3
+__device__ __forceinline__ bool inv_det(const double *m, double *mi, double &det) {
+#pragma clang fp contract(off)
+  const double c0 = det2(m[4], m[8], m[5], m[7]), c1 = det2(m[5], m[6], m[3], m[8]), c2 = det2(m[3], m[7], m[4], m[6]);
+  det = fma3(m[0], c0, m[1], c1, m[2], c2);
+  const double r = 1.0 / det;
+  mi[0] = r * c0;
+  mi[3] = r * c1;
+  mi[6] = r * c2;
+  mi[1] = r * det2(m[2], m[7], m[1], m[8]);
+  mi[4] = r * det2(m[0], m[8], m[2], m[6]);
+  mi[7] = r * det2(m[1], m[6], m[0], m[7]);
+  mi[2] = r * det2(m[1], m[5], m[2], m[4]);
+  mi[5] = r * det2(m[2], m[3], m[0], m[5]);
+  mi[8] = r * det2(m[0], m[4], m[1], m[3]);
+  return fabs(det) >= 1.0e-15;
+}
+__device__ __forceinline__ void rot_in(const double *R, const double *X, double *Y) {  // R^T X R
+  double T[9];
+  mul_ab(X, R, T);
+  mul_atb(R, T, Y);
+}
+__device__ __forceinline__ void rot_out(const double *R, const double *X, double *Y) {  // R X R^T
+  double T[9];
+  mul_ab(R, X, T);
+  mul_abt(T, R, Y);
+}
+// The same of X = I + Y, as I + R^T Y R: the orthonormality error of R (1e-16) would otherwise come
+// into the elastic strain, and times C / tau = 1e4 into the stress.
+__device__ __forceinline__ void rot_in_1(const double *R, const double *X, double *Y) {
+  const double D[9] = {X[0] - 1.0, X[1], X[2], X[3], X[4] - 1.0, X[5], X[6], X[7], X[8] - 1.0};
+  rot_in(R, D, Y);
+  Y[0] += 1.0;
+  Y[4] += 1.0;
+  Y[8] += 1.0;
+}
+__device__ __forceinline__ void rot_out_1(const double *R, const double *X, double *Y) {
+  const double D[9] = {X[0] - 1.0, X[1], X[2], X[3], X[4] - 1.0, X[5], X[6], X[7], X[8] - 1.0};
+  rot_out(R, D, Y);
+  Y[0] += 1.0;
+  Y[4] += 1.0;
+  Y[8] += 1.0;
 }
 
-// Q_a = sym(P_a S + 1/2 L:(C_e P_a)) in Voigt order, so that d tau_a / d M = 2 A^T eF Q_a
+// What of the flow and hardening rule needs pow: 0 both, 1 the saturation stress (w != 0), 2 none.
+// A kernel holds one form: twelve inlined pows are a quarter of the Newton kernel's code, which
+// has to fit the instruction cache, and one pow's constants, kept across its loop, 40 registers.
+enum : int { kFlowPow = 0, kFlowSat = 1, kFlowPlain = 2 };
+// |r_a|^e of the power-law flow rule, e = 1/m - 1, for the twelve systems.  When e is a whole
+// number (ie >= 0; the rate sensitivity m = 0.05 gives 19) it is formed by binary powering, a
+// handful of multiplies where pow takes about 130 FP64 operations; the two agree to a few ulps.
+template <int FLOW>
+__device__ __forceinline__ void flow_pow(const double (&r)[12], double e, int ie, double (&w)[12]) {
+  if constexpr (FLOW >= 1) {
+    double b[12];
+#pragma unroll
+    for (int a = 0; a < 12; ++a) {
+      b[a] = fabs(r[a]);
+      w[a] = 1.0;
+    }
+    for (int k = ie; k; k >>= 1) {
+      if (k & 1) {
+#pragma unroll
+        for (int a = 0; a < 12; ++a) w[a] *= b[a];
+      }
+#pragma unroll
+      for (int a = 0; a < 12; ++a) b[a] *= b[a];
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < 12; ++a) w[a] = pow(fabs(r[a]), e);
+  }
+}
+
+// Elastic PK2 (Voigt) in the crystal frame from eF and Ce = eF^T eF: law 0 is the cubic
+// S = L : (Ce - I)/2; law 1 is he_law, which also fills the tangent coefficients.  The
+// multiply-adds are explicit, so that every kernel gives the same bits.
 template <bool HE>
-__device__ __forceinline__ void qsym(const DevGrain &gr, int a, const CPPoint &p, double *Q6) {
-  // with P = s (x) m: P S = s (x) (S m) (S symmetric) and C_e P = (C_e s) (x) m
-  const double *s = gr.s[a], *m = gr.m[a / 3];
-  double S9[9], PS[9], CP[9], v[3], w[3];
+__device__ __forceinline__ void el_stress(const CPMaterial &cm, const double *eF, const double *Ce, double *S6,
+                                          HeTan &t) {
+  if constexpr (HE) {
+    he_law(cm, eF, Ce, S6, t);
+  } else {
+#pragma clang fp contract(off)
+    const double e0 = 0.5 * (Ce[0] - 1.0), e1 = 0.5 * (Ce[4] - 1.0), e2 = 0.5 * (Ce[8] - 1.0);
+    const double ct = cm.c12 * ((e0 + e1) + e2), sh = 0.5 * cm.c44x2;
+    S6[0] = __builtin_fma(cm.c11m12, e0, ct);
+    S6[1] = __builtin_fma(cm.c11m12, e1, ct);
+    S6[2] = __builtin_fma(cm.c11m12, e2, ct);
+    S6[3] = sh * Ce[1];
+    S6[4] = sh * Ce[5];
+    S6[5] = sh * Ce[2];
+  }
+}
+
+// eF = A M, C_e = eF^T eF, S and the twelve tau_a = (C_e S) : P_a
+struct CPStress {
+  double eF[9], Ce[9], S[6], tau[12];
+  HeTan he;  // law 1: tangent coefficients at Ce
+};
+template <bool HE>
+__device__ __forceinline__ void cp_stress(const CPMaterial &cm, const double *A, const double *M, CPStress &p) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) p.eF[i * 3 + j] = fma3(A[i * 3], M[j], A[i * 3 + 1], M[3 + j], A[i * 3 + 2], M[6 + j]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = i; j < 3; ++j)
+      p.Ce[j * 3 + i] = p.Ce[i * 3 + j] = fma3(p.eF[i], p.eF[j], p.eF[3 + i], p.eF[3 + j], p.eF[6 + i], p.eF[6 + j]);
+  el_stress<HE>(cm, p.eF, p.Ce, p.S, p.he);
+  double S9[9], Sig[9];
   v6_to_9(p.S, S9);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    v[i] = S9[i * 3 + 0] * m[0] + S9[i * 3 + 1] * m[1] + S9[i * 3 + 2] * m[2];
-    w[i] = p.Ce[i * 3 + 0] * s[0] + p.Ce[i * 3 + 1] * s[1] + p.Ce[i * 3 + 2] * s[2];
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      Sig[i * 3 + j] = fma3(p.Ce[i * 3], S9[j], p.Ce[i * 3 + 1], S9[3 + j], p.Ce[i * 3 + 2], S9[6 + j]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    double u[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) u[i] = n_dot(k, Sig[i * 3], Sig[i * 3 + 1], Sig[i * 3 + 2]);
+#pragma unroll
+    for (int a = 3 * k; a < 3 * k + 3; ++a) p.tau[a] = kR6 * s_dot(a, u);
   }
+}
+
+// Material-point evaluation at x = (M, lambda, g).  Returns false outside the domain, where p is
+// of no use; every lane runs through it, since a branch around it would keep its registers
+// live from one turn of the Newton loop to the next.
+struct CPPoint : CPStress {
+  double T[9];    // M^-T
+  double N[9];    // dt sum_a gdot_a P_a
+  double sd[12];  // dgdot_a / dtau_a with the sign of gdot_a
+  double pJ, gsum, gs, dgs, R[11];
+};
+
+template <bool HE, int FLOW>
+__device__ __forceinline__ bool cp_point(const CPMaterial &cm, const double *A, double det_pFn, double g_n, double dt,
+                                         const double *x, CPPoint &p) {
+  const double *M = x;
+  const double lam = x[9], g = x[10];
+  double Mi[9], dM;
+  const bool valid = inv_det(M, Mi, dM) && dM > 0.0 && g > 0.0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) p.T[i * 3 + j] = Mi[j * 3 + i];
+  p.pJ = det_pFn / dM;
+  cp_stress<HE>(cm, A, M, p);
+  // one reciprocal of g for the twelve systems (the divisions are software sequences)
+  const double rg = 1.0 / g, cdg = cm.gd0_m * rg;
+  double r[12], w[12], V[4][3] = {};  // V_k = sum over plane k of gdot_a s_a
+#pragma unroll
+  for (int a = 0; a < 12; ++a) r[a] = p.tau[a] * rg;
+  flow_pow<FLOW>(r, cm.expo, cm.ipow, w);
+  p.gsum = 0.0;
+#pragma unroll
+  for (int a = 0; a < 12; ++a) {
+    const double gdot = cm.gd0 * r[a] * w[a];
+    p.sd[a] = r[a] < 0.0 ? -(cdg * w[a]) : cdg * w[a];
+    p.gsum += fabs(gdot);
+    s_add(a, gdot, V[a / 3]);
+  }
+  p.gs = cm.gs0;
+  p.dgs = 0.0;
+  if (FLOW != kFlowPlain && cm.w != 0.0) {
+    const bool flows = p.gsum / cm.gds > 1.0e-15;
+    p.gs = flows ? cm.gs0 * pow(p.gsum / cm.gds, cm.w) : 0.0;
+    p.dgs = flows ? cm.w * p.gs / p.gsum : 0.0;
+  }
+  const double dk = dt * kR6, dl = dt * lam * p.pJ;
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      PS[i * 3 + j] = s[i] * v[j];
-      CP[i * 3 + j] = w[i] * m[j];
+      double sl = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sl += pm(n_sign(k, j), V[k][i]);
+      p.N[i * 3 + j] = dk * sl;
+      p.R[i * 3 + j] = M[i * 3 + j] - ((i == j) ? 1.0 : 0.0) + p.N[i * 3 + j] - dl * p.T[i * 3 + j];
     }
-  double LCP[6];
-  if constexpr (HE) he_dot(p.he, CP, LCP);
-  else cubic_dot(gr.R, gr.cub, CP, LCP);
+  p.R[9] = p.pJ - 1.0;
+  p.R[10] = g * (p.gs - cm.g0 + dt * cm.h0 * p.gsum) - (p.gs - cm.g0) * g_n - dt * cm.h0 * p.gs * p.gsum;
+  return valid;
+}
+
+// What one system's Q_a = sym(P_a S + 1/2 L:(C_e P_a)), d tau_a / d M = 2 A^T eF Q_a, shares
+// with its plane: v = S n, and for law 1 Ci n.
+struct CPPlane {
+  double v[3], cn[3];
+};
+template <bool HE>
+__device__ __forceinline__ void cp_plane(const CPStress &p, int k, CPPlane &q) {
+  const double *S = p.S;
+  q.v[0] = n_dot(k, S[0], S[3], S[5]);
+  q.v[1] = n_dot(k, S[3], S[1], S[4]);
+  q.v[2] = n_dot(k, S[5], S[4], S[2]);
+  if constexpr (HE) {
+    const double *C = p.he.Ci;
+    q.cn[0] = n_dot(k, C[0], C[3], C[5]);
+    q.cn[1] = n_dot(k, C[3], C[1], C[4]);
+    q.cn[2] = n_dot(k, C[5], C[4], C[2]);
+  }
+}
+// Q_a * 2 / kR6 in Voigt order.  P_a S = kR6 s (x) v, C_e P_a = kR6 w (x) n with w = C_e s.
+// Law 0: L of w (x) n by its three constants.  Law 1: he_dot of sym(w (x) n), where Ci w = s and
+// s . n = 0 leave c2 tr Ci + c3 sym(s (x) Ci n).
+template <bool HE>
+__device__ __forceinline__ void cp_q(const CPMaterial &cm, const CPStress &p, const CPPlane &pl, int a, double *q) {
+  const int k = a / 3;
+  double w[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) w[i] = s_dot(a, p.Ce + 3 * i);  // C_e is symmetric
+  const double tr = n_dot(k, w[0], w[1], w[2]);
 #pragma unroll
   for (int I = 0; I < 6; ++I) {
-    const int i = vi(I), j = vj(I);
-    Q6[I] = 0.5 * (PS[i * 3 + j] + PS[j * 3 + i]) + 0.5 * LCP[I];
-  }
-}
-
-// d tau_a / d M = 2 A^T eF sym(P_a S + 1/2 L:(C_e P_a))
-template <bool HE>
-__device__ __forceinline__ void dtau_dM(const DevGrain &gr, int a, const double *AtE, const CPPoint &p, double *D) {
-  double Q6[6], sQ[9];
-  qsym<HE>(gr, a, p, Q6);
-  v6_to_9(Q6, sQ);
-  double T[9];
-  mm3(AtE, sQ, T);
-#pragma unroll
-  for (int i = 0; i < 9; ++i) D[i] = 2.0 * T[i];
-}
-
-// d tau_a / d M from a Q_a formed earlier: 2 A^T eF sym(Q_a)
-__device__ __forceinline__ void dtau_dM_q(const double *AtE, const double *Q6, double *D) {
-  double sQ[9], T[9];
-  v6_to_9(Q6, sQ);
-  mm3(AtE, sQ, T);
-#pragma unroll
-  for (int i = 0; i < 9; ++i) D[i] = 2.0 * T[i];
-}
-
-// Bordered Jacobian [Ah b c; d^T 0 0; e^T 0 f] at p.
-struct Border {
-  double b[9], c[9], d[9], e[9], f, dRg;
-};
-
-// Bordered Jacobian of the local system at p; the per-system slip quantities are recomputed
-// from the Mandel stress with cp_point's arithmetic.  QPRE: the Q_a of qsym were formed
-// earlier and sit in LDS at qpre[(a * 6 + I) * 64].
-template <bool HE, bool QPRE = false>
-__device__ __forceinline__ void cp_jacobian_re(const CPMaterial &cm, const DevGrain &gr, double dt, const double *x,
-                                            const double *A, const CPPoint &p, double g_n,
-                                            double (&Ah)[81], Border &B, const double *qpre = nullptr) {
-  const double lam = x[9], g = x[10];
-  double AtE[9];
-  mtm3(A, p.eF, AtE);
-#pragma unroll
-  for (int i = 0; i < 81; ++i) Ah[i] = 0.0;
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    B.c[i] = 0.0;
-    B.e[i] = 0.0;
-  }
-  double sg = 0.0;
-  const double expo = 1.0 / cm.m - 1.0;
-  const double rg = 1.0 / g, cdg = cm.gd0 * rg / cm.m;
-  for (int a = 0; a < 12; ++a) {
-    // slip-system quantities recomputed from the Mandel stress (as cp_point evaluates them)
-    const double t = resolved(gr, a, p.Sig);
-    const double r = t * rg;
-    const double pw = flow_pow(fabs(r), expo, cm.ipow);
-    const double gd = cm.gd0 * r * pw;
-    const double dgdt = cdg * pw;
-    const double dgdg = -dgdt * r;
-    double D[9];
-    if constexpr (QPRE) {
-      double Q6[6];
-#pragma unroll
-      for (int I = 0; I < 6; ++I) Q6[I] = qpre[(a * 6 + I) * 64];
-      dtau_dM_q(AtE, Q6, D);
+    const int i = voigt_i(I), j = voigt_j(I);
+    double x = 0.0;  // s_i v_j + s_j v_i
+    if (s_sign(a, i) != 0) x += pm(s_sign(a, i), pl.v[j]);
+    if (s_sign(a, j) != 0) x += pm(s_sign(a, j), pl.v[i]);
+    if constexpr (HE) {
+      double y = 0.0;  // s_i cn_j + s_j cn_i
+      if (s_sign(a, i) != 0) y += pm(s_sign(a, i), pl.cn[j]);
+      if (s_sign(a, j) != 0) y += pm(s_sign(a, j), pl.cn[i]);
+      q[I] = x + p.he.c2 * tr * p.he.Ci[I] + 0.5 * p.he.c3 * y;
+    } else if (I < 3) {
+      q[I] = x + (cm.c11m12 * pm(n_sign(k, i), w[i]) + cm.c12 * tr);
     } else {
-      dtau_dM<HE>(gr, a, AtE, p, D);
+      q[I] = x + 0.5 * cm.c44x2 * (pm(n_sign(k, j), w[i]) + pm(n_sign(k, i), w[j]));
     }
-    const double co = dt * dgdt;
-    const double sgn = (gd < 0) ? -1.0 : 1.0;
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-      const double Pr = gr.s[a][r / 3] * gr.m[a / 3][r % 3];
-      const double pr = Pr * co;
-#pragma unroll
-      for (int c = 0; c < 9; ++c) Ah[r * 9 + c] += pr * D[c];
-      B.c[r] += dt * Pr * dgdg;
-    }
-#pragma unroll
-    for (int c = 0; c < 9; ++c) B.e[c] += sgn * dgdt * D[c];
-    sg += sgn * dgdg;
   }
-  const double *Mi = p.Mi;
-  const double lp = dt * lam * p.pJ;
+}
+
+// The Jacobian of the local system at p is bordered,
+//   [A b c; d^T 0 0; e^T 0 f],  d = -pJ M^-T, b = dt d,
+// and A and e see dM only through the six numbers K dM = sym(A^T eF dM) (K_I: the diagonal
+// entries of Y = AtE^T dM, then Y_ij + Y_ji), since dtau_a does:
+//   e = es eq K,  A - c e^T / f = I + lp T (.)^T T + G K,  T = M^-T, lp = dt lambda pJ,
+// less A's term lp T (x) T = (lambda / pJ) b d^T: where d . u = s is an equation of the system,
+// that term only moves (lambda / pJ) s between A u and b y.
+// G = sum_a dt dgdt_a / 6 (s_a n_k) (x) q_a - c (es eq) / f.  The power law gives the rest from
+// what the point has: dgdot_a/dg = -gdot_a / (m g), so c = -N / (m g).
+struct LocalLin {
+  double G[9][6], eq[6], es, f;
+};
+// G and eq without the factors of cp_fold
+template <bool HE>
+__device__ __forceinline__ void cp_slip_sums(const CPMaterial &cm, const CPStress &p, const double *sd, LocalLin &L) {
+#pragma unroll
+  for (int I = 0; I < 6; ++I) L.eq[I] = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    CPPlane pl;
+    cp_plane<HE>(p, k, pl);
+    double V[3][6] = {};
+#pragma unroll
+    for (int a = 3 * k; a < 3 * k + 3; ++a) {
+      double q[6];
+      cp_q<HE>(cm, p, pl, a, q);
+#pragma unroll
+      for (int I = 0; I < 6; ++I) {
+        L.eq[I] += sd[a] * q[I];
+        q[I] *= fabs(sd[a]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          if (s_sign(a, i) != 0) V[i][I] += pm(s_sign(a, i), q[I]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int I = 0; I < 6; ++I)
+          L.G[i * 3 + j][I] = k == 0 ? V[i][I] : L.G[i * 3 + j][I] + pm(n_sign(k, j), V[i][I]);
+#pragma unroll
+    for (int r = 0; r < 9; ++r) pin(L.G[r]);
+    end_stage();
+  }
+}
+__device__ __forceinline__ void cp_fold(const CPMaterial &cm, double dt, double g, double g_n, double gsum, double gs,
+                                        double dgs, const double *c, LocalLin &L) {
+  const double dRg = g * (dgs + dt * cm.h0) - dgs * g_n - dt * cm.h0 * (dgs * gsum + gs);
+  L.f = (gs - cm.g0 + dt * cm.h0 * gsum) - dRg * gsum / (cm.m * g);
+  L.es = dRg * kR6;
+  const double as = dt * (kR6 * kR6), rf = L.es / L.f;
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    const double cr = c[r] * rf;
+#pragma unroll
+    for (int I = 0; I < 6; ++I) L.G[r][I] = as * L.G[r][I] - cr * L.eq[I];
+  }
+}
+// the matrix I + lp T (.)^T T + G K
+__device__ __forceinline__ void cp_matrix(const LocalLin &L, const double *AtE, const double *T, double lp,
+                                          double (&Ah)[81]) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int j = 0; j < 3; ++j) {
+      const int r = i * 3 + j;
+      double G9[9];
+      v6_to_9(L.G[r], G9);
+      double lt[3];
+#pragma unroll
+      for (int l = 0; l < 3; ++l) lt[l] = lp * T[i * 3 + l];
 #pragma unroll
       for (int k = 0; k < 3; ++k)
 #pragma unroll
         for (int l = 0; l < 3; ++l)
-          Ah[(i * 3 + j) * 9 + k * 3 + l] +=
-              ((i == k && j == l) ? 1.0 : 0.0) + lp * (Mi[j * 3 + i] * Mi[l * 3 + k] + Mi[l * 3 + i] * Mi[j * 3 + k]);
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      B.b[i * 3 + j] = -dt * p.pJ * Mi[j * 3 + i];
-      B.d[i * 3 + j] = -p.pJ * Mi[j * 3 + i];
+          Ah[r * 9 + k * 3 + l] = ((i == k && j == l) ? 1.0 : 0.0) + AtE[k * 3] * G9[l] + AtE[k * 3 + 1] * G9[3 + l] +
+                                  AtE[k * 3 + 2] * G9[6 + l] + lt[l] * T[k * 3 + j];
     }
-  B.dRg = g * (p.dgs + dt * cm.h0) - p.dgs * g_n - dt * cm.h0 * (p.dgs * p.gsum + p.gs);
-#pragma unroll
-  for (int c = 0; c < 9; ++c) B.e[c] *= B.dRg;
-  B.f = (p.gs - cm.g0 + dt * cm.h0 * p.gsum) + B.dRg * sg;
-  // Schur: Ah <- A - c e^T / f
-  const double rf = 1.0 / B.f;
-#pragma unroll
-  for (int r = 0; r < 9; ++r)
-#pragma unroll
-    for (int c = 0; c < 9; ++c) Ah[r * 9 + c] -= B.c[r] * B.e[c] * rf;
 }
 
-// Solve [A b c; d^T 0 0; e^T 0 f] [u; y; z] = [r; s; t] given LU(Ah) and v = Ah^-1 b.
-__device__ __forceinline__ void bordered_solve(const double (&LU)[81], const int (&piv)[9], const Border &B,
-                                               const double (&v)[9], double dTv, const double *r, double s,
-                                               double t, double *out) {
-  double u[9];
-  const double tf = t / B.f;
+// Gaussian elimination of A with NR right-hand sides, solutions in B, without pivoting; false
+// where a multiplier exceeds max_mult or a pivot is no number, and the caller takes
+// eliminate_pivot.  The local system is the identity plus the slip systems' positive part, so
+// large multipliers are rare (above 1000 in 0.1% of the matrices of a plastic step), and partial
+// pivoting by predicated swaps is more instructions than the elimination.  A Newton step only has
+// to be a good direction: the residual, not the matrix, fixes the point that the iteration ends
+// at, and at 1e6 its relative error stays near 1e-10.  At 1e3 one turn of the wave in ten waited
+// for a lane's pivoting, and cp_newton took 2295 us instead of 740 (998,250 QPs).  The tangent is
+// a result, and its bound lower.
+constexpr double kMaxMultStep = 1.0e6, kMaxMultTangent = 1.0e4;
+template <int N, int NR>
+__device__ __forceinline__ bool eliminate(double (&A)[N * N], double (&B)[NR][N], double max_mult) {
+  double lmax = 0.0, rd[N];
 #pragma unroll
-  for (int i = 0; i < 9; ++i) u[i] = r[i] - B.c[i] * tf;
-  lu9_solve(LU, piv, u);
-  double dTu = 0.0;
+  for (int k = 0; k < N; ++k) {
+    rd[k] = 1.0 / A[k * N + k];
 #pragma unroll
-  for (int i = 0; i < 9; ++i) dTu += B.d[i] * u[i];
-  const double y = (dTu - s) / dTv;
-  double eTx = 0.0;
+    for (int i = k + 1; i < N; ++i) {
+      const double l = A[i * N + k] * rd[k];
+      lmax = fmax(lmax, fabs(l));
 #pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    out[i] = u[i] - y * v[i];
-    eTx += B.e[i] * out[i];
+      for (int j = k + 1; j < N; ++j) A[i * N + j] -= l * A[k * N + j];
+#pragma unroll
+      for (int q = 0; q < NR; ++q) B[q][i] -= l * B[q][k];
+    }
+    asm volatile("" : "+v"(lmax));  // now, not from multipliers kept to the end
   }
-  out[9] = y;
-  out[10] = (t - eTx) / B.f;
+#pragma unroll
+  for (int i = N - 1; i >= 0; --i)
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      double s = B[q][i];
+#pragma unroll
+      for (int j = i + 1; j < N; ++j) s -= A[i * N + j] * B[q][j];
+      B[q][i] = s * rd[i];
+    }
+  return lmax <= max_mult && fabs(rd[N - 1]) < __builtin_huge_val();
+}
+// The same with partial pivoting, in scratch memory: rare, and kept from costing the common path
+// registers (the system is stored before the common path consumes it, and solved after it).
+// False for a singular matrix.
+template <int N, int NR>
+__device__ __forceinline__ void store_system(const double (&A)[N * N], const double (&B)[NR][N], double *a) {
+  constexpr int W = N + NR;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) a[i * W + j] = A[i * N + j];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) a[i * W + N + q] = B[q][i];
+  }
+}
+template <int N, int NR>
+__device__ __forceinline__ bool eliminate_pivot(double *a, double (&B)[NR][N]) {
+  constexpr int W = N + NR;
+  bool ok = true;
+#pragma unroll 1
+  for (int k = 0; k < N; ++k) {
+    int p = k;
+    double amax = fabs(a[k * W + k]);
+#pragma unroll 1
+    for (int i = k + 1; i < N; ++i) {
+      const double v = fabs(a[i * W + k]);
+      p = v > amax ? i : p;
+      amax = v > amax ? v : amax;
+    }
+    ok = ok && amax > 0.0;
+    double row[W];
+    const double r = 1.0 / a[p * W + k];
+#pragma unroll
+    for (int j = 0; j < W; ++j) row[j] = a[p * W + j] * r;
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[p * W + j] = a[k * W + j];
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[k * W + j] = row[j];
+#pragma unroll 1
+    for (int i = 0; i < N; ++i) {  // to the diagonal: the rows above take part
+      const double l = i == k ? 0.0 : a[i * W + k];
+#pragma unroll
+      for (int j = 0; j < W; ++j) a[i * W + j] -= l * row[j];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int i = 0; i < N; ++i) B[q][i] = a[i * W + N + q];
+  return ok;
 }
 
 __device__ __forceinline__ double cp_merit(const CPPoint &p, double gscale) {
@@ -536,107 +682,40 @@ __device__ __forceinline__ double cp_merit(const CPPoint &p, double gscale) {
   return 0.5 * (r + rg * rg);
 }
 
-// The merit of x without keeping the point: the same arithmetic as cp_point's residual (slip
-// contributions accumulated in slip-system order), so acceptance decisions match it.
-template <bool HE>
-__device__ __forceinline__ bool cp_merit_at(const CPMaterial &cm, const DevGrain &gr, const double *A,
-                                            double det_pFn, double g_n, double dt, const double *x, double gscale,
-                                            double &merit) {
-  const double *M = x;
-  const double lam = x[9], g = x[10];
-  if (!(g > 0.0)) return false;
-  const double dM = det3(M);
-  if (!(dM > 0.0)) return false;
-  double Mi[9];
-  if (!inv3(M, Mi)) return false;
-  const double pJ = det_pFn / dM;
-  double eF[9], Ce[9], S[6], S9[9], Sig[9];
-  mm3(A, M, eF);
-  mtm3(eF, eF, Ce);
-  HeTan ht;
-  el_stress<HE>(cm, gr, eF, Ce, S, ht);
-  v6_to_9(S, S9);
-  mm3(Ce, S9, Sig);
-  const double expo = 1.0 / cm.m - 1.0;
-  const double rg = 1.0 / g;
-  double gsum = 0.0, sl[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int a = 0; a < 12; ++a) {
-    const double t = resolved(gr, a, Sig);
-    const double r = t * rg;
-    const double gd = cm.gd0 * r * flow_pow(fabs(r), expo, cm.ipow);
-    gsum += fabs(gd);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const double c = gd * gr.s[a][i];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) sl[i * 3 + j] += c * gr.m[a / 3][j];
-    }
-  }
-  double gs;
-  if (cm.w == 0.0) gs = cm.gs0;
-  else if (gsum / cm.gds > 1.0e-15) gs = cm.gs0 * pow(gsum / cm.gds, cm.w);
-  else gs = 0.0;
-  double r2 = 0.0;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double R = M[i * 3 + j] - ((i == j) ? 1.0 : 0.0) + dt * sl[i * 3 + j] - dt * lam * pJ * Mi[j * 3 + i];
-      r2 += R * R;
-    }
-  const double R9 = pJ - 1.0;
-  r2 += R9 * R9;
-  const double R10 = (g * (gs - cm.g0 + dt * cm.h0 * gsum) - (gs - cm.g0) * g_n - dt * cm.h0 * gs * gsum) * gscale;
-  merit = 0.5 * (r2 + R10 * R10);
-  return true;
-}
-
 // max_a |tau_a| / g at M (elastic part eF = A M)
 template <bool HE>
-__device__ __forceinline__ double tau_ratio_max(const CPMaterial &cm, const DevGrain &gr, const double *A,
-                                                const double *M, double rg) {
-  double eF[9], Ce[9], S[6], S9[9], Sig[9];
-  mm3(A, M, eF);
-  mtm3(eF, eF, Ce);
-  HeTan ht;
-  el_stress<HE>(cm, gr, eF, Ce, S, ht);
-  v6_to_9(S, S9);
-  mm3(Ce, S9, Sig);
+__device__ __forceinline__ double tau_ratio_max(const CPMaterial &cm, const double *A, const double *M, double rg) {
+  CPStress p;
+  cp_stress<HE>(cm, A, M, p);
   double mx = 0.0;
 #pragma unroll
-  for (int a = 0; a < 12; ++a) mx = fmax(mx, fabs(resolved(gr, a, Sig)));
+  for (int a = 0; a < 12; ++a) mx = fmax(mx, fabs(p.tau[a]));
   return mx * rg;
 }
 
-// Plain start x = (M, lambda_n, g_n): the fully plastic predictor pulled back to yield.
+// Plain start x = (M, lambda_n, g_n) in the crystal frame: the fully plastic predictor
+// Mp = pF(n) F^-1 F(n) pF(n)^-1 (not yet scaled to det 1), pulled back to yield.
 template <bool HE>
-__device__ __forceinline__ bool cp_start(const CPMaterial &cm, const DevGrain &gr, const double *A,
-                                         const double *F, const double *Fn,
-                                         const double *pFn, const double *pFi, double g_n, double lam_n,
-                                         double *x) {
-  double Fi[9], T[9], Mp[9];
-  if (!inv3(F, Fi)) return false;
-  mm3(pFn, Fi, T);
-  mm3(T, Fn, Mp);
-  mm3(Mp, pFi, T);
-  const double dp = det3(T);
+__device__ __forceinline__ bool cp_start(const CPMaterial &cm, const double *A, double (&Mp)[9], double g_n,
+                                         double lam_n, double *x) {
+  const double dp = det3(Mp);
   if (!(dp > 0.0)) return false;
   const double c = 1.0 / cbrt(dp);
 #pragma unroll
-  for (int i = 0; i < 9; ++i) Mp[i] = T[i] * c;
+  for (int i = 0; i < 9; ++i) Mp[i] *= c;
   const double rg = 1.0 / g_n;
   const double I9[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
   double al = 0.0;
-  if (tau_ratio_max<HE>(cm, gr, A, I9, rg) > 1.0) {
+  if (tau_ratio_max<HE>(cm, A, I9, rg) > 1.0) {
     al = 1.0;
-    if (!(tau_ratio_max<HE>(cm, gr, A, Mp, rg) > 1.0)) {
+    if (!(tau_ratio_max<HE>(cm, A, Mp, rg) > 1.0)) {
       double lo = 0.0, hi = 1.0;
       for (int k = 0; k < 8; ++k) {
         const double mid = 0.5 * (lo + hi);
         double Mm[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) Mm[i] = I9[i] + mid * (Mp[i] - I9[i]);
-        if (tau_ratio_max<HE>(cm, gr, A, Mm, rg) > 1.0) lo = mid;
+        if (tau_ratio_max<HE>(cm, A, Mm, rg) > 1.0) lo = mid;
         else hi = mid;
       }
       al = hi;
@@ -727,36 +806,50 @@ __global__ __launch_bounds__(256) void cp_kinematics(CPArgs a) {
 // qpbuf holds the plain start x(0..10) and the choice kStartFlag (bit 0: the plain start
 // failed, bit 1: take the caller's start) until the tangent kernel overwrites it.
 constexpr int kStartFlag = 11;
-template <bool HE>
+template <bool HE, int FLOW>
 __global__ __launch_bounds__(64) void cp_start_kernel(CPArgs a) {
   const int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (q >= a.nq) return;
   const int64_t NQ = a.n_qp;
   const int64_t qg = a.qp_base + q;
   const CPMaterial cm = a.cpmats[0];
-  const DevGrain &gr = a.grains[a.qgrain[q]];
-  double F[9], pFn[9], pFi[9], Fn[9], A[9], x[11];
+  const double *R = a.grains[a.qgrain[q]].R;
+  double F[9], pFn[9], pFi[9], Fn[9], Fi[9], A[9] = {}, T[9], Mp[9], x[11], det_pFn = 1.0, det_F;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
     F[i] = a.F_np1[i * NQ + qg];
     pFn[i] = a.pF_n[i * NQ + qg];
     Fn[i] = a.F_n[i * NQ + qg];
+    x[i] = 0.0;
   }
-  inv3(pFn, pFi);
-  mm3(F, pFi, A);
+  bool bad = !inv_det(pFn, pFi, det_pFn) || !inv_det(F, Fi, det_F);
   const double g_n = a.g_n[qg];
-  const bool bad = !cp_start<HE>(cm, gr, A, F, Fn, pFn, pFi, g_n, a.lam_n[qg], x);
+  x[9] = x[10] = 0.0;
+  if (!bad) {
+    mul_ab(F, pFi, T);
+    rot_in_1(R, T, A);
+    mul_ab(pFn, Fi, T);
+    mul_ab(T, Fn, Mp);
+    mul_ab(Mp, pFi, T);
+    rot_in_1(R, T, Mp);
+    bad = !cp_start<HE>(cm, A, Mp, g_n, a.lam_n[qg], x);
+  }
   int flag = bad ? 1 : 0;
   if (a.warm) {
     // a caller's start is taken when its residual merit is below the plain start's
-    const double det_pFn = det3(pFn);
     const double gscale = 1.0 / (fabs(cm.gs0 - cm.g0) * g_n + 1e-300);
     double xw[11];
 #pragma unroll
-    for (int i = 0; i < 11; ++i) xw[i] = a.warm[i * NQ + qg];
+    for (int i = 0; i < 9; ++i) T[i] = a.warm[i * NQ + qg];
+    rot_in_1(R, T, xw);
+    xw[9] = a.warm[9 * NQ + qg];
+    xw[10] = a.warm[10 * NQ + qg];
+    CPPoint p;
     double mw = 0.0, mp = 0.0;
-    const bool okw = cp_merit_at<HE>(cm, gr, A, det_pFn, g_n, a.dt, xw, gscale, mw);
-    const bool okp = !bad && cp_merit_at<HE>(cm, gr, A, det_pFn, g_n, a.dt, x, gscale, mp);
+    const bool okw = cp_point<HE, FLOW>(cm, A, det_pFn, g_n, a.dt, xw, p);
+    if (okw) mw = cp_merit(p, gscale);
+    const bool okp = !bad && cp_point<HE, FLOW>(cm, A, det_pFn, g_n, a.dt, x, p);
+    if (okp) mp = cp_merit(p, gscale);
     if (okw && (!okp || mw < mp)) flag |= 2;
   }
   double *row = a.qpbuf + qrec(qg);
@@ -766,214 +859,277 @@ __global__ __launch_bounds__(64) void cp_start_kernel(CPArgs a) {
 }
 
 // ------------------------------------------------------------------- Newton kernel
-// One wave per workgroup.  With a.qnext set, every wave takes its QPs from one global queue:
-// at each refill the wave's first lane that needs a QP claims as many consecutive QPs as lanes
-// need one, so lanes stay busy until the queue runs dry.  Otherwise wave w owns QPs
-// [w*chunk, (w+1)*chunk) of the block.  Which lane takes a QP does not change its result.  The
-// starting points come from cp_start_kernel (qpbuf).
-template <bool HE>
+// One wave per workgroup, one QP per lane, 64 QPs at a time: wave w works through QPs
+// [w*chunk, (w+1)*chunk) of the block, or, with a.qnext set, draws its batches from one global
+// queue.  Which lane takes a QP does not change its result.  A batch ends when its last QP has
+// converged (mean 5.1 iterations, largest 8): handing a free lane the next QP instead gained
+// nothing, since the wave then reads and writes that QP's state alone.  The starting points come
+// from cp_start_kernel (qpbuf).
+//
+// Bound by FP64 issue: a turn is about 3300 instructions for 64 QPs.  A turn has no divergent
+// branch around its stages (values would be kept across it), and each stage is closed by pin, so
+// the widest stretch, the 9 x 9 elimination, fits 306 registers with nothing spilled.  One wave
+// per SIMD: at two, 256 registers spill and it takes 800 us instead of 740 (998,250 QPs; 2743 us
+// in the sample frame, with the pivoting and the slip systems' tensors in registers).
+template <bool HE, int FLOW>
 __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
   const int lane = threadIdx.x;
-  const bool gq = a.qnext != nullptr;
-  const int64_t q_lo = gq ? 0 : int64_t(blockIdx.x) * chunk;
-  const int64_t q_hi = (gq || q_lo + chunk >= a.nq) ? a.nq : q_lo + chunk;
-  int64_t cursor = q_lo;  // wave-uniform
   const int64_t NQ = a.n_qp;
-  bool need = true, done = false;
-  int64_t q = -1;
   // The lane's QP data that lives across turns sits in LDS (lane-fastest; each lane touches
   // only its own slots), read where used, rather than in registers held through the material
-  // point and the Jacobian's LU, where it spilled: A (9), x (11), dx (11), det pF(n), g(n),
-  // gscale.  17 KB per wave.
+  // point and the elimination: A (9), x (11), dx (11), det pF(n), g(n), gscale.  17 KB per wave.
   __shared__ double sPk[34 * 64];
   double *pk = sPk + lane;  // field i at pk[i * 64]
   constexpr int kA = 0, kX = 9, kDX = 20, kDet = 31, kGn = 32, kGs = 33;
   const double dt = a.dt;
-  int it = 0, it_att = 0, gid = 0;
-  bool bad_start = false;
-  int kind = 0;  // the QP's start: 0 plain, 1 the caller's (learned), 2 the caller's, then the plain fallback
-  // the lane's phase: evaluate the start, a line-search trial x + alpha dx, or the full step
-  // after 40 halvings without a decrease
-  constexpr int kPhStart = 0, kPhTrial = 1, kPhFull = 2;
-  int phase = kPhStart, ls = 0;
-  double f0 = 0.0, alpha = 1.0;
   const CPMaterial cm = a.cpmats[0];  // one material for every CP point: wave-uniform, loaded once
-  for (;;) {
-    // refill the lanes that need a QP, in lane order, from the wave's range
-    const uint64_t mask = __ballot(need && !done);
-    const int nneed = __popcll(mask);
-    if (gq && nneed > 0) {  // claim nneed QPs from the global queue (wave-uniform branch)
-      const int leader = __ffsll((unsigned long long)mask) - 1;
-      long long base = 0;
-      if (lane == leader) base = (long long)atomicAdd(a.qnext, (unsigned long long)nneed);
-      cursor = __shfl(base, leader);
+  // the lane's phase: evaluate the start, a line-search trial x + alpha dx, the full step after 40
+  // halvings without a decrease, or x once more, for a step with a pivoting elimination
+  constexpr int kPhStart = 0, kPhTrial = 1, kPhFull = 2, kPhAgain = 3, kPhDone = 4;
+  int64_t q0 = int64_t(blockIdx.x) * chunk;
+  const int64_t q_hi = a.qnext ? a.nq : (q0 + chunk < a.nq ? q0 + chunk : a.nq);
+  for (;; q0 += 64) {
+    if (a.qnext) {
+      unsigned long long base = 0;
+      if (lane == 0) base = atomicAdd(a.qnext, 64ull);
+      q0 = int64_t(__shfl((long long)base, 0));
     }
-    if (need && !done) {
-      const int rank = __popcll(mask & ((uint64_t(1) << lane) - 1));
-      const int64_t cand = cursor + rank;
-      if (cand >= q_hi) {
-        done = true;
+    if (q0 >= q_hi) break;
+    const int64_t qg = a.qp_base + q0 + lane;
+    const bool live = q0 + lane < q_hi;
+    int kind = 0;  // the QP's start: 0 plain, 1 the caller's (learned), 2 the caller's, then the plain fallback
+    int phase = kPhDone, it = 0, it_att = 0, ls = 0;
+    bool bad_start = false, failed = false;
+    double f0 = 0.0, alpha = 1.0;
+    if (live) {
+      double F[9], pFn[9], pFi[9], T[9], A[9], det = 0.0;
+#pragma unroll
+      for (int i = 0; i < 9; ++i) {
+        F[i] = a.F_np1[i * NQ + qg];
+        pFn[i] = a.pF_n[i * NQ + qg];
+        pFi[i] = 0.0;
+      }
+      const double *R = a.grains[a.qgrain[q0 + lane]].R;
+      inv_det(pFn, pFi, det);
+      mul_ab(F, pFi, T);
+      rot_in_1(R, T, A);
+#pragma unroll
+      for (int i = 0; i < 9; ++i) pk[(kA + i) * 64] = A[i];
+      pk[kDet * 64] = det;
+      const double g_n = a.g_n[qg];
+      pk[kGn * 64] = g_n;
+      pk[kGs * 64] = 1.0 / (fabs(cm.gs0 - cm.g0) * g_n + 1e-300);
+      phase = kPhStart;
+      // start: the caller's warm start where cp_start_kernel chose it, else the plain start
+      const double *row = a.qpbuf + qrec(qg);
+      const int flag = int(row[kStartFlag * kRecStride]);
+      bad_start = (flag & 1) != 0;
+      if (flag & 2) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) T[i] = a.warm[i * NQ + qg];
+        rot_in_1(R, T, A);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) pk[(kX + i) * 64] = A[i];
+        pk[(kX + 9) * 64] = a.warm[9 * NQ + qg];
+        pk[(kX + 10) * 64] = a.warm[10 * NQ + qg];
+        kind = 1;
+        bad_start = false;
       } else {
-        q = cand;
-        need = false;
-        const int64_t qg = a.qp_base + q;
-        double F[9], pFn[9], pFi[9], A[9];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) {
-          F[i] = a.F_np1[i * NQ + qg];
-          pFn[i] = a.pF_n[i * NQ + qg];
-        }
-        inv3(pFn, pFi);
-        mm3(F, pFi, A);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) pk[(kA + i) * 64] = A[i];
-        pk[kDet * 64] = det3(pFn);
-        const double g_n = a.g_n[qg];
-        pk[kGn * 64] = g_n;
-        gid = a.qgrain[q];
-        pk[kGs * 64] = 1.0 / (fabs(cm.gs0 - cm.g0) * g_n + 1e-300);
-        it = 0;
-        it_att = 0;
-        phase = kPhStart;
-        // start: the caller's warm start where cp_start_kernel chose it, else the plain start
-        const double *row = a.qpbuf + qrec(qg);
-        const int flag = int(row[kStartFlag * kRecStride]);
-        bad_start = (flag & 1) != 0;
-        kind = 0;
-        if (flag & 2) {
-#pragma unroll
-          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = a.warm[i * NQ + qg];
-          kind = 1;
-          bad_start = false;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
-        }
+        for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
       }
     }
-    if (!gq) cursor += nneed;
-    if (__all(done)) break;
-    if (done || need) continue;
-
-    // ---- one turn of this lane's QP: every live lane evaluates the material point once, at its
-    // start or at its line-search trial x + alpha dx; a lane whose start or accepted trial this
-    // is then takes a Newton step from it.  A trial's evaluation is thus also the point of the
-    // next iteration (one evaluation per iteration, and none of it at a refill's masked width).
-    const DevGrain &gr = a.grains[gid];
-    const int64_t qg = a.qp_base + q;
-    bool fail = false, conv = false, step = false;
-    double xc[11], A[9];
+    // One turn: every live lane evaluates the material point once, at its start or at its
+    // line-search trial x + alpha dx; a lane whose start or accepted trial this is then takes a
+    // Newton step from it.  A trial's evaluation is thus also the point of the next iteration.
+    while (__any(phase != kPhDone)) {
+      // A step that asked for pivoting is taken in a turn of its own, in which the wave's other
+      // lanes wait: the choice of elimination is then the wave's, not the lane's.
+      const bool pivots = __builtin_amdgcn_readfirstlane(__any(phase == kPhAgain)) != 0;
+      const bool turn = pivots ? phase == kPhAgain : phase != kPhDone;
+      const bool moved = phase == kPhTrial || phase == kPhFull;
+      const double len = phase == kPhTrial ? alpha : (phase == kPhFull ? 1.0 : 0.0);
+      double xc[11], A[9];
 #pragma unroll
-    for (int i = 0; i < 11; ++i)
-      xc[i] = (phase == kPhStart) ? pk[(kX + i) * 64]
-                                  : pk[(kX + i) * 64] + (phase == kPhTrial ? alpha : 1.0) * pk[(kDX + i) * 64];
+      for (int i = 0; i < 11; ++i) {
+        const double x = pk[(kX + i) * 64], xm = x + len * pk[(kDX + i) * 64];
+        xc[i] = moved ? xm : x;
+      }
 #pragma unroll
-    for (int i = 0; i < 9; ++i) A[i] = pk[(kA + i) * 64];
-    CPPoint p;
-    const bool valid =
-        !(phase == kPhStart && bad_start) && cp_point<HE>(cm, gr, A, pk[kDet * 64], pk[kGn * 64], dt, xc, p);
-    if (phase == kPhStart) {
-      ++it;
-      ++it_att;
-      if (valid) step = true;
-      else fail = true;
-    } else {
-      bool accept = false;
-      if (phase == kPhTrial) {
-        accept = valid && cp_merit(p, pk[kGs * 64]) <= (1.0 - 1e-4 * alpha) * f0;
-        if (!accept) {
-          alpha *= 0.5;
-          if (++ls == 40) phase = kPhFull;  // no decrease found: the full step, if it is valid
-        }
-      } else {
-        accept = valid;
-        if (!valid) fail = true;
+      for (int i = 0; i < 9; ++i) A[i] = pk[(kA + i) * 64];
+      CPPoint p;
+      bool valid = cp_point<HE, FLOW>(cm, A, pk[kDet * 64], pk[kGn * 64], dt, xc, p);
+      valid = valid && !(phase == kPhStart && bad_start);
+      const double merit = cp_merit(p, pk[kGs * 64]);
+      const bool accept = turn && moved && valid && (phase == kPhFull || merit <= (1.0 - 1e-4 * alpha) * f0);
+      bool fail = turn && !valid && phase != kPhTrial;
+      if (turn && phase == kPhTrial && !accept) {
+        alpha *= 0.5;
+        if (++ls == 40) phase = kPhFull;  // no decrease found: the full step, if it is valid
       }
       if (accept) {
 #pragma unroll
         for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = xc[i];
-        if (it_att >= cm.maxit) {  // the end of the iteration that took this step
-          fail = true;
-        } else {
-          ++it;
-          ++it_att;
-          step = true;
+      }
+      // the iteration that took this step may have been the last
+      fail = fail || (accept && it_att >= cm.maxit);
+      const bool step = turn && !fail && (accept || (!moved && valid));
+      if (phase == kPhStart ? turn : (accept && step)) {
+        ++it;
+        ++it_att;
+      }
+      if (__builtin_amdgcn_readfirstlane(__any(step))) {
+        // The point of this step (the start, or the accepted trial) is x in LDS.  The slip sums are
+        // the widest stretch, so the residual waits in dx's slots and the frames are formed again
+        // from A and x afterwards; e then takes those slots over the elimination.
+        double Ah[81], u[2][9], f;
+        const double lam = pk[(kX + 9) * 64], rhs_s = -p.R[9], rhs_t = -p.R[10];
+        if (step) {
+          f0 = merit;
+#pragma unroll
+          for (int i = 0; i < 9; ++i) pk[(kDX + i) * 64] = p.R[i];
+        }
+        pin(p.S);
+        pin(p.sd);
+        LocalLin L;
+        end_stage();
+        cp_slip_sums<HE>(cm, p, p.sd, L);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) pin(L.G[r]);
+        pin(L.eq);
+        end_stage();
+        pk = reload(sPk, lane);
+        {
+          double M[9], Mi[9], eF[9], AtE[9], T[9], E9[9], E9e[9], c[9], dM;
+#pragma unroll
+          for (int i = 0; i < 9; ++i) {
+            M[i] = pk[(kX + i) * 64];
+            A[i] = pk[(kA + i) * 64];
+          }
+          inv_det(M, Mi, dM);
+          const double pJ = pk[kDet * 64] / dM, g = pk[(kX + 10) * 64], dl = dt * lam * pJ, mg = -1.0 / (cm.m * g);
+          mm3(A, M, eF);
+          mtm3(A, eF, AtE);
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const int r = i * 3 + j;
+              T[r] = Mi[j * 3 + i];
+              u[0][r] = pk[(kDX + r) * 64];
+              c[r] = mg * (u[0][r] - (M[r] - ((i == j) ? 1.0 : 0.0)) + dl * T[r]);  // N from the residual
+            }
+          cp_fold(cm, dt, g, pk[kGn * 64], p.gsum, p.gs, p.dgs, c, L);
+          f = L.f;
+          const double tf = rhs_t / f;
+          v6_to_9(L.eq, E9);
+          mm3(AtE, E9, E9e);
+#pragma unroll
+          for (int r = 0; r < 9; ++r) {
+            u[0][r] = -u[0][r] - c[r] * tf;
+            u[1][r] = -pJ * T[r];  // d
+          }
+          if (step) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) pk[(kDX + r) * 64] = L.es * E9e[r];
+          }
+          pin(u[0]);
+          pin(u[1]);
+#pragma unroll
+          for (int r = 0; r < 9; ++r) pin(L.G[r]);
+          end_stage();
+          cp_matrix(L, AtE, T, dl, Ah);
+        }
+        pin(Ah);
+        end_stage();
+        pk = reload(sPk, lane);
+        double system[9 * 11];
+        if (pivots) store_system<9, 2>(Ah, u, system);
+        bool solved = eliminate<9, 2>(Ah, u, kMaxMultStep);
+        if (pivots) solved = eliminate_pivot<9, 2>(system, u);
+        double M[9], Mi[9], dM, du = 0.0, dv = 0.0, ex = 0.0, dx[11];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) M[i] = pk[(kX + i) * 64];
+        inv_det(M, Mi, dM);
+        const double pJ = pk[kDet * 64] / dM;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const double d = -pJ * Mi[j * 3 + i];
+            du += d * u[0][i * 3 + j];
+            dv += d * u[1][i * 3 + j];
+          }
+        const double yd = (du - rhs_s) / dv;  // dt times the step's multiplier of b
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+          dx[i] = u[0][i] - yd * u[1][i];
+          ex += pk[(kDX + i) * 64] * dx[i];
+        }
+        dx[9] = yd / dt - lam / pJ * rhs_s;
+        dx[10] = (rhs_t - ex) / f;
+        double size = 0.0;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) size = fmax(size, fabs(dx[i]));
+        size = fmax(size, fabs(dx[9]) * dt);
+        size = fmax(size, fabs(dx[10]) / pk[kGn * 64]);
+        if (step) {
+          if (!solved) {
+            fail = pivots;  // singular
+            phase = kPhAgain;
+          } else if (size < cm.tol) {
+#pragma unroll
+            for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = pk[(kX + i) * 64] + dx[i];
+            phase = kPhDone;
+          } else {  // backtracking on half the squared residual norm, from the full step
+#pragma unroll
+            for (int i = 0; i < 11; ++i) pk[(kDX + i) * 64] = dx[i];
+            alpha = 1.0;
+            ls = 0;
+            phase = kPhTrial;
+          }
         }
       }
-    }
-    if (step) {
-      double Ah[81];
-      Border B;
-      // the point of this step (the start, or the accepted trial); the Jacobian reads lambda and g
-      double xj[11] = {};
-      xj[9] = pk[(kX + 9) * 64];
-      xj[10] = pk[(kX + 10) * 64];
-      cp_jacobian_re<HE>(cm, gr, dt, xj, A, p, pk[kGn * 64], Ah, B);
-      int piv[9];
-      if (!lu9(Ah, piv)) {
-        fail = true;
-      } else {
-        double v[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) v[i] = dt * B.d[i];  // b = dt d
-        lu9_solve(Ah, piv, v);
-        double dTv = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) dTv += B.d[i] * v[i];
-        double r9[9], dx[11];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) r9[i] = -p.R[i];
-        bordered_solve(Ah, piv, B, v, dTv, r9, -p.R[9], -p.R[10], dx);
-        double du = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) du = fmax(du, fabs(dx[i]));
-        du = fmax(du, fabs(dx[9]) * dt);
-        du = fmax(du, fabs(dx[10]) / pk[kGn * 64]);
-        if (du < cm.tol) {
-#pragma unroll
-          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = pk[(kX + i) * 64] + dx[i];
-          conv = true;
-        } else {  // backtracking on half the squared residual norm, from the full step
-#pragma unroll
-          for (int i = 0; i < 11; ++i) pk[(kDX + i) * 64] = dx[i];
-          f0 = cp_merit(p, pk[kGs * 64]);
-          alpha = 1.0;
-          ls = 0;
-          phase = kPhTrial;
-        }
-      }
-    }
-    if (fail && kind == 1) {
-      // the warm start did not converge: fall back to the plain start with a fresh budget
-      // (iterations keep counting)
-      kind = 2;
-      it_att = 0;
-      const double *row = a.qpbuf + qrec(qg);
-#pragma unroll
-      for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
-      bad_start = (int(row[kStartFlag * kRecStride]) & 1) != 0;
-      fail = false;
-      phase = kPhStart;
-    }
-    if (conv || fail) {
-      a.iters[qg] = it | (kind << 24);  // iterations, and the start in the high byte
       if (fail) {
+        if (kind == 1) {
+          // the warm start did not converge: fall back to the plain start with a fresh budget
+          // (iterations keep counting)
+          kind = 2;
+          it_att = 0;
+          const double *row = a.qpbuf + qrec(qg);
+#pragma unroll
+          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
+          bad_start = (int(row[kStartFlag * kRecStride]) & 1) != 0;
+          phase = kPhStart;
+        } else {
+          failed = true;
+          phase = kPhDone;
+        }
+      }
+    }
+    if (live) {
+      // read R and pF(n) again rather than keep them from the batch's start
+      int again = lane;
+      asm volatile("" : "+v"(again));
+      const int64_t q = q0 + again, qg = a.qp_base + q;
+      a.iters[qg] = it | (kind << 24);  // iterations, and the start in the high byte
+      if (failed) {
         atomicAdd(a.err, 1);
       } else {
         // pF(n+1) = M^-1 pF(n)
-        double x[11], Mi[9], pFn[9], pF1[9];
+        double x[11], Mc[9], Mi[9] = {}, pFn[9], pF1[9], det;
 #pragma unroll
         for (int i = 0; i < 11; ++i) x[i] = pk[(kX + i) * 64];
-        inv3(x, Mi);
+        rot_out_1(a.grains[a.qgrain[q]].R, x, Mc);
+        inv_det(Mc, Mi, det);
 #pragma unroll
         for (int i = 0; i < 9; ++i) pFn[i] = a.pF_n[i * NQ + qg];
-        mm3(Mi, pFn, pF1);
+        mul_ab(Mi, pFn, pF1);
 #pragma unroll
         for (int i = 0; i < 9; ++i) a.pF_np1[i * NQ + qg] = pF1[i];
         a.Sc_np1[qg] = x[10];
         a.Sc_np1[NQ + qg] = x[9];
       }
-      need = true;
     }
   }
 }
@@ -981,157 +1137,257 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
 // ------------------------------------------------------------------- tangent kernel
 // At the stored converged state (F, pF(n), pF(n+1), g, lambda): S, tau, gdot, Me, pJ and,
 // with WITH_D, dMe/dF = pF(n)^-1 dM/dF from the implicit derivative of the local system.
-template <bool HE, bool WITH_D>
+//
+// Column c = (i, j) of F moves the system like dM does, through six numbers: dtau_a/dF_c =
+// kR6 q_a . kappa_c with kappa_c the symmetric part of u (x) w, u row i of R eF and w row j of
+// R pF(n)^-1 M (products in the crystal frame, their outer index in the sample frame, where F
+// is).  So with the hardening row eliminated its right-hand side is -G kappa_c, and
+//   (B + G K) z_c = -G kappa_c,  B = I + lp T (.)^T T,
+//   z_c = -H (I + K H)^-1 kappa_c,  H = B^-1 G:
+// a 6 x 6 system serves the nine columns and the border's b, with no sum over slip systems and
+// no 9 x 9 factor.  lp is of the order of the squared strain increment (1e-7 at 1e-3), so H
+// comes by the series in lp, to the last bit.  A point where lp is not small, or where the
+// 6 x 6 elimination meets a multiplier above kMaxMultTangent, takes the 9 x 9 system with
+// pivoting.  998,250 QPs in 436 us instead of the 1066 us of the sample-frame kernel with its
+// pivoted 9 x 9 (and 28 instead of 61 us for 10,368, one wave per workgroup spread over the chip).
+constexpr double kMaxLp = 0.01;
+
+// X <- T X^T T scaled by c
+__device__ __forceinline__ void lp_term(const double *T, double c, double *X) {
+  double Y[9];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      Y[i * 3 + j] = c * (T[i * 3] * X[j * 3] + T[i * 3 + 1] * X[j * 3 + 1] + T[i * 3 + 2] * X[j * 3 + 2]);
+  mm3(Y, T, X);
+}
+// K X
+__device__ __forceinline__ void k_of(const double *AtE, const double *X, double *k) {
+  double Y[9];
+  mtm3(AtE, X, Y);
+#pragma unroll
+  for (int I = 0; I < 3; ++I) k[I] = Y[I * 4];
+  k[3] = Y[1] + Y[3];
+  k[4] = Y[5] + Y[7];
+  k[5] = Y[2] + Y[6];
+}
+__device__ __forceinline__ void kappa(const double *u, const double *w, double *k) {
+#pragma unroll
+  for (int I = 0; I < 3; ++I) k[I] = u[I] * w[I];
+  k[3] = u[0] * w[1] + u[1] * w[0];
+  k[4] = u[1] * w[2] + u[2] * w[1];
+  k[5] = u[0] * w[2] + u[2] * w[0];
+}
+
+struct TangentPoint {
+  double R[9], pFi[9], A[9], Me[9], x[11], pJ, g_n;
+  CPPoint p;
+};
+template <bool HE, int FLOW>
+__device__ __forceinline__ bool tangent_point(const CPArgs &a, const CPMaterial &cm, int64_t t, TangentPoint &q) {
+  const int64_t NQ = a.n_qp, qg = a.qp_base + t;
+  const double *R = a.grains[a.qgrain[t]].R;
+  double F[9], pFn[9], pF1[9], T[9], det_pFn;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    q.R[i] = R[i];
+    F[i] = a.F_np1[i * NQ + qg];
+    pFn[i] = a.pF_n[i * NQ + qg];
+    pF1[i] = a.pF_np1[i * NQ + qg];
+  }
+  q.g_n = a.g_n[qg];
+  if (!inv_det(pFn, q.pFi, det_pFn) || !inv_det(pF1, q.Me, q.pJ)) return false;
+  mul_ab(F, q.pFi, T);
+  rot_in_1(q.R, T, q.A);
+  mul_ab(pFn, q.Me, T);
+  rot_in_1(q.R, T, q.x);  // M = pF(n) pF(n+1)^-1
+  q.x[9] = a.Sc_np1[NQ + qg];
+  q.x[10] = a.Sc_np1[qg];
+  return cp_point<HE, FLOW>(cm, q.A, det_pFn, q.g_n, a.dt, q.x, q.p);
+}
+// U = R eF, W = R pF(n)^-1 M and R pF(n)^-1 (second indices in the crystal frame)
+__device__ __forceinline__ void tangent_frames(const TangentPoint &q, double *U, double *W, double *RpFi) {
+  double T[9];
+  mul_ab(q.R, q.p.eF, U);
+  mul_ab(q.pFi, q.R, RpFi);
+  mul_ab(RpFi, q.x, W);
+}
+// dMe/dF[:, c] = pF(n)^-1 dM/dF[:, c], from dM in the crystal frame
+__device__ __forceinline__ void store_dMe(const TangentPoint &q, const double *RpFi, const double *dM, int c, double *out) {
+  double H[9], D[9];
+  mm3(RpFi, dM, H);
+  mmt3(H, q.R, D);
+#pragma unroll
+  for (int r = 0; r < 9; ++r) out[(16 + c * 9 + r) * kRecStride] = D[r];
+}
+
+template <bool HE>
+__device__ __forceinline__ void tangent_lin(const CPMaterial &cm, double dt, const TangentPoint &q, double *AtE,
+                                            LocalLin &L) {
+  double c[9];
+  const double mg = -1.0 / (cm.m * q.x[10]);
+#pragma unroll
+  for (int r = 0; r < 9; ++r) c[r] = mg * q.p.N[r];
+  cp_slip_sums<HE>(cm, q.p, q.p.sd, L);
+  cp_fold(cm, dt, q.x[10], q.g_n, q.p.gsum, q.p.gs, q.p.dgs, c, L);
+  mtm3(q.A, q.p.eF, AtE);
+}
+// The nine columns by the 9 x 9 system with pivoting.  A function of its own, so that the common
+// path keeps nothing in registers for it.
+template <bool HE, int FLOW>
+__device__ __attribute__((noinline)) void tangent_pivot(CPArgs a, int64_t t) {
+  const CPMaterial cm = a.cpmats[0];
+  double *out = a.qpbuf + qrec(a.qp_base + t);
+  TangentPoint q;
+  tangent_point<HE, FLOW>(a, cm, t, q);
+  double U[9], W[9], RpFi[9], Y[10][9], system[9 * 19];
+  tangent_frames(q, U, W, RpFi);
+  {
+    double Ah[81], AtE[9];
+    LocalLin L;
+    tangent_lin<HE>(cm, a.dt, q, AtE, L);
+    cp_matrix(L, AtE, q.p.T, a.dt * q.x[9] * q.p.pJ, Ah);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+      double kp[6];
+      kappa(U + (c / 3) * 3, W + (c % 3) * 3, kp);
+#pragma unroll
+      for (int r = 0; r < 9; ++r) {
+        double s = 0.0;
+#pragma unroll
+        for (int I = 0; I < 6; ++I) s -= L.G[r][I] * kp[I];
+        Y[c][r] = s;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) Y[9][r] = q.p.T[r];
+    store_system<9, 10>(Ah, Y, system);
+  }
+  if (!eliminate_pivot<9, 10>(system, Y)) {
+    atomicAdd(a.err, 1);
+    return;
+  }
+  double dv = 0.0;
+#pragma unroll
+  for (int r = 0; r < 9; ++r) dv += q.p.T[r] * Y[9][r];
+#pragma unroll
+  for (int c = 0; c < 9; ++c) {
+    double du = 0.0, dM[9];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) du += q.p.T[r] * Y[c][r];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) dM[r] = Y[c][r] - du / dv * Y[9][r];
+    store_dMe(q, RpFi, dM, c, out);
+  }
+}
+
+template <bool HE, int FLOW, bool WITH_D>
 __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
-  // the Q_a of the twelve systems, formed once for the right-hand sides and read back by the
-  // Jacobian (lane-fastest: conflict-free)
-  __shared__ double sQ[WITH_D ? 72 * 64 : 1];
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= nqb) return;
   const int64_t NQ = a.n_qp;
   const int64_t qg = a.qp_base + t;
   const CPMaterial cm = a.cpmats[0];
-  const DevGrain &gr = a.grains[a.qgrain[t]];
-  double F[9], pFn[9], pF1[9], pFi[9], A[9], Me[9], x[11];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) {
-    F[i] = a.F_np1[i * NQ + qg];
-    pFn[i] = a.pF_n[i * NQ + qg];
-    pF1[i] = a.pF_np1[i * NQ + qg];
-  }
-  bool ok = inv3(pFn, pFi) && inv3(pF1, Me);
-  mm3(F, pFi, A);
-  mm3(pFn, Me, x);  // M = pF(n) pF(n+1)^-1
-  x[9] = a.Sc_np1[NQ + qg];
-  x[10] = a.Sc_np1[qg];
-  const double g_n = a.g_n[qg];
-  CPPoint p;
-  ok = ok && cp_point<HE>(cm, gr, A, det3(pFn), g_n, a.dt, x, p);
   double *out = a.qpbuf + qrec(qg);  // field i at out[i * kRecStride]
-  if (!ok) {
+  TangentPoint q;
+  if (!tangent_point<HE, FLOW>(a, cm, t, q)) {
     atomicAdd(a.err, 1);
 #pragma unroll
     for (int i = 0; i < kCPBuf; ++i) out[i * kRecStride] = 0.0;
     return;
   }
-  const double expo = 1.0 / cm.m - 1.0;
-  const double rg = 1.0 / x[10], cdg = cm.gd0 * rg / cm.m;
-  for (int al = 0; al < 12; ++al) {  // tau and gamma_dot as cp_point evaluates them
-    const double tt = resolved(gr, al, p.Sig);
-    const double r = tt * rg;
-    a.tau[al * NQ + qg] = tt;
-    a.gdot[al * NQ + qg] = cm.gd0 * r * flow_pow(fabs(r), expo, cm.ipow);
-  }
-  // elastic PK2 from the stored state (eF = F pF(n+1)^-1)
-  double eF[9], Ce[9], S[6];
-  mm3(F, Me, eF);
-  mtm3(eF, eF, Ce);
+  const CPPoint &p = q.p;
   {
-    HeTan ht;
-    el_stress<HE>(cm, gr, eF, Ce, S, ht);
-  }
-#pragma unroll
-  for (int i = 0; i < 9; ++i) out[i * kRecStride] = Me[i];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) out[(9 + i) * kRecStride] = S[i];
-  out[15 * kRecStride] = det3(pF1);
-  if constexpr (WITH_D) {
-    // dtau_a/dF = A^-T D_a (pF(n)^-1 M)^T with D_a = 2 A^T eF Q_a, so dtau_a/dF = 2 eF Q_a BM^T
-    // (BM = pF(n)^-1 M).  Column c = (i, j) of F has the right-hand side
-    // rhs[r] = sum_a co_a P_a[r] q_a and the hardening row -sum_a sg_a q_a, with
-    // q_a = 2 (eF Q_a BM^T)_ij = 2 (Q_a u).w (u = row i of eF, w = row j of BM).  They are formed
-    // after the factorization from the Q_a in LDS, three columns (one row of eF) at a time, so
-    // no accumulator over the slip systems is live across the Jacobian and its LU.
-    double BM[9];
-    mm3(pFi, x, BM);
-    // d gamma_dot_a / d tau_a, with the sign of gamma_dot_a (co_a = -dt |dg_a|, sg_a = dg_a)
-    double dg[12];
+    const double rg = 1.0 / q.x[10];
 #pragma unroll
     for (int al = 0; al < 12; ++al) {
-      double Q[6];
-      qsym<HE>(gr, al, p, Q);
-#pragma unroll
-      for (int I = 0; I < 6; ++I) sQ[(al * 6 + I) * 64 + threadIdx.x] = Q[I];
-      const double tt = resolved(gr, al, p.Sig);
-      const double rr = tt * rg;
-      const double pw = flow_pow(fabs(rr), expo, cm.ipow);
-      const double dgdt = cdg * pw;
-      dg[al] = (cm.gd0 * rr * pw < 0) ? -dgdt : dgdt;
+      a.tau[al * NQ + qg] = p.tau[al];
+      a.gdot[al * NQ + qg] = (fabs(p.sd[al]) * cm.m * q.x[10]) * (p.tau[al] * rg);
     }
-    // the local Jacobian at the converged point, factored once for the ten solves
-    double Ah[81];
-    Border B;
-    cp_jacobian_re<HE, true>(cm, gr, a.dt, x, A, p, g_n, Ah, B, sQ + threadIdx.x);
-    int piv[9];
-    if (!lu9(Ah, piv)) {
-      atomicAdd(a.err, 1);
-      return;
-    }
-    double v[9];
+    double S9[9], S[9];
+    v6_to_9(p.S, S9);
+    rot_out(q.R, S9, S);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) v[i] = B.b[i];
-    lu9_solve(Ah, piv, v);
-    double dTv = 0.0;
+    for (int i = 0; i < 9; ++i) out[i * kRecStride] = q.Me[i];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) dTv += B.d[i] * v[i];
+    for (int I = 0; I < 6; ++I) out[(9 + I) * kRecStride] = S[voigt_i(I) * 3 + voigt_j(I)];
+    out[15 * kRecStride] = q.pJ;
+  }
+  if constexpr (WITH_D) {
+    LocalLin L;
+    double AtE[9];
+    tangent_lin<HE>(cm, a.dt, q, AtE, L);
+    const double lp = a.dt * q.x[9] * p.pJ;
+    double v[9];  // B^-1 T, T the border's b and d up to factors
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const double *u = p.eF + i * 3;
-      double rhs[3][9], rgc[3];
+    for (int r = 0; r < 9; ++r) v[r] = p.T[r];
+    bool ok = fabs(lp) <= kMaxLp;
+    {  // H = B^-1 G and v by the series sum (-lp)^k (T (.)^T T)^k
+      double tv[9], size = fabs(lp);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        rgc[j] = 0.0;
+      for (int r = 0; r < 9; ++r) tv[r] = v[r];
+      for (double sz = size; ok && sz > 1e-17; sz *= 2.0 * size) {
+        lp_term(p.T, -lp, tv);
 #pragma unroll
-        for (int r = 0; r < 9; ++r) rhs[j][r] = 0.0;
+        for (int r = 0; r < 9; ++r) v[r] += tv[r];
       }
-      // the slip directions and plane normals read where used: with the grain's address visible
-      // the compiler keeps the Jacobian's loads of them live through the LU, and spills
-      const DevGrain &go = *reinterpret_cast<const DevGrain *>(opaque(reinterpret_cast<const double *>(&gr)));
-      // P_a = s_a (x) m_a: the three systems of plane k summed (vs = sum co_a q_a s_a) before
-      // the outer product with m_k
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        double vs[3][3];
+      for (int I = 0; I < 6; ++I) {
+        double h[9], th[9];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) vs[j][0] = vs[j][1] = vs[j][2] = 0.0;
+        for (int r = 0; r < 9; ++r) h[r] = th[r] = L.G[r][I];
+        for (double sz = size; ok && sz > 1e-17; sz *= 2.0 * size) {
+          lp_term(p.T, -lp, th);
 #pragma unroll
-        for (int al = 3 * k; al < 3 * k + 3; ++al) {
-          double Q[6];
-#pragma unroll
-          for (int I = 0; I < 6; ++I) Q[I] = sQ[(al * 6 + I) * 64 + threadIdx.x];
-          const double Qu[3] = {Q[0] * u[0] + Q[3] * u[1] + Q[5] * u[2], Q[3] * u[0] + Q[1] * u[1] + Q[4] * u[2],
-                                Q[5] * u[0] + Q[4] * u[1] + Q[2] * u[2]};
-          const double cad = -a.dt * fabs(dg[al]);
-#pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            const double *w = BM + j * 3;
-            const double q = 2.0 * (Qu[0] * w[0] + Qu[1] * w[1] + Qu[2] * w[2]);
-            const double ta = cad * q;
-            rgc[j] -= dg[al] * q;
-#pragma unroll
-            for (int l = 0; l < 3; ++l) vs[j][l] += ta * go.s[al][l];
-          }
+          for (int r = 0; r < 9; ++r) h[r] += th[r];
         }
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-          for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int n = 0; n < 3; ++n) rhs[j][l * 3 + n] += vs[j][l] * go.m[k][n];
+        for (int r = 0; r < 9; ++r) L.G[r][I] = h[r];
       }
+    }
+    double U[9], W[9], RpFi[9], S6[36], Y[10][6];
+    tangent_frames(q, U, W, RpFi);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const int c = i * 3 + j;
-        double sol[11];
-        bordered_solve(Ah, piv, B, v, dTv, rhs[j], 0.0, B.dRg * rgc[j], sol);
-        // dMe/dF[:, c] = pF(n)^-1 dM/dF[:, c]
+    for (int I = 0; I < 6; ++I) {
+      double h[9], k6[6];
 #pragma unroll
-        for (int ii = 0; ii < 3; ++ii)
+      for (int r = 0; r < 9; ++r) h[r] = L.G[r][I];
+      k_of(AtE, h, k6);
 #pragma unroll
-          for (int jj = 0; jj < 3; ++jj)
-            out[(16 + c * 9 + ii * 3 + jj) * kRecStride] =
-                pFi[ii * 3 + 0] * sol[0 * 3 + jj] + pFi[ii * 3 + 1] * sol[1 * 3 + jj] + pFi[ii * 3 + 2] * sol[2 * 3 + jj];
+      for (int J = 0; J < 6; ++J) S6[J * 6 + I] = k6[J] + (I == J ? 1.0 : 0.0);
+    }
+#pragma unroll
+    for (int c = 0; c < 9; ++c) kappa(U + (c / 3) * 3, W + (c % 3) * 3, Y[c]);
+    k_of(AtE, v, Y[9]);
+    ok = eliminate<6, 10>(S6, Y, kMaxMultTangent) && ok;
+    if (!ok) {
+      tangent_pivot<HE, FLOW>(a, t);
+      return;
+    }
+    double dv = 0.0;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+#pragma unroll
+      for (int I = 0; I < 6; ++I) v[r] -= L.G[r][I] * Y[9][I];
+      dv += p.T[r] * v[r];
+    }
+    const double rdv = 1.0 / dv;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+      double dM[9], du = 0.0;
+#pragma unroll
+      for (int r = 0; r < 9; ++r) {
+        double z = 0.0;
+#pragma unroll
+        for (int I = 0; I < 6; ++I) z -= L.G[r][I] * Y[c][I];
+        dM[r] = z;
+        du += p.T[r] * z;
       }
+      du *= rdv;
+#pragma unroll
+      for (int r = 0; r < 9; ++r) dM[r] -= du * v[r];
+      store_dMe(q, RpFi, dM, c, out);
     }
   }
 }
@@ -2040,9 +2296,16 @@ __global__ __launch_bounds__(256) void output_kernel(OutArgs o) {
       inv3(pF, pFi);
       mm3(F, pFi, eF);
       mtm3(eF, eF, Ce);
-      HeTan t;
-      if (cm.law == 1) el_stress<true>(cm, o.grains[o.qgrain[q - o.qp_base]], eF, Ce, S6, t);
-      else el_stress<false>(cm, o.grains[o.qgrain[q - o.qp_base]], eF, Ce, S6, t);
+      if (cm.law == 1) {
+        HeTan t;
+        he_law(cm, eF, Ce, S6, t);
+      } else {
+        double E[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) E[i] = 0.5 * (Ce[i] - ((i % 4 == 0) ? 1.0 : 0.0));
+        const double cub[3] = {cm.c11m12, cm.c12, cm.c44x2};
+        cubic_dot(o.grains[o.qgrain[q - o.qp_base]].R, cub, E, S6);
+      }
       v6_to_9(S6, S9);
       const double rte = 1.0 / det3(eF);
       mm3(eF, S9, T);
@@ -2226,6 +2489,18 @@ __global__ void cp_queue_reset(unsigned long long *q) { *q = 0; }
 // resident waves of the persistent Newton kernel on an MI355X: 256 CUs x 4 SIMDs, one wave each
 constexpr int64_t kQueueWaves = 1024;
 
+// run(HE, FLOW) for the material's elastic law and flow rule
+template <class F>
+void by_law(const CPArgs &a, F run) {
+  const auto flow = [&](auto he) {
+    if (a.flow == kFlowPlain) run(he, std::integral_constant<int, kFlowPlain>{});
+    else if (a.flow == kFlowSat) run(he, std::integral_constant<int, kFlowSat>{});
+    else run(he, std::integral_constant<int, kFlowPow>{});
+  };
+  if (a.law == 1) flow(std::true_type{});
+  else flow(std::false_type{});
+}
+
 void launch_cp_newton(const CPArgs &a, int64_t chunk, hipStream_t s) {
   const int64_t nq = a.nq;
   if (nq <= 0) return;
@@ -2240,26 +2515,25 @@ void launch_cp_newton(const CPArgs &a, int64_t chunk, hipStream_t s) {
   const unsigned grid = a.qnext ? unsigned(std::min<int64_t>((nq + 63) / 64, kQueueWaves))
                                 : unsigned((nq + chunk - 1) / chunk);
   const unsigned sgrid = unsigned((nq + 63) / 64);
-  if (a.law == 1) {
-    cp_start_kernel<true><<<sgrid, 64, 0, s>>>(a);
-    cp_newton<true><<<grid, 64, 0, s>>>(a, chunk);
-  } else {
-    cp_start_kernel<false><<<sgrid, 64, 0, s>>>(a);
-    cp_newton<false><<<grid, 64, 0, s>>>(a, chunk);
-  }
+  const auto run = [&](auto he, auto fl) {
+    constexpr bool HE = decltype(he)::value;
+    constexpr int FLOW = decltype(fl)::value;
+    cp_start_kernel<HE, FLOW><<<sgrid, 64, 0, s>>>(a);
+    cp_newton<HE, FLOW><<<grid, 64, 0, s>>>(a, chunk);
+  };
+  by_law(a, run);
 }
 
 void launch_cp_tangent(const CPArgs &a, bool with_D, hipStream_t s) {
   const int64_t nq = a.nq;
   if (nq <= 0) return;
   const unsigned grid = unsigned((nq + 63) / 64);
-  if (a.law == 1) {
-    if (with_D) cp_tangent<true, true><<<grid, 64, 0, s>>>(a, nq);
-    else cp_tangent<true, false><<<grid, 64, 0, s>>>(a, nq);
-  } else {
-    if (with_D) cp_tangent<false, true><<<grid, 64, 0, s>>>(a, nq);
-    else cp_tangent<false, false><<<grid, 64, 0, s>>>(a, nq);
-  }
+  by_law(a, [&](auto he, auto fl) {
+    constexpr bool HE = decltype(he)::value;
+    constexpr int FLOW = decltype(fl)::value;
+    if (with_D) cp_tangent<HE, FLOW, true><<<grid, 64, 0, s>>>(a, nq);
+    else cp_tangent<HE, FLOW, false><<<grid, 64, 0, s>>>(a, nq);
+  });
 }
 
 void launch_cp_elem(int nne, int mode, const CPElemArgs &a, int64_t e0, int64_t e1, hipStream_t s) {

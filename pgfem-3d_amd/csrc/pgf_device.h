@@ -107,16 +107,15 @@ enum : int { MODE_INTEGRATE = 1, MODE_RESIDUAL = 2, MODE_TANGENT = 4, MODE_DEFL_
 struct DevGrain {
   double P[12][9];
   double Lv[36];
-  double s[12][3];  // slip directions in the sample frame; P_a = s_a (x) m[a / 3]
-  double m[4][3];   // the four slip-plane normals (systems 3k..3k+2 share plane k)
-  double R[9];                // crystal -> sample rotation
-  double cub[3];              // cubic constants C11 - C12, C12, 2 C44 (crystal frame)
+  double R[9];  // crystal -> sample rotation
 };
 
 // law 0: cubic St Venant-Kirchhoff through the grain's Lv; law 1: neo-Hookean deviatoric part
 // (m10) and the volumetric potential vol_flag (kappa) on the elastic part eF.
 struct CPMaterial {
   double gd0, m, h0, g0, gs0, gds, w, tol;
+  double c11m12, c12, c44x2;  // law 0: C11 - C12, C12, 2 C44
+  double expo, gd0_m;         // 1/m - 1, gd0 / m
   double m10, kappa;
   int32_t maxit, law, vol_flag;
   int32_t ipow;  // 1/m - 1 when it is a whole number in [0, 64] (binary powering), else -1
@@ -152,6 +151,7 @@ struct CPArgs {
   int32_t *err;
   unsigned long long *qnext;  // global work queue of the local Newton (cp_chunk = 1), else null
   int32_t law;                // cpmats[0].law, read on the host to pick the kernels
+  int32_t flow;               // likewise: 2 cpmats[0].ipow >= 0 and w = 0, 1 ipow >= 0, 0 neither
   // three-field (CM3F) blocks: per block element theta = tf_V + tf_dV; the kinematics then
   // stores the model's F(n+1) = (theta/J)^(1/3) F.  Null otherwise.
   const double *tf_V, *tf_dV;
