@@ -103,9 +103,8 @@ void rot_to_quat(const double *R, float *q) {
 }
 
 // Host tables of one grain: the 12 FCC {111}<110> systems (unit slip direction s and plane
-// normal m, Schmid tensor s (x) m) and the cubic stiffness, both rotated by R (crystal ->
-// sample frame).
-void make_grain(const double *R, double C11, double C12, double C44, DevGrain &g) {
+// normal m, Schmid tensor s (x) m) rotated by R (crystal -> sample frame).
+void make_grain(const double *R, DevGrain &g) {
   const double n[4][3] = {{1, 1, 1}, {-1, 1, 1}, {1, -1, 1}, {1, 1, -1}};
   const double sd[12][3] = {{0, 1, -1}, {-1, 0, 1}, {1, -1, 0}, {0, 1, -1}, {1, 0, 1}, {1, 1, 0},
                             {0, 1, 1},  {1, 0, -1}, {1, 1, 0},  {0, 1, 1},  {1, 0, 1}, {1, -1, 0}};
@@ -119,25 +118,7 @@ void make_grain(const double *R, double C11, double C12, double C44, DevGrain &g
     for (int i = 0; i < 3; ++i)
       for (int j = 0; j < 3; ++j) g.P[a][i * 3 + j] = s[i] * m[j];
   }
-  auto L0 = [&](int i, int j, int k, int l) {
-    double v = 0.0;
-    if (i == j && k == l) v += (i == k) ? C11 : C12;
-    if (i != j && ((i == k && j == l) || (i == l && j == k))) v += C44;
-    return v;
-  };
   for (int i = 0; i < 9; ++i) g.R[i] = R[i];
-  static const int vi[6] = {0, 1, 2, 0, 1, 0}, vj[6] = {0, 1, 2, 1, 2, 2};
-  for (int I = 0; I < 6; ++I)
-    for (int J = 0; J < 6; ++J) {
-      const int i = vi[I], j = vj[I], k = vi[J], l = vj[J];
-      double v = 0.0;
-      for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b)
-          for (int c = 0; c < 3; ++c)
-            for (int d = 0; d < 3; ++d)
-              v += R[i * 3 + a] * R[j * 3 + b] * R[k * 3 + c] * R[l * 3 + d] * L0(a, b, c, d);
-      g.Lv[I * 6 + J] = v * (J < 3 ? 1.0 : 2.0);  // tensor-component E: shear pairs count twice
-    }
 }
 
 }  // namespace pgf
@@ -241,7 +222,6 @@ struct pgf_handle_s {
   float *d_norm = nullptr;     // shift [34], scale [34], out_scale [12]
   float *d_feat = nullptr;     // [n_qp][34]
   double *d_sur_warm = nullptr;  // [11][n_qp]
-  std::vector<double> cp_mat_host;  // C11, C12, C44
   // hipGraph of a whole pass
   bool use_graph = false;
   hipGraphExec_t gexec = nullptr;
@@ -342,6 +322,7 @@ pgf::CPArgs cp_args(pgf_handle h, const Block &b, const pgf_nodal_input *in) {
   c.err = h->d_err;
   c.law = h->cp_law;
   c.flow = h->cp_flow;
+  c.tf = h->tf ? 1 : 0;
   if (h->tf && b.ne > 0 && b.model == PGF_MODEL_CRYSTAL_PLASTICITY) {  // CM3F: the kinematics scales F
     c.tf_V = h->d_tf + b.e_base;
     c.tf_dV = h->d_tf + 6 * h->n_elem + b.e_base;
@@ -368,9 +349,17 @@ pgf::CPArgs cp_args_all(pgf_handle h, const pgf_nodal_input *in) {
 void cp_prepass(pgf_handle h, const pgf_nodal_input *in, int mode) {
   if (!h->cp_nq) return;
   pgf::CPArgs all = cp_args_all(h, in);
-  if (mode & pgf::MODE_INTEGRATE) {
+  if (mode & pgf::MODE_INTEGRATE) all.kin |= pgf::kKinState;
+  if (mode & pgf::MODE_DEFL_LOAD) all.kin |= pgf::kKinDefl;
+  if (!h->tf && (mode & (pgf::MODE_RESIDUAL | pgf::MODE_TANGENT))) all.kin |= pgf::kKinRec;
+  if (all.kin & (pgf::kKinState | pgf::kKinRec))
     for (auto &b : h->blocks)
-      if (b.model == PGF_MODEL_CRYSTAL_PLASTICITY) pgf::launch_cp_kinematics(b.nne, cp_args(h, b, in), h->stream);
+      if (b.model == PGF_MODEL_CRYSTAL_PLASTICITY) {
+        pgf::CPArgs c = cp_args(h, b, in);
+        c.kin = all.kin;
+        pgf::launch_cp_kinematics(b.nne, c, h->stream);
+      }
+  if (mode & pgf::MODE_INTEGRATE) {
     if (h->sur && !h->warm) {  // learned start: features -> MLP -> (M, lambda, g)
       pgf::launch_cp_features(all, h->d_gquat, h->d_norm, h->d_norm + 34, h->d_feat, h->stream);
       const float *Y = nullptr;
@@ -515,11 +504,8 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
         ce.row_start = h->d_row_start;
         ce.rowlen = h->d_rowlen;
         ce.conn = b.d_conn;
-        ce.grain = b.d_egrain;
         ce.off = b.d_off;
-        ce.grains = h->d_grains;
         ce.cpmats = h->d_cpmat;
-        ce.law = h->cp_law;
         ce.qpbuf = h->d_qpbuf;  // indexed by device QP (pgf::qrec)
         ce.qp_base = b.qp_base;
         ce.r = in->r;
@@ -1117,7 +1103,6 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     h->cp_g0 = cpm.g0;
     h->cp_law = cpm.cp_elastic;
     h->cp_flow = c.ipow < 0 ? 0 : (c.w != 0.0 ? 1 : 2);
-    h->cp_mat_host = {cpm.C11, cpm.C12, cpm.C44};
     if ((rc = pgf::upload(&h->d_cpmat, &c, 1))) return fail(rc);
     for (int t = 0; t < 2; ++t) {
       if ((rc = pgf::dalloc(&h->d_tau[t], size_t(h->n_qp) * 12))) return fail(rc);
@@ -1533,6 +1518,7 @@ int pgf_tf_initial(pgf_handle h, const pgf_nodal_input *in_n, const pgf_nodal_in
       // compute_cm_initial_conditions, src/constitutive_model.cc:4097-4105)
       pgf::CPArgs c = cp_args(h, b, in);
       c.F_np1 = h->d_F[s == 0 ? 1 : 2];
+      c.kin = pgf::kKinState;
       c.tf_V = c.tf_dV = nullptr;
       pgf::launch_cp_kinematics(b.nne, c, h->stream);
     }
@@ -1713,7 +1699,7 @@ int pgf_set_orientations(pgf_handle h, int32_t n_grains, const double *R, const 
   std::vector<pgf::DevGrain> g(n_grains);
   std::vector<float> q(size_t(n_grains) * 4);
   for (int32_t k = 0; k < n_grains; ++k) {
-    pgf::make_grain(R + 9 * k, h->cp_mat_host[0], h->cp_mat_host[1], h->cp_mat_host[2], g[k]);
+    pgf::make_grain(R + 9 * k, g[k]);
     pgf::rot_to_quat(R + 9 * k, q.data() + 4 * k);
   }
   std::vector<std::vector<int32_t>> egs(h->blocks.size()), qgs(h->blocks.size());

@@ -26,13 +26,13 @@
 //   cp_kinematics  F(n+1) at every QP of a block (gather of the element nodes)
 //   cp_start_kernel  the starting points (and the choice of a caller's start), one per lane
 //   cp_newton      persistent: each wave works through a QP range, 64 QPs at a time
-//   cp_tangent     at the converged state: S, tau, gdot and dMe/dF (Me = pF(n+1)^-1), for the
-//                  element kernel (qpbuf)
-//   cp_elem        coloured element rows: the reference contraction (compute_stiffness_matrix,
-//                  src/constitutive_model.cc:1520-1616) regrouped per row (a,b) as
-//                  K_ab,wg = pJ w [ z_ab : (e_g (x) dN_w) + (Fr W_ab dN_w)_g + d_bg dN_a.Sh.dN_w ]
-//                  with Z_ab = Cr Me Y + 2 sAA Me S - (B:S) Me^-T, z_ab = Z_ab : dMe/dF,
-//                  B = Me^T sAA Me, Y = L:B, W = Me Y Me^T, Sh = Me S Me^T, Cr = Fr^T Fr.
+//   cp_tangent     at the converged state: tau, gdot, and per point the stress and the moduli that
+//                  the element kernel contracts (qpbuf); for the three-field element Me, S, pJ
+//                  and dMe/dF (Me = pF(n+1)^-1)
+//   cp_elem        element rows: the reference contraction (compute_stiffness_matrix,
+//                  src/constitutive_model.cc:1520-1616) is linear in the two gradients, so it is
+//                  f_ab = sum_j T_bj dN_a,j, K_ab,wg = sum_jl dN_a,j A[b j][g l] dN_w,l with the
+//                  first Piola-Kirchhoff stress T and its derivative A, formed per point
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -72,23 +72,6 @@ __device__ __forceinline__ void mmt3(const double *A, const double *B, double *C
 #pragma unroll
     for (int j = 0; j < 3; ++j) C[i * 3 + j] = A[i * 3] * B[j * 3] + A[i * 3 + 1] * B[j * 3 + 1] + A[i * 3 + 2] * B[j * 3 + 2];
 }
-// S (Voigt tensor comps) = Lv : E, E symmetric 3x3 given as full 3x3
-__device__ __forceinline__ void lv_dot(const double *Lv, const double *E9, double *S6) {
-  const double e[6] = {E9[0], E9[4], E9[8], 0.5 * (E9[1] + E9[3]), 0.5 * (E9[5] + E9[7]), 0.5 * (E9[2] + E9[6])};
-#pragma unroll
-  for (int I = 0; I < 6; ++I) {
-    double s = 0.0;
-#pragma unroll
-    for (int J = 0; J < 6; ++J) s += Lv[I * 6 + J] * e[J];
-    S6[I] = s;
-  }
-}
-// S (Voigt tensor comps) = L : sym(X) for the grain's cubic stiffness, through the crystal
-// frame: E' = R^T sym(X) R, S'_ii = (C11 - C12) E'_ii + C12 tr E', S'_ij = 2 C44 E'_ij,
-// S = R S' R^T.  12 numbers of the grain (R and the constants) instead of the 36 of its rotated
-// stiffness; the same tensor up to rounding.  Every multiply-add is an explicit fma and nothing
-// else is contracted, so the result does not depend on the code around a call (the residual
-// and the fused residual-tangent passes give the same bits).
 __device__ __forceinline__ double fma3(double a0, double b0, double a1, double b1, double a2, double b2) {
 #pragma clang fp contract(off)
   return __builtin_fma(a0, b0, __builtin_fma(a1, b1, a2 * b2));
@@ -625,7 +608,7 @@ __device__ __forceinline__ bool eliminate(double (&A)[N * N], double (&B)[NR][N]
 }
 // The same with partial pivoting, in scratch memory: rare, and kept from costing the common path
 // registers (the system is stored before the common path consumes it, and solved after it).
-// False for a singular matrix.
+// The solutions take the right-hand sides' places; false for a singular matrix.
 template <int N, int NR>
 __device__ __forceinline__ void store_system(const double (&A)[N * N], const double (&B)[NR][N], double *a) {
   constexpr int W = N + NR;
@@ -638,7 +621,7 @@ __device__ __forceinline__ void store_system(const double (&A)[N * N], const dou
   }
 }
 template <int N, int NR>
-__device__ __forceinline__ bool eliminate_pivot(double *a, double (&B)[NR][N]) {
+__device__ __forceinline__ bool eliminate_pivot(double *a) {
   constexpr int W = N + NR;
   bool ok = true;
 #pragma unroll 1
@@ -667,10 +650,6 @@ __device__ __forceinline__ bool eliminate_pivot(double *a, double (&B)[NR][N]) {
       for (int j = 0; j < W; ++j) a[i * W + j] -= l * row[j];
     }
   }
-#pragma unroll
-  for (int q = 0; q < NR; ++q)
-#pragma unroll
-    for (int i = 0; i < N; ++i) B[q][i] = a[i * W + N + q];
   return ok;
 }
 
@@ -751,7 +730,8 @@ __global__ __launch_bounds__(256) void cp_kinematics(CPArgs a) {
       const int32_t d = a.dofid[int64_t(node) * 3 + b];
       double uu = 0.0;  // def_elem_total, src/utils.cc:1391-1412
       if (d > 0) uu = a.r[d - 1] + (a.d_r ? a.d_r[d - 1] : 0.0);
-      else if (d < 0) uu = (a.defl ? a.defl[-d - 1] : 0.0) + (a.defl_d ? a.defl_d[-d - 1] : 0.0);
+      else if (d < 0)  // the prescribed-load pass takes K at defl
+        uu = (a.defl ? a.defl[-d - 1] : 0.0) + (a.defl_d && !(a.kin & kKinDefl) ? a.defl_d[-d - 1] : 0.0);
       u[n * 3 + b] = uu;
     }
   }
@@ -766,8 +746,9 @@ __global__ __launch_bounds__(256) void cp_kinematics(CPArgs a) {
     for (int ib = 0; ib < 3; ++ib)
 #pragma unroll
       for (int ic = 0; ic < 3; ++ic) dX[ib * 3 + ic] += dN[n * 3 + ic] * x[n * 3 + ib];
-  double Xi[9];
-  const bool ok = det3(dX) > 0.0 && inv3(dX, Xi);
+  double Xi[9] = {};
+  const double J0 = det3(dX);
+  const bool ok = J0 > 0.0 && inv3(dX, Xi);
   double F[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
 #pragma unroll
   for (int n = 0; n < NNE; ++n) {
@@ -781,6 +762,18 @@ __global__ __launch_bounds__(256) void cp_kinematics(CPArgs a) {
       for (int ic = 0; ic < 3; ++ic) F[ib * 3 + ic] += u[n * 3 + ib] * g[ic];
   }
   const int64_t q = a.qp_base + tq;
+  if (a.kin & kKinRec) {
+    double *rec = a.qpbuf + qrec(q);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) rec[(kRecXi + i) * kRecStride] = Xi[i];
+    rec[kRecW * kRecStride] = ok ? J0 * wt : 0.0;
+    if (!ok) atomicAdd(a.err, 1);
+    if (!(a.kin & kKinState)) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) rec[i * kRecStride] = F[i];
+    }
+  }
+  if (!(a.kin & kKinState)) return;
   const double J = det3(F);
   bool okF = ok && J > 0.0;  // getJacobian, src/utils.cc:513-527
   if (a.tf_V) {
@@ -1046,7 +1039,14 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
         double system[9 * 11];
         if (pivots) store_system<9, 2>(Ah, u, system);
         bool solved = eliminate<9, 2>(Ah, u, kMaxMultStep);
-        if (pivots) solved = eliminate_pivot<9, 2>(system, u);
+        if (pivots) {
+          solved = eliminate_pivot<9, 2>(system);
+#pragma unroll
+          for (int i = 0; i < 9; ++i) {
+            u[0][i] = system[i * 11 + 9];
+            u[1][i] = system[i * 11 + 10];
+          }
+        }
         double M[9], Mi[9], dM, du = 0.0, dv = 0.0, ex = 0.0, dx[11];
 #pragma unroll
         for (int i = 0; i < 9; ++i) M[i] = pk[(kX + i) * 64];
@@ -1148,8 +1148,10 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
 // no 9 x 9 factor.  lp is of the order of the squared strain increment (1e-7 at 1e-3), so H
 // comes by the series in lp, to the last bit.  A point where lp is not small, or where the
 // 6 x 6 elimination meets a multiplier above kMaxMultTangent, takes the 9 x 9 system with
-// pivoting.  998,250 QPs in 436 us instead of the 1066 us of the sample-frame kernel with its
-// pivoted 9 x 9 (and 28 instead of 61 us for 10,368, one wave per workgroup spread over the chip).
+// pivoting.  998,250 QPs in 571 us, of them 130 for the moduli, instead of the 1066 us of the
+// sample-frame kernel with its pivoted 9 x 9 and without the moduli (25 instead of 61 us for 10,368).
+// Bound by FP64 issue and latency at one wave per SIMD: G, the columns and the frames are 512
+// registers.  The columns run in a rolled loop with what is indexed by the column in LDS.
 constexpr double kMaxLp = 0.01;
 
 // X <- T X^T T scaled by c
@@ -1208,7 +1210,6 @@ __device__ __forceinline__ bool tangent_point(const CPArgs &a, const CPMaterial 
 }
 // U = R eF, W = R pF(n)^-1 M and R pF(n)^-1 (second indices in the crystal frame)
 __device__ __forceinline__ void tangent_frames(const TangentPoint &q, double *U, double *W, double *RpFi) {
-  double T[9];
   mul_ab(q.R, q.p.eF, U);
   mul_ab(q.pFi, q.R, RpFi);
   mul_ab(RpFi, q.x, W);
@@ -1233,18 +1234,111 @@ __device__ __forceinline__ void tangent_lin(const CPMaterial &cm, double dt, con
   cp_fold(cm, dt, q.x[10], q.g_n, q.p.gsum, q.p.gs, q.p.dgs, c, L);
   mtm3(q.A, q.p.eF, AtE);
 }
+
+// What the element kernel needs of a point, at its deformation gradient Fr (the pass's; the state's
+// own when the pass integrates): T = detJ w pJ Fr Sh, Sh = Me S Me^T, whose rows give the residual, and
+// for a tangent the moduli A[b j][g l] = dT_bj / dF_gl.  With column (g, l)'s dM (crystal frame),
+// U = Fr W and E = sym(U^T (e_g (x) w_l + V dM)) the strain's derivative, V = Fr R pF(n)^-1,
+//   dSh = W (L:E) W^T + X + X^T, X = R pF(n)^-1 dM S W^T,
+//   A[. j][g l] = detJ w pJ (Fr dSh + e_g (x) Sh_l)_.j
+// (dM keeps det M, so -Sh tr(Me^-1 dMe) is zero).  On a lane per point this is 230 multiply-adds a
+// column; in the element kernel, from dMe/dF, it ran on one lane of an element's sixteen and then
+// on nine.
+template <bool HE>
+struct PointFrame {
+  double Fr[9], U[9], W[9], RpFi[9], AtE[9], N[9], Sh[6], wq;
+  HeTan t;
+};
+template <bool HE>
+__device__ __forceinline__ void point_frame(const CPArgs &a, const CPMaterial &cm, int64_t t, const TangentPoint &q,
+                                            bool moduli, PointFrame<HE> &f, double *T) {
+  const int64_t qg = a.qp_base + t;
+  const double *rec = a.qpbuf + qrec(qg);
+  if (a.kin & kKinState) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) f.Fr[i] = a.F_np1[i * a.n_qp + qg];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) f.Fr[i] = rec[i * kRecStride];
+  }
+  f.wq = rec[kRecW * kRecStride] * q.pJ;
+  double S9[9], V[9], Sh9[9];
+  mul_ab(q.pFi, q.R, f.RpFi);
+  mul_ab(f.RpFi, q.x, f.W);
+  mul_ab(f.Fr, f.W, f.U);
+  v6_to_9(q.p.S, S9);
+  mul_abt(S9, f.W, f.N);
+  mul_ab(f.W, f.N, Sh9);
+#pragma unroll
+  for (int I = 0; I < 6; ++I) f.Sh[I] = Sh9[vi(I) * 3 + vj(I)];
+  v6_to_9(f.Sh, Sh9);
+  mul_ab(f.Fr, Sh9, T);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) T[i] *= f.wq;
+  if (moduli) {
+    mul_ab(f.Fr, f.RpFi, V);
+    mul_atb(V, f.U, f.AtE);
+    if constexpr (HE) {
+      double Ce[9], Sx[6];
+      mul_atb(f.U, f.U, Ce);
+      he_law(cm, f.U, Ce, Sx, f.t);
+    }
+  }
+}
+// Column (g, l) of the moduli to the record, from its dM; u = row g of U, w = row l of W.
+template <bool HE>
+__device__ __forceinline__ void store_moduli(const CPMaterial &cm, const PointFrame<HE> &f, const double *u,
+                                             const double *w, const double *dM, int g, int l, double *out) {
+  double E[6], kd[6], dS[6];
+  kappa(u, w, E);
+  k_of(f.AtE, dM, kd);
+#pragma unroll
+  for (int I = 0; I < 6; ++I) E[I] += kd[I];
+  if constexpr (HE) {
+    const double E9[9] = {E[0], 0.5 * E[3], 0.5 * E[5], 0.5 * E[3], E[1], 0.5 * E[4], 0.5 * E[5], 0.5 * E[4], E[2]};
+    he_dot(f.t, E9, dS);
+  } else {
+    const double tr = cm.c12 * (E[0] + E[1] + E[2]);
+#pragma unroll
+    for (int I = 0; I < 6; ++I) dS[I] = I < 3 ? cm.c11m12 * E[I] + tr : 0.5 * cm.c44x2 * E[I];
+  }
+  double dS9[9], X[9], Y[9], Z[9], H[9], Q[9], Sl[3];
+  v6_to_9(dS, dS9);
+  mul_ab(dM, f.N, Y);
+  mul_ab(f.RpFi, Y, X);
+  mul_ab(f.W, dS9, Z);
+  mul_abt(Z, f.W, H);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = i; j < 3; ++j) H[i * 3 + j] = H[j * 3 + i] = H[i * 3 + j] + X[i * 3 + j] + X[j * 3 + i];
+  mul_ab(f.Fr, H, Q);
+  Sl[0] = l == 0 ? f.Sh[0] : (l == 1 ? f.Sh[3] : f.Sh[5]);
+  Sl[1] = l == 0 ? f.Sh[3] : (l == 1 ? f.Sh[1] : f.Sh[4]);
+  Sl[2] = l == 0 ? f.Sh[5] : (l == 1 ? f.Sh[4] : f.Sh[2]);
+  double *o = out + (kRecA + (g * 3 + l) * 9) * kRecStride;
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) o[(b * 3 + j) * kRecStride] = f.wq * (Q[b * 3 + j] + (b == g ? Sl[j] : 0.0));
+}
+
+// What the tangent kernel leaves in a point's record: T; T and the moduli; or, for the
+// three-field element, Me, S, pJ and dMe/dF.
+enum : int { kOutPoint = 0, kOutModuli = 1, kOutMe = 2 };
+
 // The nine columns by the 9 x 9 system with pivoting.  A function of its own, so that the common
 // path keeps nothing in registers for it.
-template <bool HE, int FLOW>
+template <bool HE, int FLOW, int OUT>
 __device__ __attribute__((noinline)) void tangent_pivot(CPArgs a, int64_t t) {
   const CPMaterial cm = a.cpmats[0];
   double *out = a.qpbuf + qrec(a.qp_base + t);
   TangentPoint q;
   tangent_point<HE, FLOW>(a, cm, t, q);
-  double U[9], W[9], RpFi[9], Y[10][9], system[9 * 19];
+  double U[9], W[9], RpFi[9], system[9 * 19];
   tangent_frames(q, U, W, RpFi);
   {
-    double Ah[81], AtE[9];
+    double Ah[81], AtE[9], Y[10][9];
     LocalLin L;
     tangent_lin<HE>(cm, a.dt, q, AtE, L);
     cp_matrix(L, AtE, q.p.T, a.dt * q.x[9] * q.p.pJ, Ah);
@@ -1264,26 +1358,49 @@ __device__ __attribute__((noinline)) void tangent_pivot(CPArgs a, int64_t t) {
     for (int r = 0; r < 9; ++r) Y[9][r] = q.p.T[r];
     store_system<9, 10>(Ah, Y, system);
   }
-  if (!eliminate_pivot<9, 10>(system, Y)) {
+  if (!eliminate_pivot<9, 10>(system)) {
     atomicAdd(a.err, 1);
     return;
   }
+  PointFrame<HE> f;
+  // (T may take the place of Fr in the record: stored last)
+  double T[9];
+  if constexpr (OUT == kOutModuli) point_frame<HE>(a, cm, t, q, true, f, T);
   double dv = 0.0;
 #pragma unroll
-  for (int r = 0; r < 9; ++r) dv += q.p.T[r] * Y[9][r];
-#pragma unroll
+  for (int r = 0; r < 9; ++r) dv += q.p.T[r] * system[r * 19 + 18];
+#pragma unroll 1
   for (int c = 0; c < 9; ++c) {
     double du = 0.0, dM[9];
 #pragma unroll
-    for (int r = 0; r < 9; ++r) du += q.p.T[r] * Y[c][r];
+    for (int r = 0; r < 9; ++r) du += q.p.T[r] * system[r * 19 + 9 + c];
+    du /= dv;
 #pragma unroll
-    for (int r = 0; r < 9; ++r) dM[r] = Y[c][r] - du / dv * Y[9][r];
-    store_dMe(q, RpFi, dM, c, out);
+    for (int r = 0; r < 9; ++r) dM[r] = system[r * 19 + 9 + c] - du * system[r * 19 + 18];
+    if constexpr (OUT == kOutModuli) {
+      const int g = c / 3, l = c % 3;
+      double u[3], w[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        u[i] = g == 0 ? f.U[i] : (g == 1 ? f.U[3 + i] : f.U[6 + i]);
+        w[i] = l == 0 ? f.W[i] : (l == 1 ? f.W[3 + i] : f.W[6 + i]);
+      }
+      store_moduli<HE>(cm, f, u, w, dM, g, l, out);
+    } else {
+      store_dMe(q, RpFi, dM, c, out);
+    }
+  }
+  if constexpr (OUT == kOutModuli) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];
   }
 }
 
-template <bool HE, int FLOW, bool WITH_D>
+template <bool HE, int FLOW, int OUT>
 __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
+  // The columns' kappa -- then their solutions -- and U, W, by a run-time column.  36 KB per wave.
+  __shared__ double sCol[(OUT == kOutPoint ? 1 : 72) * 64];
+  constexpr int kY = 0, kU = 54, kW = 63;
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= nqb) return;
   const int64_t NQ = a.n_qp;
@@ -1293,8 +1410,17 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
   TangentPoint q;
   if (!tangent_point<HE, FLOW>(a, cm, t, q)) {
     atomicAdd(a.err, 1);
+    if constexpr (OUT == kOutMe) {
 #pragma unroll
-    for (int i = 0; i < kCPBuf; ++i) out[i * kRecStride] = 0.0;
+      for (int i = 0; i < 97; ++i) out[i * kRecStride] = 0.0;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) out[i * kRecStride] = 0.0;
+      if constexpr (OUT == kOutModuli) {
+#pragma unroll
+        for (int i = 0; i < 81; ++i) out[(kRecA + i) * kRecStride] = 0.0;
+      }
+    }
     return;
   }
   const CPPoint &p = q.p;
@@ -1305,16 +1431,24 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
       a.tau[al * NQ + qg] = p.tau[al];
       a.gdot[al * NQ + qg] = (fabs(p.sd[al]) * cm.m * q.x[10]) * (p.tau[al] * rg);
     }
-    double S9[9], S[9];
-    v6_to_9(p.S, S9);
-    rot_out(q.R, S9, S);
+    if constexpr (OUT == kOutMe) {
+      double S9[9], S[9];
+      v6_to_9(p.S, S9);
+      rot_out(q.R, S9, S);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) out[i * kRecStride] = q.Me[i];
+      for (int i = 0; i < 9; ++i) out[i * kRecStride] = q.Me[i];
 #pragma unroll
-    for (int I = 0; I < 6; ++I) out[(9 + I) * kRecStride] = S[voigt_i(I) * 3 + voigt_j(I)];
-    out[15 * kRecStride] = q.pJ;
+      for (int I = 0; I < 6; ++I) out[(9 + I) * kRecStride] = S[voigt_i(I) * 3 + voigt_j(I)];
+      out[15 * kRecStride] = q.pJ;
+    }
   }
-  if constexpr (WITH_D) {
+  if constexpr (OUT == kOutPoint) {
+    PointFrame<HE> f;
+    double T[9];
+    point_frame<HE>(a, cm, t, q, false, f, T);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];
+  } else {
     LocalLin L;
     double AtE[9];
     tangent_lin<HE>(cm, a.dt, q, AtE, L);
@@ -1346,48 +1480,83 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
         for (int r = 0; r < 9; ++r) L.G[r][I] = h[r];
       }
     }
-    double U[9], W[9], RpFi[9], S6[36], Y[10][6];
-    tangent_frames(q, U, W, RpFi);
+    double *col = sCol + threadIdx.x;  // field i at col[i * 64]
+    {
+      double U[9], W[9], RpFi[9], S6[36], Y[10][6];
+      tangent_frames(q, U, W, RpFi);
 #pragma unroll
-    for (int I = 0; I < 6; ++I) {
-      double h[9], k6[6];
+      for (int I = 0; I < 6; ++I) {
+        double h[9], k6[6];
 #pragma unroll
-      for (int r = 0; r < 9; ++r) h[r] = L.G[r][I];
-      k_of(AtE, h, k6);
+        for (int r = 0; r < 9; ++r) h[r] = L.G[r][I];
+        k_of(AtE, h, k6);
 #pragma unroll
-      for (int J = 0; J < 6; ++J) S6[J * 6 + I] = k6[J] + (I == J ? 1.0 : 0.0);
+        for (int J = 0; J < 6; ++J) S6[J * 6 + I] = k6[J] + (I == J ? 1.0 : 0.0);
+      }
+#pragma unroll
+      for (int c = 0; c < 9; ++c) kappa(U + (c / 3) * 3, W + (c % 3) * 3, Y[c]);
+      k_of(AtE, v, Y[9]);
+      ok = eliminate<6, 10>(S6, Y, kMaxMultTangent) && ok;
+#pragma unroll
+      for (int c = 0; c < 9; ++c)
+#pragma unroll
+        for (int I = 0; I < 6; ++I) col[(kY + c * 6 + I) * 64] = Y[c][I];
+#pragma unroll
+      for (int r = 0; r < 9; ++r)
+#pragma unroll
+        for (int I = 0; I < 6; ++I) v[r] -= L.G[r][I] * Y[9][I];
     }
-#pragma unroll
-    for (int c = 0; c < 9; ++c) kappa(U + (c / 3) * 3, W + (c % 3) * 3, Y[c]);
-    k_of(AtE, v, Y[9]);
-    ok = eliminate<6, 10>(S6, Y, kMaxMultTangent) && ok;
     if (!ok) {
-      tangent_pivot<HE, FLOW>(a, t);
+      tangent_pivot<HE, FLOW, OUT>(a, t);
       return;
     }
     double dv = 0.0;
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
-#pragma unroll
-      for (int I = 0; I < 6; ++I) v[r] -= L.G[r][I] * Y[9][I];
-      dv += p.T[r] * v[r];
-    }
+    for (int r = 0; r < 9; ++r) dv += p.T[r] * v[r];
     const double rdv = 1.0 / dv;
+    PointFrame<HE> f;
+    double RpFi[9];
+    if constexpr (OUT == kOutModuli) {
+      double T[9];
+      point_frame<HE>(a, cm, t, q, true, f, T);
 #pragma unroll
+      for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) {
+        col[(kU + i) * 64] = f.U[i];
+        col[(kW + i) * 64] = f.W[i];
+      }
+    } else {
+      mul_ab(q.pFi, q.R, RpFi);
+    }
+#pragma unroll 1
     for (int c = 0; c < 9; ++c) {
-      double dM[9], du = 0.0;
+      double dM[9], du = 0.0, y[6];
+#pragma unroll
+      for (int I = 0; I < 6; ++I) y[I] = col[(kY + c * 6 + I) * 64];
 #pragma unroll
       for (int r = 0; r < 9; ++r) {
         double z = 0.0;
 #pragma unroll
-        for (int I = 0; I < 6; ++I) z -= L.G[r][I] * Y[c][I];
+        for (int I = 0; I < 6; ++I) z -= L.G[r][I] * y[I];
         dM[r] = z;
         du += p.T[r] * z;
       }
       du *= rdv;
 #pragma unroll
       for (int r = 0; r < 9; ++r) dM[r] -= du * v[r];
-      store_dMe(q, RpFi, dM, c, out);
+      if constexpr (OUT == kOutModuli) {
+        const int g = c / 3, l = c - 3 * g;
+        double u[3], w[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          u[i] = col[(kU + g * 3 + i) * 64];
+          w[i] = col[(kW + l * 3 + i) * 64];
+        }
+        store_moduli<HE>(cm, f, u, w, dM, g, l, out);
+      } else {
+        store_dMe(q, RpFi, dM, c, out);
+      }
     }
   }
 }
@@ -1401,238 +1570,79 @@ constexpr int cp_stage_round(int epb, int nde, int room) {
   return re;
 }
 
-template <bool HE, int NNE, int MODE, bool STG>
+// Rows of the displacement element from the points' records: with T and the moduli A of
+// store_moduli, f_ab = sum_j T_bj dN_a,j and K_ab,wg = sum_l (sum_j dN_a,j A[b j][g l]) dN_w,l.
+// One lane per row, the points one after another.  Bound by memory: 538 us for 998,250 tet4, 2.3 GB
+// moved at 4.3 TB/s, the rate of a copy.  (1417 us with the point's tensors formed here; 716 with the
+// rows stored by their lanes, 8 bytes every 104, instead of through LDS.)
+template <int NNE, int MODE, bool STG>
 __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, int64_t e_end) {
   constexpr int NQP = nqp_of(NNE);
   constexpr int NDE = NNE * 3;
   constexpr int TPE = (NNE == 4) ? 16 : 32;
-  constexpr int EPB = (NNE == 8) ? 4 : 256 / TPE;
+  constexpr int EPB = 256 / TPE;
+  constexpr int QPB = EPB * NQP;  // points per workgroup: a power of two
   constexpr bool RES = (MODE & MODE_RESIDUAL) != 0;
   constexpr bool TAN = (MODE & MODE_TANGENT) != 0;
   constexpr bool DFL = (MODE & MODE_DEFL_LOAD) != 0;  // K times the prescribed increments
   static_assert(!DFL || (TAN && !RES), "MODE_DEFL_LOAD goes with MODE_TANGENT alone");
+  static_assert(256 % QPB == 0, "a thread's point is its index modulo QPB");
   constexpr bool WK = TAN && !DFL;  // K rows are written
   constexpr bool WR = RES || DFL;   // the residual entry is written
-  // dMe/dF to LDS by all of an element's lanes (tets), or by each QP's lane (hex8, where the
-  // 648 values of eight QPs measured slower spread over 32 lanes)
-  constexpr bool SPREAD_D = NNE != 8;
-  __shared__ double s_x[EPB][NDE], s_u[EPB][NDE];
   __shared__ double s_dl[EPB][DFL ? NDE : 1];
   __shared__ int32_t s_dof[EPB][NDE], s_node[EPB][NNE];
   __shared__ double s_dN[EPB][NQP][NDE];
-  __shared__ double s_Fr[EPB][NQP][9], s_Me[EPB][NQP][9], s_MeS[EPB][NQP][9], s_CrMe[EPB][NQP][9];
-  __shared__ double s_MiT[EPB][NQP][9], s_Sh[EPB][NQP][6], s_S[EPB][NQP][6], s_w[EPB][NQP];
-  __shared__ double s_D[EPB][NQP][TAN ? 81 : 1];
-  __shared__ double s_he[EPB][NQP][(HE && TAN) ? 9 : 1];  // law 1: Ci, c1, c2, c3 at the QP
+  __shared__ double s_T[EPB][NQP][RES ? 9 : 1];
+  __shared__ double s_D[EPB][NQP][TAN ? 81 : 1];  // A[b j][g l], row-major
 
   const int slot = threadIdx.x / TPE, lane = threadIdx.x % TPE;
   const int64_t ie = e_begin + int64_t(blockIdx.x) * EPB + slot;
-  const bool active = (threadIdx.x < EPB * TPE) && ie < e_end;
+  const bool active = ie < e_end;
   const int64_t e = (a.elist && active) ? int64_t(a.elist[ie]) : ie;
   if (active && lane < NNE) {
     const int32_t node = a.conn[e * NNE + lane];
     s_node[slot][lane] = node;
 #pragma unroll
     for (int b = 0; b < 3; ++b) {
-      s_x[slot][lane * 3 + b] = a.X[int64_t(node) * 3 + b];
       const int32_t d = a.dofid[int64_t(node) * 3 + b];
       s_dof[slot][lane * 3 + b] = d;
-      double u = 0.0, dl = 0.0;
-      if (d > 0) {
-        u = a.r[d - 1] + (a.d_r ? a.d_r[d - 1] : 0.0);
-      } else if (d < 0) {
-        dl = a.defl_d ? a.defl_d[-d - 1] : 0.0;
-        u = (a.defl ? a.defl[-d - 1] : 0.0) + (DFL ? 0.0 : dl);  // the prescribed-load pass: K at defl
+      if constexpr (DFL) s_dl[slot][lane * 3 + b] = (d < 0 && a.defl_d) ? a.defl_d[-d - 1] : 0.0;
+    }
+  }
+  {
+    // A thread reads fields of one point, 256 / QPB apart, so that eight consecutive threads read
+    // the eight consecutive doubles a field has in a group of records.
+    const int qi = threadIdx.x % QPB, sl = qi / NQP, ip = qi % NQP;
+    const int64_t iq = e_begin + int64_t(blockIdx.x) * EPB + sl;
+    if (iq < e_end) {
+      const int64_t eq = a.elist ? int64_t(a.elist[iq]) : iq;
+      const double *qb = a.qpbuf + qrec(a.qp_base + eq * NQP + ip);
+      if constexpr (TAN) {
+        for (int f = threadIdx.x / QPB; f < 81; f += 256 / QPB)
+          s_D[sl][ip][(f % 9) * 9 + f / 9] = qb[(kRecA + f) * kRecStride];
       }
-      s_u[slot][lane * 3 + b] = u;
-      if constexpr (DFL) s_dl[slot][lane * 3 + b] = dl;
+      if constexpr (RES) {
+        for (int f = threadIdx.x / QPB; f < 9; f += 256 / QPB) s_T[sl][ip][f] = qb[f * kRecStride];
+      }
+      if (threadIdx.x < QPB) {
+        double k, ee, z, wt, Xi[9];
+        int_point(NNE, ip, k, ee, z, wt);
+        double dN[NDE];
+        shape_dN<NNE>(k, ee, z, dN);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) Xi[i] = qb[(kRecXi + i) * kRecStride];
+#pragma unroll
+        for (int n = 0; n < NNE; ++n)
+#pragma unroll
+          for (int ib = 0; ib < 3; ++ib)
+            s_dN[sl][ip][n * 3 + ib] =
+                dN[n * 3 + 0] * Xi[0 * 3 + ib] + dN[n * 3 + 1] * Xi[1 * 3 + ib] + dN[n * 3 + 2] * Xi[2 * 3 + ib];
+      }
     }
   }
   __syncthreads();
-  if (active && lane < NQP) {
-    const int ip = lane;
-    double k, ee, z, wt;
-    int_point(NNE, ip, k, ee, z, wt);
-    double dN[NDE];
-    shape_dN<NNE>(k, ee, z, dN);
-    double dX[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int n = 0; n < NNE; ++n)
-#pragma unroll
-      for (int ib = 0; ib < 3; ++ib)
-#pragma unroll
-        for (int ic = 0; ic < 3; ++ic) dX[ib * 3 + ic] += dN[n * 3 + ic] * s_x[slot][n * 3 + ib];
-    const double J0 = det3(dX);
-    double Xi[9];
-    const bool ok = J0 > 0.0 && inv3(dX, Xi);
-    if (!ok) atomicAdd(a.err, 1);
-    double Fr[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
-#pragma unroll
-    for (int n = 0; n < NNE; ++n) {
-      double g[3];
-#pragma unroll
-      for (int ib = 0; ib < 3; ++ib)
-        g[ib] = dN[n * 3 + 0] * Xi[0 * 3 + ib] + dN[n * 3 + 1] * Xi[1 * 3 + ib] + dN[n * 3 + 2] * Xi[2 * 3 + ib];
-#pragma unroll
-      for (int ib = 0; ib < 3; ++ib) {
-        s_dN[slot][ip][n * 3 + ib] = g[ib];
-#pragma unroll
-        for (int ic = 0; ic < 3; ++ic) Fr[ib * 3 + ic] += s_u[slot][n * 3 + ib] * g[ic];
-      }
-    }
-    const double *qb = a.qpbuf + qrec(a.qp_base + e * NQP + ip);  // field i at qb[i * kRecStride]
-    double Me[9], S9[9], Mi[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Me[i] = qb[i * kRecStride];
-    double S6[6];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) S6[i] = qb[(9 + i) * kRecStride];
-    v6_to_9(S6, S9);
-    const double pJ = qb[15 * kRecStride];
-    inv3(Me, Mi);
-    double MeS[9], Sh9[9], Cr[9], CrMe[9];
-    mm3(Me, S9, MeS);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        Sh9[i * 3 + j] = MeS[i * 3 + 0] * Me[j * 3 + 0] + MeS[i * 3 + 1] * Me[j * 3 + 1] + MeS[i * 3 + 2] * Me[j * 3 + 2];
-    mtm3(Fr, Fr, Cr);
-    mm3(Cr, Me, CrMe);
-    if constexpr (HE && TAN) {
-      double eF[9], Ce[9], Sx[6];
-      HeTan ht;
-      mm3(Fr, Me, eF);
-      mtm3(eF, eF, Ce);
-      he_law(a.cpmats[0], eF, Ce, Sx, ht);
-#pragma unroll
-      for (int i = 0; i < 6; ++i) s_he[slot][ip][i] = ht.Ci[i];
-      s_he[slot][ip][6] = ht.c1;
-      s_he[slot][ip][7] = ht.c2;
-      s_he[slot][ip][8] = ht.c3;
-    }
-    s_w[slot][ip] = ok ? J0 * wt * pJ : 0.0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-      s_Fr[slot][ip][i] = Fr[i];
-      s_Me[slot][ip][i] = Me[i];
-      s_MeS[slot][ip][i] = MeS[i];
-      s_CrMe[slot][ip][i] = CrMe[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) s_MiT[slot][ip][i * 3 + j] = Mi[j * 3 + i];
-#pragma unroll
-    for (int I = 0; I < 6; ++I) {
-      s_S[slot][ip][I] = S6[I];
-      s_Sh[slot][ip][I] = Sh9[vi(I) * 3 + vj(I)];
-    }
-    if constexpr (TAN && !SPREAD_D) {
-#pragma unroll
-      for (int f = 0; f < 81; ++f) s_D[slot][ip][(f % 9) * 9 + f / 9] = qb[(16 + f) * kRecStride];
-    }
-  }
-  if constexpr (TAN && SPREAD_D) {
-    // the element's dMe/dF (NQP x 81) copied by all of its lanes, consecutive lanes on
-    // consecutive record fields (field 16 + 9 c + r holds D[r][c]), rather than 81 loads on each
-    // QP's lane
-    if (active)
-      for (int j = lane; j < NQP * 81; j += TPE) {
-        const int ip = j / 81, f = j % 81;
-        s_D[slot][ip][(f % 9) * 9 + f / 9] = a.qpbuf[qrec(a.qp_base + e * NQP + ip) + (16 + f) * kRecStride];
-      }
-  }
-  __syncthreads();
-  if constexpr (TAN) {
-    // The row-dependent part of a K row is linear in sAA = sym(Fr^T (e_b (x) g_a)), so in the
-    // row's g_a: per QP, the nine vectors z_bj of z = detJ w (Z : dMe/dF + Fr W) for
-    // sAA = sym(Fr^T (e_b (x) e_j)) (b the row's component, j a component of g_a) replace the
-    // per-row evaluation of B, L:B, Z, Z:dMe/dF and W; a row combines three of them.  They
-    // are computed from dMe/dF and then overwrite it in LDS.
-    constexpr int NT = EPB * TPE, NIT = EPB * NQP * 9, NPASS = (NIT + NT - 1) / NT;
-    double zr[NPASS][9];
-#pragma unroll
-    for (int p = 0; p < NPASS; ++p) {
-      const int t = int(threadIdx.x) + p * NT;
-      const int sl = t / (NQP * 9), ip = (t / 9) % NQP, bj = t % 9, b = bj / 3, j = bj - 3 * b;
-      const int64_t iet = e_begin + int64_t(blockIdx.x) * EPB + sl;
-#pragma unroll
-      for (int c = 0; c < 9; ++c) zr[p][c] = 0.0;
-      if (t < NIT && iet < e_end) {
-        const double *Fr = s_Fr[sl][ip], *Me = s_Me[sl][ip];
-        double sAA[9];  // sym(Fr^T (e_b (x) e_j))_ik = (Fr_bi d_jk + Fr_bk d_ij) / 2
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-            sAA[i * 3 + k] = 0.5 * ((k == j ? Fr[b * 3 + i] : 0.0) + (i == j ? Fr[b * 3 + k] : 0.0));
-        double T[9], Bm[9];
-        mm3(sAA, Me, T);
-        mtm3(Me, T, Bm);  // Me^T sAA Me
-        double Y6[6];
-        if constexpr (HE) {
-          const double *hv = s_he[sl][ip];
-          HeTan ht;
-#pragma unroll
-          for (int i = 0; i < 6; ++i) ht.Ci[i] = hv[i];
-          ht.c1 = hv[6];
-          ht.c2 = hv[7];
-          ht.c3 = hv[8];
-          he_dot(ht, Bm, Y6);
-        } else {
-          const int64_t et = a.elist ? int64_t(a.elist[iet]) : iet;
-          lv_dot(a.grains[a.grain[et]].Lv, Bm, Y6);
-        }
-        double Y9[9];
-        v6_to_9(Y6, Y9);
-        const double *S6 = s_S[sl][ip];
-        const double BS = Bm[0] * S6[0] + Bm[4] * S6[1] + Bm[8] * S6[2] +
-                          2.0 * (0.5 * (Bm[1] + Bm[3]) * S6[3] + 0.5 * (Bm[5] + Bm[7]) * S6[4] +
-                                 0.5 * (Bm[2] + Bm[6]) * S6[5]);
-        // Z = CrMe Y + 2 sAA MeS - (B:S) Me^-T
-        double Z[9], T2[9];
-        mm3(s_CrMe[sl][ip], Y9, Z);
-        mm3(sAA, s_MeS[sl][ip], T2);
-        const double *MiT = s_MiT[sl][ip];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) Z[i] += 2.0 * T2[i] - BS * MiT[i];
-        // W = Me Y Me^T, FrW = Fr W
-        double T3[9], W[9], FrW[9];
-        mm3(Me, Y9, T3);
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-            W[i * 3 + k] = T3[i * 3 + 0] * Me[k * 3 + 0] + T3[i * 3 + 1] * Me[k * 3 + 1] + T3[i * 3 + 2] * Me[k * 3 + 2];
-        mm3(Fr, W, FrW);
-        // z[g L] = sum_ij Z_ij D[ij][g L] + (Fr W)[g L]
-        const double *D = s_D[sl][ip];
-        const double wq = s_w[sl][ip];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) {
-          double sum = 0.0;
-#pragma unroll
-          for (int r = 0; r < 9; ++r) sum += Z[r] * D[r * 9 + c];
-          zr[p][c] = wq * (sum + FrW[c]);
-        }
-      }
-    }
-    lds_barrier();  // every z_bj is computed from dMe/dF before any overwrites it
-#pragma unroll
-    for (int p = 0; p < NPASS; ++p) {
-      const int t = int(threadIdx.x) + p * NT;
-      if (t < NIT) {
-        const int sl = t / (NQP * 9), ip = (t / 9) % NQP, bj = t % 9;
-#pragma unroll
-        for (int c = 0; c < 9; ++c) s_D[sl][ip][bj * 9 + c] = zr[p][c];
-      }
-    }
-    lds_barrier();
-  }
   const bool rowlane = active && lane < NDE;
   const int ra = lane / 3, rb = lane % 3;
-  const double eb[3] = {rb == 0 ? 1.0 : 0.0, rb == 1 ? 1.0 : 0.0, rb == 2 ? 1.0 : 0.0};
   double K[TAN ? NDE : 1];
   if constexpr (TAN) {
 #pragma unroll
@@ -1642,29 +1652,17 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
   if (rowlane) {
 #pragma unroll 1
   for (int ip = 0; ip < NQP; ++ip) {
-    const double wq = s_w[slot][ip];
     const double *dN = s_dN[slot][ip];
-    const double *Fr = s_Fr[slot][ip];
     const double ga[3] = {dN[ra * 3], dN[ra * 3 + 1], dN[ra * 3 + 2]};
-    double Sh9[9];
-    v6_to_9(s_Sh[slot][ip], Sh9);
-    double ta[3];  // Sh dN_a
-#pragma unroll
-    for (int i = 0; i < 3; ++i) ta[i] = Sh9[i * 3] * ga[0] + Sh9[i * 3 + 1] * ga[1] + Sh9[i * 3 + 2] * ga[2];
-    if constexpr (RES) fe += wq * (Fr[rb * 3] * ta[0] + Fr[rb * 3 + 1] * ta[1] + Fr[rb * 3 + 2] * ta[2]);
+    if constexpr (RES) {
+      const double *T = &s_T[slot][ip][rb * 3];
+      fe += T[0] * ga[0] + T[1] * ga[1] + T[2] * ga[2];
+    }
     if constexpr (TAN) {
-      // z = sum_j g_a,j z_bj, plus the geometric term of row b: detJ w (Sh g_a)
-      const double *zb = &s_D[slot][ip][rb * 27];
+      const double *A = &s_D[slot][ip][rb * 27];
       double zz[9];
 #pragma unroll
-      for (int c = 0; c < 9; ++c) zz[c] = ga[0] * zb[c] + ga[1] * zb[9 + c] + ga[2] * zb[18 + c];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double wt = wq * ta[k];
-        zz[0 + k] += eb[0] * wt;
-        zz[3 + k] += eb[1] * wt;
-        zz[6 + k] += eb[2] * wt;
-      }
+      for (int c = 0; c < 9; ++c) zz[c] = ga[0] * A[c] + ga[1] * A[9 + c] + ga[2] * A[18 + c];
 #pragma unroll
       for (int w = 0; w < NNE; ++w) {
         const double h0 = dN[w * 3], h1 = dN[w * 3 + 1], h2 = dN[w * 3 + 2];
@@ -1687,11 +1685,10 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
   }
   }  // rowlane
   constexpr int LD = NDE + 1;
-  if constexpr (WK && STG && NNE != 4) {
-    // Gather mode: RE elements at a time, the rows go to LDS (in the dead dM/dF array) laid
-    // out as the staging blocks, then the workgroup copies each node block, zero-padded to
-    // whole lines, to its staging offset with consecutive threads on consecutive doubles.
-    // (Linear tets store their 13-double rows directly: the transpose rounds cost more.)
+  if constexpr (WK && STG) {
+    // Gather mode: RE elements at a time, the rows go to LDS (in the dead moduli) laid out as the
+    // staging blocks, then the workgroup copies each node block, zero-padded to whole lines, to
+    // its staging offset with consecutive threads on consecutive doubles.
     constexpr int PB = stage_block(NNE);
     constexpr int RE = cp_stage_round(EPB, NDE, EPB * NQP * 81);
     static_assert(RE * NDE * LD <= EPB * NQP * 81, "staging round does not fit");
@@ -2220,17 +2217,12 @@ void launch_kin(const CPArgs &a, hipStream_t s) {
 template <int NNE, int MODE>
 void launch_ce(const CPElemArgs &a, int64_t e0, int64_t e1, hipStream_t s) {
   constexpr int TPE = (NNE == 4) ? 16 : 32;
-  constexpr int EPB = (NNE == 8) ? 4 : 256 / TPE;
+  constexpr int EPB = 256 / TPE;
   const int64_t n = e1 - e0;
   if (n <= 0) return;
   const unsigned grid = unsigned((n + EPB - 1) / EPB);
-  if (a.law == 1) {
-    if (a.stage) cp_elem<true, NNE, MODE, true><<<grid, EPB * TPE, 0, s>>>(a, e0, e1);
-    else cp_elem<true, NNE, MODE, false><<<grid, EPB * TPE, 0, s>>>(a, e0, e1);
-  } else {
-    if (a.stage) cp_elem<false, NNE, MODE, true><<<grid, EPB * TPE, 0, s>>>(a, e0, e1);
-    else cp_elem<false, NNE, MODE, false><<<grid, EPB * TPE, 0, s>>>(a, e0, e1);
-  }
+  if (a.stage) cp_elem<NNE, MODE, true><<<grid, 256, 0, s>>>(a, e0, e1);
+  else cp_elem<NNE, MODE, false><<<grid, 256, 0, s>>>(a, e0, e1);
 }
 
 template <int NNE>
@@ -2531,8 +2523,9 @@ void launch_cp_tangent(const CPArgs &a, bool with_D, hipStream_t s) {
   by_law(a, [&](auto he, auto fl) {
     constexpr bool HE = decltype(he)::value;
     constexpr int FLOW = decltype(fl)::value;
-    if (with_D) cp_tangent<HE, FLOW, true><<<grid, 64, 0, s>>>(a, nq);
-    else cp_tangent<HE, FLOW, false><<<grid, 64, 0, s>>>(a, nq);
+    if (a.tf) cp_tangent<HE, FLOW, kOutMe><<<grid, 64, 0, s>>>(a, nq);
+    else if (with_D) cp_tangent<HE, FLOW, kOutModuli><<<grid, 64, 0, s>>>(a, nq);
+    else cp_tangent<HE, FLOW, kOutPoint><<<grid, 64, 0, s>>>(a, nq);
   });
 }
 

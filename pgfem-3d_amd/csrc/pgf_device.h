@@ -101,16 +101,14 @@ struct TfArgs {
 enum : int { MODE_INTEGRATE = 1, MODE_RESIDUAL = 2, MODE_TANGENT = 4, MODE_DEFL_LOAD = 8 };
 
 // ---------------------------------------------------------------- crystal plasticity
-// Per-grain tables: Schmid tensors P_a = s_a (x) m_a rotated to the sample frame (12 x 9,
-// row-major) and the rotated cubic stiffness in Voigt form Lv[I][J] (I, J in xx,yy,zz,xy,yz,
-// xz) such that S_I = sum_J Lv[I][J] E_J with E_J the tensor components of a symmetric E.
+// Per-grain tables: the rotation, and the Schmid tensors P_a = s_a (x) m_a in the sample frame
+// (12 x 9, row-major) for the slip increments that the learned start is trained on.
 struct DevGrain {
   double P[12][9];
-  double Lv[36];
   double R[9];  // crystal -> sample rotation
 };
 
-// law 0: cubic St Venant-Kirchhoff through the grain's Lv; law 1: neo-Hookean deviatoric part
+// law 0: cubic St Venant-Kirchhoff in the grain's frame; law 1: neo-Hookean deviatoric part
 // (m10) and the volumetric potential vol_flag (kappa) on the elastic part eF.
 struct CPMaterial {
   double gd0, m, h0, g0, gs0, gds, w, tol;
@@ -144,9 +142,9 @@ struct CPArgs {
   const double *tau_n;        // 12 comps at n (learned-start features)
   int32_t *iters;             // [n_qp]
   const double *warm;         // optional start (M 9, lambda, g) [11][n_qp]
-  // per-QP records (qrec): the plain start, then the tangent pass's output for the element
-  // kernel, Me 9, S 6, pJ 1, D = dMe/dF 81 by columns (field 16 + 9 c + r holds D[r][c]);
-  // indexed by device QP
+  // per-QP records (qrec), indexed by device QP: the kinematics' output and the plain start, then
+  // the tangent pass's output for the element kernel (kRec* below; for the three-field element
+  // Me 9, S 6, pJ 1, D = dMe/dF 81 by columns, field 16 + 9 c + r holding D[r][c])
   double *qpbuf;
   int32_t *err;
   unsigned long long *qnext;  // global work queue of the local Newton (cp_chunk = 1), else null
@@ -155,8 +153,18 @@ struct CPArgs {
   // three-field (CM3F) blocks: per block element theta = tf_V + tf_dV; the kinematics then
   // stores the model's F(n+1) = (theta/J)^(1/3) F.  Null otherwise.
   const double *tf_V, *tf_dV;
+  int32_t tf;                 // the handle's elements are three-field
+  int32_t kin;                // what the pass's kinematics does (kKin*)
 };
-constexpr int kCPBuf = 97;  // doubles per QP in qpbuf
+// The kinematics stores F(n+1) (an integrating pass), stores the record's geometry (a
+// displacement element follows), and leaves defl_d out of the displacements (the prescribed-load
+// pass).
+enum : int { kKinState = 1, kKinRec = 2, kKinDefl = 4 };
+// A displacement element's record: fields 0..8 the pass's F where it is not the state's, or the plain
+// start x(0..10) and its flag, then T; kRecXi the inverse of dX/dxi; kRecA the moduli, column
+// (g, l) at kRecA + 9 (3 g + l); kRecW, until the last of them is stored, detJ w.
+constexpr int kRecXi = 12, kRecA = 21, kRecW = kRecA + 80;
+constexpr int kCPBuf = 102;  // doubles per QP in qpbuf
 // qpbuf holds the records of 8 QPs at a time with the field outermost: field f of device QP q
 // is at qpbuf[qrec(q) + f * kRecStride].  A wave's store of one field over its 64 QPs then
 // writes eight 64-byte runs, and the next field's store the other halves of the same 128-byte
@@ -195,12 +203,10 @@ void launch_cp_tangent(const CPArgs &a, bool with_D, hipStream_t s);
 // Element kernel of the crystal-plasticity blocks: residual and / or tangent from qpbuf.
 struct CPElemArgs {
   const double *X;
-  const int32_t *dofid, *row_start, *rowlen, *conn, *grain;
+  const int32_t *dofid, *row_start, *rowlen, *conn;
   const int16_t *off;
   const int32_t *elist;  // coloured mode: as ElemArgs
-  const DevGrain *grains;
   const CPMaterial *cpmats;
-  int32_t law;  // cpmats[0].law
   const double *qpbuf;
   int64_t qp_base;
   const double *r, *d_r, *defl, *defl_d;

@@ -69,3 +69,27 @@ def test_pivoted_tangent_at_large_steps(device, law, m, stretch, some):
     lp = np.abs(st.lam_np1 * np.linalg.det(st.pF_np1.T.reshape(-1, 3, 3)))
     assert (lp > 0.01).any() and (lp < 0.01).any() == some
     h.close()
+
+
+@pytest.mark.parametrize("etype,n", [(P.PGF_TET4, 2), (P.PGF_TET10, 2), (P.PGF_HEX8, 2)])
+def test_three_field_initial_gradients(device, etype, n):
+    """pgf_tf_initial stores F at n and n-1 of the given displacements: an integrating pass's F at
+    them."""
+    prob, h, _ = _setup(n, etype, "hyperelastic")
+    h3 = P.Handle(prob.mesh, prob.ids, prob.ndof, prob.Ap, prob.Ai, prob.mats)
+    h3.set_orientations(prob.R, prob.grain)
+    h3.set_three_field(True)
+    f = torch.empty(prob.ndof, dtype=torch.float64, device=device)
+    args, F = [], []
+    for s in (2e-3, 1e-3):
+        r, defl = prob.displacement(s, 2e-4, seed=3)
+        rd, dd = (torch.from_numpy(np.ascontiguousarray(x)).to(device) for x in (r, defl))
+        h.residual(f, rd, defl=dd, dt=1.0)
+        F.append(h.get_state(P.STATE_F_NP1).copy())
+        args += [rd, dd]
+    h3.tf_initial(*args)
+    for fld, ref in ((P.STATE_F_N, F[0]), (P.STATE_F_NM1, F[1])):
+        assert np.abs(ref - np.eye(3).reshape(9, 1)).max() > 1e-4
+        assert np.abs(h3.get_state(fld) - ref).max() < 1e-15
+    h3.close()
+    h.close()
