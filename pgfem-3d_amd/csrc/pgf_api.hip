@@ -35,6 +35,7 @@ struct Block {
   int32_t *d_edof = nullptr;  // [ne*3nne] DOF ids of the element DOFs
   int16_t *d_off = nullptr;
   int64_t *d_soff = nullptr;       // gather mode: [ne*nne] staging offsets
+  int32_t *d_rslot = nullptr;      // and block numbers
   int32_t *d_mat = nullptr;
   int32_t *d_egrain = nullptr;  // crystal plasticity: grain per element / per QP (device order)
   int32_t *d_qgrain = nullptr;
@@ -51,6 +52,7 @@ struct CohBlock {
   int32_t *d_conn = nullptr, *d_mat = nullptr;
   int16_t *d_off = nullptr;
   int64_t *d_soff = nullptr;
+  int32_t *d_rslot = nullptr;
 };
 
 template <class T>
@@ -405,13 +407,15 @@ pgf::ElemArgs base_args(pgf_handle h, const pgf_nodal_input *in) {
 // local node), which fixes the order of every sum.  Blocks start on 128-byte lines and are
 // padded to whole lines, so the element kernels' block stores never share a line with a
 // block written at another time (a partly written line costs a read-modify-write).  off holds the groups' first-touch-marked
-// node-pair offsets; soff receives each group's [n*nne] staging offsets (-1: no block).
+// node-pair offsets; soff receives each group's [n*nne] staging offsets (-1: no block), rslot the
+// blocks' numbers in that order.
 struct GatherGroup {
   int nne;
   int64_t ne;
   const int32_t *conn;  // [ne*nne] device order
   const int16_t *off;   // [ne*nne*nne]
   std::vector<int64_t> soff;
+  std::vector<int32_t> rslot;
 };
 
 void build_gather(int64_t n_nodes, const int32_t *dofid, std::vector<GatherGroup> &groups,
@@ -434,6 +438,7 @@ void build_gather(int64_t n_nodes, const int32_t *dofid, std::vector<GatherGroup
   for (size_t gi = 0; gi < groups.size(); ++gi) {
     GatherGroup &g = groups[gi];
     g.soff.assign(g.ne * g.nne, -1);
+    g.rslot.assign(g.ne * g.nne, -1);
     for (int64_t i = 0; i < g.ne * g.nne; ++i) {
       const int32_t node = g.conn[i];
       if (!fmask(node)) continue;
@@ -459,6 +464,7 @@ void build_gather(int64_t n_nodes, const int32_t *dofid, std::vector<GatherGroup
     GatherGroup &g = groups[s_group[sl]];
     const int64_t i = s_pair[sl], k = i / g.nne;
     g.soff[i] = inc_soff[sl];
+    g.rslot[i] = int32_t(sl);
     const int16_t *orow = g.off + i * g.nne;
     for (int w = 0; w < g.nne; ++w) {
       const int o = orow[w];
@@ -515,6 +521,7 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
         ce.f = f;
         ce.vals = vals;
         ce.soff = b.d_soff;
+        ce.rslot = b.d_rslot;
         ce.stage = gather ? stage : nullptr;
         ce.elist = gather ? nullptr : b.d_clist;
         ce.err = h->d_err;
@@ -534,6 +541,7 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
         a.edof = b.d_edof;
         a.off = b.d_off;
         a.soff = b.d_soff;
+        a.rslot = b.d_rslot;
         a.elist = gather ? nullptr : b.d_clist;
         a.mat = b.d_mat;
         a.qp_base = b.qp_base;
@@ -579,6 +587,7 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
         ca.mat = cb.d_mat;
         ca.off = cb.d_off;
         ca.soff = cb.d_soff;
+        ca.rslot = cb.d_rslot;
         ca.elist = gather ? nullptr : cb.d_clist;
         ca.cqp_base = cb.cqp_base;
         pgf::launch_coh_elem(cb.nn, mode, ca, e0, e1, h->stream);
@@ -964,9 +973,9 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
   }
   std::vector<GatherGroup> groups;
   for (size_t bi = 0; bi < h->blocks.size(); ++bi)
-    groups.push_back({h->blocks[bi].nne, h->blocks[bi].ne, bconn[bi].data(), boff[bi].data(), {}});
+    groups.push_back({h->blocks[bi].nne, h->blocks[bi].ne, bconn[bi].data(), boff[bi].data(), {}, {}});
   for (size_t bi = 0; bi < h->cblocks.size(); ++bi)
-    groups.push_back({2 * h->cblocks[bi].nn, h->cblocks[bi].nc, cconn[bi].data(), cboff[bi].data(), {}});
+    groups.push_back({2 * h->cblocks[bi].nn, h->cblocks[bi].nc, cconn[bi].data(), cboff[bi].data(), {}, {}});
   std::vector<int64_t> inc_ptr, inc_soff, inc_poff;
   std::vector<int32_t> inc_nne;
   std::vector<uint32_t> gpos;
@@ -988,10 +997,12 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     pgf::CohBlock &cb = h->cblocks[bi];
     const std::vector<int32_t> zero(cb.nc, 0);
     const std::vector<int64_t> &soff = groups[h->blocks.size() + bi].soff;
+    const std::vector<int32_t> &rslot = groups[h->blocks.size() + bi].rslot;
     if ((rc = pgf::upload(&cb.d_conn, cconn[bi].data(), cconn[bi].size()))) return fail(rc);
     if ((rc = pgf::upload(&cb.d_mat, zero.data(), zero.size()))) return fail(rc);
     if ((rc = pgf::upload(&cb.d_off, cboff[bi].data(), cboff[bi].size()))) return fail(rc);
     if ((rc = pgf::upload(&cb.d_soff, soff.data(), soff.size()))) return fail(rc);
+    if ((rc = pgf::upload(&cb.d_rslot, rslot.data(), rslot.size()))) return fail(rc);
     if ((rc = pgf::upload(&cb.d_clist, cb.clist.data(), cb.clist.size()))) return fail(rc);
   }
   if (h->n_cqp) {
@@ -1065,6 +1076,7 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     if ((rc = pgf::upload(&b.d_mat, mat.data(), mat.size()))) return fail(rc);
     if ((rc = pgf::upload(&b.d_off, boff[bi].data(), boff[bi].size()))) return fail(rc);
     if ((rc = pgf::upload(&b.d_soff, groups[bi].soff.data(), groups[bi].soff.size()))) return fail(rc);
+    if ((rc = pgf::upload(&b.d_rslot, groups[bi].rslot.data(), groups[bi].rslot.size()))) return fail(rc);
     if ((rc = pgf::upload(&b.d_clist, b.clist.data(), b.clist.size()))) return fail(rc);
   }
   for (int t = 0; t < 3; ++t) {
@@ -1145,6 +1157,7 @@ int pgf_destroy(pgf_handle h) {
     hipFree(b.d_edof);
     hipFree(b.d_off);
     hipFree(b.d_soff);
+    hipFree(b.d_rslot);
     hipFree(b.d_clist);
     hipFree(b.d_mat);
     hipFree(b.d_egrain);
@@ -1154,6 +1167,7 @@ int pgf_destroy(pgf_handle h) {
     hipFree(cb.d_mat);
     hipFree(cb.d_off);
     hipFree(cb.d_soff);
+    hipFree(cb.d_rslot);
     hipFree(cb.d_clist);
   }
   hipFree(h->d_inc_ptr);

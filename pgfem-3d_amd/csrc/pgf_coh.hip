@@ -301,8 +301,9 @@ __global__ __launch_bounds__(256) void coh_elem(CohArgs a, int64_t e_begin, int6
       fr += s_live[slot][q] ? qd[0] * qd[1 + NN + M] * qd[1 + P] : 0.0;
     }
     fr *= sr;
-    if (a.stage) {
-      a.stage[a.soff[e * NT + ra] + M * (ND + 1) + ND] = fr;
+    if (a.stage) {  // gather mode: into the row, or the entry alone
+      if constexpr (TAN) a.stage[a.soff[e * NT + ra] + M * (ND + 1) + ND] = fr;
+      else a.stage[int64_t(a.rslot[e * NT + ra]) * 3 + M] = fr;
     } else {
       const bool first = off[ra] <= -2;
       if (first) a.f[dof - 1] = fr;
@@ -330,7 +331,7 @@ __global__ __launch_bounds__(256) void coh_elem(CohArgs a, int64_t e_begin, int6
 #pragma unroll
       for (int c = 0; c < ND; ++c) fl += K[c] * s_dl[slot][c];
       if (a.stage) {
-        a.stage[a.soff[e * NT + ra] + M * (ND + 1) + ND] = fl;
+        a.stage[int64_t(a.rslot[e * NT + ra]) * 3 + M] = fl;
       } else {
         const bool first = off[ra] <= -2;
         if (first) a.f[dof - 1] = fl;

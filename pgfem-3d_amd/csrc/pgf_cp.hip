@@ -1725,13 +1725,8 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
   if (!rowlane) return;
   const int32_t dof = s_dof[slot][lane];
   if (dof <= 0) return;
-  if constexpr (STG) {  // gather mode: the row straight into its staging block
-    double *srow = a.stage + a.soff[e * NNE + ra] + rb * LD;
-    if constexpr (WK) {
-#pragma unroll
-      for (int i = 0; i < NDE; ++i) srow[i] = K[i];
-    }
-    if constexpr (WR) srow[NDE] = fe;
+  if constexpr (STG) {  // gather mode, no K rows: the entry alone
+    a.stage[int64_t(a.rslot[e * NNE + ra]) * 3 + rb] = fe;
     return;
   }
   const int16_t *off = a.off + (e * NNE + ra) * NNE;
@@ -2147,13 +2142,15 @@ __global__ __launch_bounds__(256) void cp_tf_elem(CPElemArgs a, int64_t e_begin,
   const int32_t dof = s_dof[slot][lane];
   if (dof <= 0) return;
   constexpr int LD = NDE + 1;
-  if constexpr (STG) {  // gather mode: the row straight into its staging block
-    double *srow = a.stage + a.soff[e * NNE + ra] + rb * LD;
+  if constexpr (STG) {  // gather mode: the row straight into its staging block, or the entry alone
     if constexpr (WK) {
+      double *srow = a.stage + a.soff[e * NNE + ra] + rb * LD;
 #pragma unroll
       for (int i = 0; i < NDE; ++i) srow[i] = K[i];
+      if constexpr (WR) srow[NDE] = fe;
+    } else {
+      a.stage[int64_t(a.rslot[e * NNE + ra]) * 3 + rb] = fe;
     }
-    if constexpr (WR) srow[NDE] = fe;
     return;
   }
   const int16_t *off = a.off + (e * NNE + ra) * NNE;

@@ -62,10 +62,12 @@ struct ElemArgs {
   double *Sc_np1;           // scalars n+1
   double dt;                // time step (J2 damage viscosity)
   // outputs: coloured mode adds into f / vals through off; gather mode (stage != null)
-  // writes row (a, b) of element e to stage[soff[e*nne + a] + b*(3nne+1) ...], residual last
+  // writes row (a, b) of element e to stage[soff[e*nne + a] + b*(3nne+1) ...], residual last; a
+  // pass without K rows its residual alone, to stage[3 rslot[e*nne + a] + b]
   double *f;                // [ndof]
   double *vals;             // [nnz]
   const int64_t *soff;      // [ne*nne] staging offsets of the element's node blocks
+  const int32_t *rslot;     // [ne*nne] their numbers
   double *stage;
   int32_t *err;             // failure counter
   // three-field (CM3F) blocks, per block element (block-local index): theta = V(n+1) + dV and
@@ -212,6 +214,7 @@ struct CPElemArgs {
   const double *r, *d_r, *defl, *defl_d;
   double *f, *vals;
   const int64_t *soff;  // gather mode: as ElemArgs
+  const int32_t *rslot;
   double *stage;
   int32_t *err;
   // three-field (CM3F) blocks: as ElemArgs (block-local per element)
@@ -252,6 +255,7 @@ struct CohArgs {
   double *vars_np1;        // [2][n_cqp] at n+1 (written by integrating passes)
   double *f, *vals;
   const int64_t *soff;     // gather mode: as ElemArgs (node blocks of 2nn nodes)
+  const int32_t *rslot;
   double *stage;
   int32_t *err;
 };

@@ -800,8 +800,8 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
   if (!rowlane) return;
   const int32_t dof = s_dof[slot][lane];
   if (dof <= 0) return;
-  if constexpr (STG) {  // gather mode, residual only: the row's entry into its staging block
-    a.stage[a.soff[e * NNE + ra] + rb * LD + NDE] = fe;
+  if constexpr (STG) {  // gather mode, no K rows: the entry alone
+    a.stage[int64_t(a.rslot[e * NNE + ra]) * 3 + rb] = fe;
     return;
   }
   const int16_t *off = a.off + (e * NNE + ra) * NNE;
@@ -859,7 +859,7 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
 // and within one block every target is distinct: the sums run in the same order on every
 // call.  Elements have at most 10 nodes (3nne + 1 <= 32 lanes).  NB and the nodes per
 // workgroup are launch choices (autotuned, pgf_autotune).
-template <bool RES, bool TAN, int NB>
+template <bool RES, int NB>
 __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
   extern __shared__ double s_acc[];
   const int wpb = blockDim.x / 64;
@@ -875,8 +875,7 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
   const int len = g.rowlen[node];
   double *acc = s_acc + int64_t(wid) * (3 * g.maxlen + 3);
   double *facc = acc + 3 * g.maxlen;  // residual entries of the node's rows
-  if constexpr (TAN)
-    for (int i = lane; i < nr * len; i += 64) acc[i] = 0.0;
+  for (int i = lane; i < nr * len; i += 64) acc[i] = 0.0;
   if (lane < 3) facc[lane] = 0.0;
   __builtin_amdgcn_wave_barrier();
   int rowoff[3];  // offset of row b in the node's values (b free)
@@ -895,7 +894,7 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
       const uint64_t rec = g.inc_rec[k];
       const int nde = 3 * int(rec >> 60);
       const double *blk = g.stage + int64_t(rec & 0xffffffffu) * 16 + c;
-      if (TAN && c < nde) {
+      if (c < nde) {
         const int w = c / 3, gg = c - 3 * w;
         const uint32_t p = g.pos[int64_t((rec >> 32) & 0x0fffffffu) + w];
         const int mw = int(p >> 28);
@@ -926,11 +925,35 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
         __builtin_amdgcn_wave_barrier();
       }
   }
-  if constexpr (TAN) {
-    double *out = g.vals + g.row_start[node];
-    for (int i = lane; i < nr * len; i += 64) __builtin_nontemporal_store(acc[i], out + i);
-  }
+  double *out = g.vals + g.row_start[node];
+  for (int i = lane; i < nr * len; i += 64) __builtin_nontemporal_store(acc[i], out + i);
   if (RES && lane < 3 && ((fm >> lane) & 1)) g.f[g.dofid[node * 3 + lane] - 1] = facc[lane];
+}
+
+// A pass without K rows stages three entries per block, block k's at stage[3 k], so a node's are
+// contiguous: one thread per DOF adds its blocks in the order of gather_kernel.  The element
+// kernels write 24 bytes per (element, node) instead of 8 in each of three lines, and the sums read
+// as much: 43 -> 6 us on 33^3 hex8 (their element kernel 47 -> 41), 443 -> 22 us on 998,250 tet4
+// with crystal plasticity (537 -> 151).
+__global__ __launch_bounds__(256) void gather_residual_kernel(GatherArgs g) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= 3 * g.n_nodes) return;
+  const int32_t d = g.dofid[i];
+  if (d <= 0) return;
+  const int64_t node = i / 3;
+  const int b = int(i - 3 * node);
+  const int64_t ke = g.inc_ptr[node + 1];
+  double s = 0.0;
+  int64_t k = g.inc_ptr[node];
+  for (; k + 4 <= ke; k += 4) {  // four loads in flight
+    double v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = g.stage[(k + j) * 3 + b];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += v[j];
+  }
+  for (; k < ke; ++k) s += g.stage[k * 3 + b];
+  g.f[d - 1] = s;
 }
 
 __global__ void fill_kernel(double *p, int64_t n, double v) {
@@ -1135,24 +1158,26 @@ int gather_waves(int32_t maxlen) {
 }
 
 template <int NB>
-void launch_gather_nb(bool res, bool tan, const GatherArgs &g, unsigned grid, int threads, size_t lds,
-                      hipStream_t s) {
-  if (res && tan) gather_kernel<true, true, NB><<<grid, threads, lds, s>>>(g);
-  else if (res) gather_kernel<true, false, NB><<<grid, threads, lds, s>>>(g);
-  else if (tan) gather_kernel<false, true, NB><<<grid, threads, lds, s>>>(g);
+void launch_gather_nb(bool res, const GatherArgs &g, unsigned grid, int threads, size_t lds, hipStream_t s) {
+  if (res) gather_kernel<true, NB><<<grid, threads, lds, s>>>(g);
+  else gather_kernel<false, NB><<<grid, threads, lds, s>>>(g);
 }
 
 void launch_gather(int mode, const GatherArgs &g, int waves, int batch, hipStream_t s) {
   const int wpb = std::min(gather_waves(g.maxlen), std::max(waves, 1));
   if (g.n_nodes <= 0 || wpb < 1) return;
-  const unsigned grid = unsigned((g.n_nodes + wpb - 1) / wpb);
-  const size_t lds = size_t(wpb) * (3 * size_t(std::max<int32_t>(g.maxlen, 1)) + 3) * sizeof(double);
   // the prescribed-load pass stages its vector in the residual entries and no K rows
   const bool dfl = (mode & MODE_DEFL_LOAD) != 0;
   const bool res = (mode & MODE_RESIDUAL) != 0 || dfl, tan = (mode & MODE_TANGENT) != 0 && !dfl;
-  if (batch <= 2) launch_gather_nb<2>(res, tan, g, grid, 64 * wpb, lds, s);
-  else if (batch <= 4) launch_gather_nb<4>(res, tan, g, grid, 64 * wpb, lds, s);
-  else launch_gather_nb<8>(res, tan, g, grid, 64 * wpb, lds, s);
+  if (!tan) {
+    if (res) gather_residual_kernel<<<unsigned((3 * g.n_nodes + 255) / 256), 256, 0, s>>>(g);
+    return;
+  }
+  const unsigned grid = unsigned((g.n_nodes + wpb - 1) / wpb);
+  const size_t lds = size_t(wpb) * (3 * size_t(std::max<int32_t>(g.maxlen, 1)) + 3) * sizeof(double);
+  if (batch <= 2) launch_gather_nb<2>(res, g, grid, 64 * wpb, lds, s);
+  else if (batch <= 4) launch_gather_nb<4>(res, g, grid, 64 * wpb, lds, s);
+  else launch_gather_nb<8>(res, g, grid, 64 * wpb, lds, s);
 }
 
 void launch_tf_update(int nne, const TfArgs &t, hipStream_t s) {
