@@ -859,6 +859,14 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
 // and within one block every target is distinct: the sums run in the same order on every
 // call.  Elements have at most 10 nodes (3nne + 1 <= 32 lanes).  NB and the nodes per
 // workgroup are launch choices (autotuned, pgf_autotune).
+//
+// Bound by the latency of its loads on small meshes and by memory on large ones, so a node's
+// records are read at once, one per lane, and a block's values and places together: two loads
+// deep per batch (values waiting for places, and those for records, were four).  58 us -> 46 on
+// 33^3 hex8, 540 -> 373 on 998,250 tet4 (5.2 TB/s), 1461 -> 1280 on 663,552 tet10, 21 -> 13.6 on
+// 6,000 tet4.  With the next batch's loads issued before the adds, 104 registers instead of 56, it was
+// slower (516 and 1710 us); NB of 2 and 8 are within 8%.
+constexpr uint32_t kResidual = 0xffffffffu;  // in place of a column's position, whose bit 31 is never set
 template <bool RES, int NB>
 __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
   extern __shared__ double s_acc[];
@@ -883,47 +891,58 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherArgs g) {
   for (int b = 0; b < 3; ++b) rowoff[b] = __popc(fm & ((1 << b) - 1)) * len;
   const int half = lane >> 5, c = lane & 31;
   const int64_t kb = g.inc_ptr[node], ke = g.inc_ptr[node + 1];
-  for (int64_t k0 = kb; k0 < ke; k0 += 2 * NB) {
-    double v[NB][3];
-    int dst[NB];  // column in the rows, -2 = residual entries, -1 = nothing
+  const int cw = c / 3, cg = c - 3 * cw;
+  for (int64_t w0 = kb; w0 < ke; w0 += 64) {
+    // the window's records, one per lane
+    const int nw = int(ke - w0 < 64 ? ke - w0 : 64);
+    const uint64_t mine = lane < nw ? g.inc_rec[w0 + lane] : 0;
+    const int lo = int(uint32_t(mine)), hi = int(uint32_t(mine >> 32));
+    // A block's values are read whether or not its column has a place, so that they are in
+    // flight together with the places.
+    auto load = [&](int k0, double (&v)[NB][3], uint32_t (&at)[NB]) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      dst[j] = -1;
-      const int64_t k = k0 + 2 * j + half;
-      if (k >= ke) continue;
-      const uint64_t rec = g.inc_rec[k];
-      const int nde = 3 * int(rec >> 60);
-      const double *blk = g.stage + int64_t(rec & 0xffffffffu) * 16 + c;
-      if (c < nde) {
-        const int w = c / 3, gg = c - 3 * w;
-        const uint32_t p = g.pos[int64_t((rec >> 32) & 0x0fffffffu) + w];
-        const int mw = int(p >> 28);
-        if ((mw >> gg) & 1) dst[j] = int(p & 0x0fffffffu) + __popc(mw & ((1 << gg) - 1));
-      } else if (RES && c == nde) {
-        dst[j] = -2;
-      }
-      if (dst[j] != -1) {
+      for (int j = 0; j < NB; ++j) {
+        const int k = k0 + 2 * j + half;
+        const uint32_t unit = uint32_t(__shfl(lo, k)), rest = uint32_t(__shfl(hi, k));
+        const int nde = 3 * int(rest >> 28);
+        at[j] = 0;
+        if (k >= nw || c > nde || (!RES && c == nde)) continue;
+        const double *blk = g.stage + int64_t(unit) * 16 + c;
 #pragma unroll
         for (int b = 0; b < 3; ++b)
           v[j][b] = ((fm >> b) & 1) ? __builtin_nontemporal_load(blk + b * (nde + 1)) : 0.0;
+        at[j] = c < nde ? g.pos[int64_t(rest & 0x0fffffffu) + cw] : kResidual;
       }
-    }
+    };
     // the three rows of one block are distinct targets: read the three sums, then write them
+    auto add = [&](const double (&v)[NB][3], const uint32_t (&at)[NB]) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+      for (int j = 0; j < NB; ++j) {
+        const int mw = int(at[j] >> 28);
+        const bool row = at[j] != kResidual;
+        const bool any = row ? ((mw >> cg) & 1) != 0 : true;
+        const int dst = int(at[j] & 0x0fffffffu) + __popc(mw & ((1 << cg) - 1));
+        double *t0 = row ? acc + rowoff[0] + dst : facc + 0;
+        double *t1 = row ? acc + rowoff[1] + dst : facc + 1;
+        double *t2 = row ? acc + rowoff[2] + dst : facc + 2;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (half == h && dst[j] != -1) {
-          double *t0 = (dst[j] >= 0) ? acc + rowoff[0] + dst[j] : facc + 0;
-          double *t1 = (dst[j] >= 0) ? acc + rowoff[1] + dst[j] : facc + 1;
-          double *t2 = (dst[j] >= 0) ? acc + rowoff[2] + dst[j] : facc + 2;
-          const double o0 = (fm & 1) ? *t0 : 0.0, o1 = (fm & 2) ? *t1 : 0.0, o2 = (fm & 4) ? *t2 : 0.0;
-          if (fm & 1) *t0 = o0 + v[j][0];
-          if (fm & 2) *t1 = o1 + v[j][1];
-          if (fm & 4) *t2 = o2 + v[j][2];
+        for (int h = 0; h < 2; ++h) {
+          if (half == h && any) {
+            const double o0 = (fm & 1) ? *t0 : 0.0, o1 = (fm & 2) ? *t1 : 0.0, o2 = (fm & 4) ? *t2 : 0.0;
+            if (fm & 1) *t0 = o0 + v[j][0];
+            if (fm & 2) *t1 = o1 + v[j][1];
+            if (fm & 4) *t2 = o2 + v[j][2];
+          }
+          __builtin_amdgcn_wave_barrier();
         }
-        __builtin_amdgcn_wave_barrier();
       }
+    };
+    for (int k0 = 0; k0 < nw; k0 += 2 * NB) {
+      double v[NB][3];
+      uint32_t at[NB];
+      load(k0, v, at);
+      add(v, at);
+    }
   }
   double *out = g.vals + g.row_start[node];
   for (int i = lane; i < nr * len; i += 64) __builtin_nontemporal_store(acc[i], out + i);
