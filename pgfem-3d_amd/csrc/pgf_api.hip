@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -195,7 +197,9 @@ struct pgf_handle_s {
   int nsc = 2;       // scalar components per QP of d_Sc
   bool j2_damage = false;  // a J2 material with continuum damage (mu > 0)
   bool he_linear = false;  // a hyperelastic material with the linear deviatoric law (devPotFlag 2)
-  int32_t *d_err = nullptr;
+  int32_t *d_err = nullptr;        // failure counter of the pass, zero between passes
+  int32_t *err_host = nullptr;     // pinned: where a pass leaves its count (-1 until then)
+  bool err_dirty = true;           // d_err may hold something else (new, or an aborted pass)
   double *d_red = nullptr;  // one scalar of a device reduction (pgf_subdivision_param)
   // crystal plasticity
   bool has_cp = false;
@@ -477,11 +481,10 @@ void build_gather(int64_t n_nodes, const int32_t *dofid, std::vector<GatherGroup
 
 // One pass over all elements in the pass schedule.
 // Every launch of one pass, in order, on the handle's stream (also what a captured graph
-// holds; the error counter is cleared by a kernel, not a memset node).
+// holds), the last of them leaving the failure count in h->err_host.
 // stage: the gather mode's staging blocks (stage_size doubles); nullptr selects the coloured
 // mode.
 int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, double *vals, double *stage) {
-  pgf::launch_fill_i32(h->d_err, 1, 0, h->stream);
   pgf::ElemArgs a = base_args(h, in);
   a.f = f;
   a.vals = vals;
@@ -610,7 +613,38 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
     pgf::launch_gather(mode, g, h->gather_waves, h->gather_batch, h->stream);
     ++launches;
   }
+  pgf::launch_publish(h->d_err, h->err_host, h->stream);
   return launches;
+}
+
+// Before a pass is launched.
+void begin_pass(pgf_handle h) {
+  if (h->err_dirty) pgf::launch_fill_i32(h->d_err, 1, 0, h->stream);
+  h->err_dirty = true;
+  *static_cast<volatile int32_t *>(h->err_host) = -1;
+}
+
+// Wait for the pass and return its failure count.  Its last kernel runs when all of its results
+// are written, so the count's arrival in host memory ends it: with a 4-byte copy to host memory, a
+// stream synchronization and a launch to clear the counter, a pass over 6,000 tet4 took 48 us, so
+// 33.  The wait in host memory is bounded; a long pass, or one that the device lost, ends in the
+// synchronization.
+int end_pass(pgf_handle h) {
+  volatile int32_t *count = h->err_host;
+  const auto t0 = std::chrono::steady_clock::now();
+  while (*count < 0 && std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(1)) {}
+  if (*count < 0 || h->profiling) {
+    if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  if (*count < 0) return PGF_EHIP;
+  h->err_dirty = false;
+  if (h->profiling) {
+    float ms = 0.f;
+    if (hipEventElapsedTime(&ms, h->ev0, h->ev1) != hipSuccess) return PGF_EHIP;
+    h->last_ms = ms;
+  }
+  return *count;
 }
 
 // Finish the handle's work and forget its captured pass: for setters that free or replace a
@@ -638,6 +672,8 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
                h->gather_batch};
   if (graph && !(h->gexec && key == h->gkey)) {
     if (h->gexec) {
+      // its last kernel may still be retiring (end_pass)
+      if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
       hipGraphExecDestroy(h->gexec);
       h->gexec = nullptr;
     }
@@ -653,6 +689,7 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
     }
     h->gkey = key;
   }
+  begin_pass(h);
   if (h->profiling) hipEventRecord(h->ev0, h->stream);
   if (graph) {
     if (hipGraphLaunch(h->gexec, h->stream) != hipSuccess) return PGF_EHIP;
@@ -662,16 +699,7 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
   }
   if (h->profiling) hipEventRecord(h->ev1, h->stream);
   if (hipGetLastError() != hipSuccess) return PGF_EHIP;
-  int32_t err = 0;
-  if (hipMemcpyAsync(&err, h->d_err, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream) != hipSuccess)
-    return PGF_EHIP;
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
-  if (h->profiling) {
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, h->ev0, h->ev1) != hipSuccess) return PGF_EHIP;
-    h->last_ms = ms;
-  }
-  return err;
+  return end_pass(h);
 }
 
 int field_buffer(pgf_handle h, int32_t field, double **buf, int32_t *ncomp) {
@@ -1138,6 +1166,7 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     if ((rc = pgf_set_orientations(h, 1, I9, nullptr))) return fail(rc);
   }
   if ((rc = pgf::dalloc(&h->d_err, 1))) return fail(rc);
+  if (hipHostMalloc(reinterpret_cast<void **>(&h->err_host), sizeof(int32_t)) != hipSuccess) return fail(PGF_ENOMEM);
   if ((rc = pgf::dalloc(&h->d_red, 1))) return fail(rc);
   if ((rc = set_identity_state(h))) return fail(rc);
   *out = h;
@@ -1206,6 +1235,7 @@ int pgf_destroy(pgf_handle h) {
     hipFree(h->d_Sc[t]);
   }
   hipFree(h->d_err);
+  if (h->err_host) hipHostFree(h->err_host);
   hipFree(h->d_red);
   if (h->ev0) hipEventDestroy(h->ev0);
   if (h->ev1) hipEventDestroy(h->ev1);
@@ -1287,21 +1317,13 @@ int pgf_residual_tangent_static(pgf_handle h, const pgf_nodal_input *in, double 
   if (dt > 0.0) h->dt = dt;
   // eager launches only: instantiating a graph may allocate.  Every staging block the pass
   // reads is written earlier in the same pass, so what an earlier call left is never read.
+  begin_pass(h);
   if (h->profiling) hipEventRecord(h->ev0, h->stream);
   h->last_launches = enqueue_pass(h, in, pgf::MODE_INTEGRATE | pgf::MODE_RESIDUAL | pgf::MODE_TANGENT, f, vals,
                                   h->stage_size ? stage : nullptr);
   if (h->profiling) hipEventRecord(h->ev1, h->stream);
   if (hipGetLastError() != hipSuccess) return PGF_EHIP;
-  int32_t err = 0;
-  if (hipMemcpyAsync(&err, h->d_err, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream) != hipSuccess)
-    return PGF_EHIP;
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
-  if (h->profiling) {
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, h->ev0, h->ev1) != hipSuccess) return PGF_EHIP;
-    h->last_ms = ms;
-  }
-  return err;
+  return end_pass(h);
 }
 
 int pgf_output_variables(pgf_handle h, int32_t level, double *S, double *E, double *sigma, double *eps) {
@@ -1516,6 +1538,7 @@ int pgf_tf_initial(pgf_handle h, const pgf_nodal_input *in_n, const pgf_nodal_in
   if (!h || !h->tf || !in_n || !in_n->r) return PGF_EINVAL;
   const int64_t NE = h->n_elem;
   pgf::launch_fill_i32(h->d_err, 1, 0, h->stream);
+  h->err_dirty = true;
   for (int s = 0; s < 2; ++s) {
     const pgf_nodal_input *in = (s == 1 && in_nm1) ? in_nm1 : in_n;
     if (!in->r) return PGF_EINVAL;

@@ -314,6 +314,7 @@ void launch_tf_initial(int nne, const TfArgs &t, hipStream_t s);
 void launch_axpy(double *y, const double *x, double g, int64_t n, hipStream_t s);  // y += g x
 void launch_fill(double *p, int64_t n, double v, hipStream_t s);
 void launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s);
+void launch_publish(int32_t *count, int32_t *host, hipStream_t s);
 void launch_rate_max(const double *a, int ncomp, int64_t stride, int64_t n, double scale, const double *d1,
                      const double *d0, double scale_d, unsigned long long *out, hipStream_t s);
 void launch_copy(double *dst, const double *src, int64_t n, hipStream_t s);

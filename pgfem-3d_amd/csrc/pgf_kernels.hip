@@ -979,6 +979,13 @@ __global__ void fill_kernel(double *p, int64_t n, double v) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
     p[i] = v;
 }
+// The end of a pass: the failure count to pinned host memory, and the counter cleared for the next
+// pass.  Every earlier kernel of the stream is done when it runs.
+__global__ void publish_kernel(int32_t *count, int32_t *host) {
+  const int32_t n = *count;
+  *count = 0;
+  __hip_atomic_store(host, n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 __global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
     p[i] = v;
@@ -1227,6 +1234,7 @@ void launch_fill(double *p, int64_t n, double v, hipStream_t s) {
   fill_kernel<<<unsigned(blocks), 256, 0, s>>>(p, n, v);
 }
 
+void launch_publish(int32_t *count, int32_t *host, hipStream_t s) { publish_kernel<<<1, 1, 0, s>>>(count, host); }
 void launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t s) {
   if (n <= 0) return;
   const int64_t blocks = std::min<int64_t>((n + 255) / 256, 8192);

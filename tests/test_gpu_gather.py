@@ -52,3 +52,25 @@ def test_fan_of_tets(device, m, batch):
         h.close()
     for a, b in zip(*out):
         assert np.abs(a - b).max() <= TOL * np.abs(b).max()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_failure_counts_belong_to_their_pass(device, graph):
+    """Inverted elements are counted by the pass that meets them, eager and replayed, and by no
+    later one."""
+    mesh, ids, ndof = _fan(9)
+    Ap, Ai = P.psparse_apai(mesh, ids, ndof)
+    good = torch.zeros(ndof, dtype=torch.float64, device=device)
+    bad = good.clone()
+    bad[int(ids[0, 2]) - 1] = -2.5  # the upper end node below the lower one: all nine inverted
+    h = P.Handle(mesh, ids, ndof, Ap, Ai, [P.neo_hookean(200e3, 0.3)])
+    h.set_graph(graph)
+    f, buf = torch.empty_like(good), good.clone()
+    counts = []
+    for r in (good, bad, bad, good, bad, good, good):
+        buf.copy_(r)
+        torch.cuda.synchronize()
+        counts.append(h.residual(f, buf, run_integration=True))
+    n = counts[1]
+    assert n >= 9 and counts == [0, n, n, 0, n, 0, 0]
+    h.close()
