@@ -1562,19 +1562,12 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
 }
 
 // ------------------------------------------------------------------- element kernel
-// Elements per round of the LDS transpose of the staged rows (gather mode): the largest
-// divisor of epb whose rows (nde x (nde+1) doubles each) fit in the dead dM/dF array.
-constexpr int cp_stage_round(int epb, int nde, int room) {
-  int re = epb;
-  while (re > 1 && (epb % re != 0 || re * nde * (nde + 1) > room)) --re;
-  return re;
-}
-
 // Rows of the displacement element from the points' records: with T and the moduli A of
 // store_moduli, f_ab = sum_j T_bj dN_a,j and K_ab,wg = sum_l (sum_j dN_a,j A[b j][g l]) dN_w,l.
-// One lane per row, the points one after another.  Bound by memory: 538 us for 998,250 tet4, 2.3 GB
-// moved at 4.3 TB/s, the rate of a copy.  (1417 us with the point's tensors formed here; 716 with the
-// rows stored by their lanes, 8 bytes every 104, instead of through LDS.)
+// One lane per row, the points one after another.  Bound by memory: 490 us for 998,250 tet4, 2.3 GB
+// moved at 4.8 TB/s, the rate of a copy.  (1417 us with the point's tensors formed here; 716 with the
+// rows stored by their lanes, 8 bytes every 104, instead of through LDS; 538 with each store's
+// staging offset loaded just before it.)
 template <int NNE, int MODE, bool STG>
 __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, int64_t e_end) {
   constexpr int NQP = nqp_of(NNE);
@@ -1593,7 +1586,15 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
   __shared__ int32_t s_dof[EPB][NDE], s_node[EPB][NNE];
   __shared__ double s_dN[EPB][NQP][NDE];
   __shared__ double s_T[EPB][NQP][RES ? 9 : 1];
-  __shared__ double s_D[EPB][NQP][TAN ? 81 : 1];  // A[b j][g l], row-major
+  // staging offsets: loaded with the nodes, so that the stores at the end wait for no load
+  __shared__ int64_t s_so[EPB][WK && STG ? NNE : 1];
+  constexpr int LD = NDE + 1;
+  constexpr int EPW = 64 / TPE;
+  constexpr int kD = EPB * NQP * (TAN ? 81 : 1);
+  constexpr int RE = stage_round(EPW, NDE, kD);
+  constexpr int kS = WK && STG ? 4 * RE * NDE * LD : 0;
+  __shared__ double s_work[kD > kS ? kD : kS];  // A[b j][g l], row-major, then the staged rows
+  auto s_D = reinterpret_cast<double (*)[NQP][TAN ? 81 : 1]>(s_work);
 
   const int slot = threadIdx.x / TPE, lane = threadIdx.x % TPE;
   const int64_t ie = e_begin + int64_t(blockIdx.x) * EPB + slot;
@@ -1602,6 +1603,7 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
   if (active && lane < NNE) {
     const int32_t node = a.conn[e * NNE + lane];
     s_node[slot][lane] = node;
+    if constexpr (WK && STG) s_so[slot][lane] = a.soff[e * NNE + lane];
 #pragma unroll
     for (int b = 0; b < 3; ++b) {
       const int32_t d = a.dofid[int64_t(node) * 3 + b];
@@ -1684,41 +1686,40 @@ __global__ __launch_bounds__(256) void cp_elem(CPElemArgs a, int64_t e_begin, in
     fe = s;
   }
   }  // rowlane
-  constexpr int LD = NDE + 1;
   if constexpr (WK && STG) {
-    // Gather mode: RE elements at a time, the rows go to LDS (in the dead moduli) laid out as the
-    // staging blocks, then the workgroup copies each node block, zero-padded to whole lines, to
-    // its staging offset with consecutive threads on consecutive doubles.
+    // Gather mode: each wave lays RE of its elements' rows out in LDS as the staging blocks
+    // ([node a][row b][K row, residual]) and copies each node block (3 (NDE+1) doubles,
+    // zero-padded to whole lines) to its staging offset, consecutive lanes on consecutive doubles.
+    // Rows of prescribed DOFs are copied too (nothing reads them; it keeps every line whole);
+    // nodes without free DOFs have no block.  No wave waits for another's rows.
     constexpr int PB = stage_block(NNE);
-    constexpr int RE = cp_stage_round(EPB, NDE, EPB * NQP * 81);
-    static_assert(RE * NDE * LD <= EPB * NQP * 81, "staging round does not fit");
-    double *s_st = &s_D[0][0][0];
-    lds_barrier();  // every lane is done with s_D
+    constexpr int PB2 = PB / 2;  // two doubles per lane (blocks are whole 128-byte lines)
+    lds_barrier();  // every lane is done with the moduli
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), wl = threadIdx.x % 64;
+    double *st = s_work + wave * (RE * NDE * LD);
 #pragma unroll 1
-    for (int r0 = 0; r0 < EPB; r0 += RE) {
+    for (int r0 = wave * EPW; r0 < (wave + 1) * EPW; r0 += RE) {
       if (rowlane && slot >= r0 && slot < r0 + RE) {
-        double *row = s_st + ((slot - r0) * NDE + lane) * LD;
+        double *row = st + ((slot - r0) * NDE + lane) * LD;
 #pragma unroll
         for (int i = 0; i < NDE; ++i) row[i] = K[i];
         row[NDE] = fe;
       }
-      lds_barrier();
-      // two doubles per thread (blocks are whole 128-byte lines, so pairs are 16-byte aligned)
-      constexpr int PB2 = PB / 2;
-      for (int idx = threadIdx.x; idx < RE * NNE * PB2; idx += blockDim.x) {
+      __builtin_amdgcn_wave_barrier();
+      for (int idx = wl; idx < RE * NNE * PB2; idx += 64) {
         const int el = idx / (NNE * PB2), o = idx - el * (NNE * PB2);
         const int na = o / PB2, ob = 2 * (o - na * PB2);
-        const int64_t ee = e_begin + int64_t(blockIdx.x) * EPB + r0 + el;
-        if (ee >= e_end) continue;
-        const int64_t so = a.soff[ee * NNE + na];
+        if (e_begin + int64_t(blockIdx.x) * EPB + r0 + el >= e_end) continue;
+        const int64_t so = s_so[r0 + el][na];
         if (so < 0) continue;
-        const double *src = s_st + (el * NDE + na * 3) * LD + ob;
+        const double *src = st + (el * NDE + na * 3) * LD + ob;
         dbl2 v;
         v.x = (ob < 3 * LD) ? src[0] : 0.0;
         v.y = (ob + 1 < 3 * LD) ? src[1] : 0.0;
+        // streamed past L2: the gather reads it in a later launch
         __builtin_nontemporal_store(v, reinterpret_cast<dbl2 *>(a.stage + so + ob));
       }
-      lds_barrier();
+      __builtin_amdgcn_wave_barrier();
     }
     return;
   }

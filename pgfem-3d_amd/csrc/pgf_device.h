@@ -24,6 +24,13 @@ __device__ __forceinline__ void lds_barrier() {
 // element's K row (3 nne) and residual entry, padded to whole 128-byte lines so every line
 // of a block is written whole by the element that owns it.
 __host__ __device__ constexpr int stage_block(int nne) { return (3 * (3 * nne + 1) + 15) & ~15; }
+// Elements whose rows a wave stages at a time, of the epw it holds (elem_kernel, cp_elem): as many
+// as four waves have LDS for in an array of `room` doubles, at least one.
+__host__ __device__ constexpr int stage_round(int epw, int nde, int room) {
+  int re = epw;
+  while (re > 1 && 4 * re * nde * (nde + 1) > room) re /= 2;
+  return re;
+}
 
 // Device copy of the per-material constants used by the kernels.
 struct DevMaterial {

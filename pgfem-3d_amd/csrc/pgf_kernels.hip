@@ -323,26 +323,30 @@ __device__ __forceinline__ void j2_point(const DevMaterial &m, bool plastic, con
   }
 }
 
-// Elements per round of the LDS transpose that turns the lanes' element rows into
-// contiguous staging-block stores: the largest divisor of epb whose rows (nde x (nde+1)
-// doubles each) fit in the `room` doubles of the dead shape-gradient and tangent arrays.
-constexpr int stage_round(int epb, int nde, int room) {
-  int re = epb;
-  while (re > 1 && (epb % re != 0 || re * nde * (nde + 1) > room)) --re;
-  return re;
-}
-
 // TF: the CM3F three-field element of the hyperelastic model (one volume and one pressure
 // variable per element, condensed): F(n+1) is always Fr (the model stores (theta/J)^1/3 Fr),
 // tau and c take the element pressure, and the rows get the condensation terms.  Its staged
 // variant runs at three waves per SIMD: at four (128 registers) the extra element terms spill.
+// Bound, on large tet10 meshes, by FP64 issue (half of the cycles) and by the rate at which the
+// staged rows are written (2.9 TB/s), which overlap as far as four workgroups per CU let them: 1.80 ms on
+// 663,552 J2 tet10 (1.75 without the stores, 1.79 with the stores alone).  The staging offsets are
+// loaded with the nodes (a load ahead of every store was 2.20 ms -> 2.00), each wave stages its own
+// rows (no barriers in the transpose: 2.00 -> 1.90), and the QP phase, one wave's, has its node
+// loops unrolled over registers (1.90 -> 1.80; three-field tet10, 93,750: 295 -> 249 us in all).
 // VAR: 0 the displacement element, 1 the three-field element (TF), 2 the displacement
 // element with J2 continuum damage (DMG: the undamaged kernels keep their register budget),
 // 3 the hyperelastic displacement element whose materials may take the linear deviatoric law
 // (LIN, chosen per element from devPotFlag).
+// Waves per SIMD: four in gather mode (128 registers).  The tangent at a displacement other than the
+// state's keeps Fr Fs^-1 as well and on hex8 spills 324 bytes at four; at three (and with VAR)
+// 142 us instead of 160 on 33^3.
+constexpr int elem_waves(int nne, int mode, bool stg, int var) {
+  const bool gen_tan = !(mode & MODE_INTEGRATE) && (mode & MODE_TANGENT);
+  return !stg ? 1 : (var != 0 || (nne == 8 && gen_tan) ? 3 : 4);
+}
 template <int NNE, int MODE, bool STG, int VAR>
-__global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel(ElemArgs a, int64_t e_begin,
-                                                                                int64_t e_end) {
+__global__ __launch_bounds__(256, elem_waves(NNE, MODE, STG, VAR)) void elem_kernel(ElemArgs a, int64_t e_begin,
+                                                                                  int64_t e_end) {
   constexpr bool TF = VAR == 1;
   constexpr bool DMG = VAR == 2;
   constexpr bool LIN = VAR == 3;
@@ -360,21 +364,27 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
   constexpr bool GEN = !INTEG && !TF;  // Fr may differ from the stored F(n+1)
   constexpr int LD = NDE + 1;   // staging row: K row, then the residual entry
   constexpr int kH = EPB * NQP * NDE, kC = EPB * NQP * (TAN ? 36 : 1);
-  constexpr int RE = stage_round(EPB, NDE, kH + kC);
-  static_assert(!TAN || RE * NDE * LD <= kH + kC, "staging round does not fit");
+  constexpr int EPW = 64 / TPE;
+  constexpr int RE = stage_round(EPW, NDE, kH + kC);
+  constexpr int kS = WK && STG ? 4 * RE * NDE * LD : 0;
 
-  __shared__ double s_u[EPB][NDE];
   __shared__ int32_t s_dof[EPB][NDE];
   __shared__ int32_t s_node[EPB][NNE];
-  __shared__ double s_x[EPB][NDE];
-  // shape gradients and tangents; reused as the staging transpose buffer after phase 2
-  __shared__ double s_work[kH + kC];
+  // shape gradients and tangents; reused as the staging transpose buffer after phase 2.  The
+  // nodes' positions and displacements are read before the QP's lanes, one wave, write its tangent
+  // over them.
+  constexpr int kX = 2 * EPB * NDE, kW = kH + (kC > kX ? kC : kX);
+  __shared__ double s_work[kW > kS ? kW : kS];
+  auto s_x = reinterpret_cast<double (*)[NDE]>(s_work + kH);
+  auto s_u = s_x + EPB;
   auto s_h = reinterpret_cast<double (*)[NQP][NDE]>(s_work);
   auto s_c = reinterpret_cast<double (*)[NQP][TAN ? 36 : 1]>(s_work + kH);
   __shared__ double s_tau[EPB][NQP][6];
   __shared__ double s_g[EPB][NQP][GEN ? 9 : 1];
   __shared__ double s_dl[EPB][DFL ? NDE : 1];  // prescribed increments of the element DOFs
   __shared__ double s_tf[EPB][NQP][TF ? 1 : 1];  // three-field: detJ w J per QP
+  // staging offsets: loaded with the nodes, so that the stores at the end wait for no load
+  __shared__ int64_t s_so[EPB][WK && STG ? NNE : 1];
   __shared__ double s_tfe[EPB][TF ? 6 : 1];      // three-field, per element: Ktt/V^2, the residual
                                                  // coefficient, fp, ft, Ktt, V
 
@@ -424,7 +434,10 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
     const int nl = lane / 3, b = lane - 3 * nl;
     const int32_t node = a.conn[e * NNE + nl];
     const int32_t d = a.edof[e * NDE + lane];
-    if (b == 0) s_node[slot][nl] = node;
+    if (b == 0) {
+      s_node[slot][nl] = node;
+      if constexpr (WK && STG) s_so[slot][nl] = a.soff[e * NNE + nl];
+    }
     s_x[slot][lane] = a.X[int64_t(node) * 3 + b];
     s_dof[slot][lane] = d;
     double u = 0.0;  // def_elem_total, src/utils.cc:1391-1412
@@ -455,30 +468,33 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
     double k, ee, z, wt;
     int_point(NNE, ip, k, ee, z, wt);
     double *hq = s_h[slot][ip];  // dN/dX first, h_a = Fs^-T dN_a/dX at the end
+    // The loops over the lane's nodes are unrolled, so that their LDS reads overlap.
+    constexpr int NPL = NNE / LPQ;
+    static_assert(NPL * LPQ == NNE, "nodes per lane");
+    double d[NPL][3];  // dN of the lane's nodes
     {
       double dN[NDE];
       shape_dN<NNE>(k, ee, z, dN);
 #pragma unroll
-      for (int n = 0; n < NNE; ++n)
-        if (n % LPQ == sub) {
-          hq[n * 3 + 0] = dN[n * 3 + 0];
-          hq[n * 3 + 1] = dN[n * 3 + 1];
-          hq[n * 3 + 2] = dN[n * 3 + 2];
+      for (int t = 0; t < NPL; ++t)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          d[t][i] = dN[t * LPQ * 3 + i];
+#pragma unroll
+          for (int l = 1; l < LPQ; ++l) d[t][i] = sub == l ? dN[(t * LPQ + l) * 3 + i] : d[t][i];
         }
     }
     double dX[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) dX[i] = 0.0;
-    for (int n = sub; n < NNE; n += LPQ) {
-      const double d0 = hq[n * 3 + 0], d1 = hq[n * 3 + 1], d2 = hq[n * 3 + 2];
+#pragma unroll
+    for (int t = 0; t < NPL; ++t)
 #pragma unroll
       for (int ib = 0; ib < 3; ++ib) {
-        const double xb = s_x[slot][n * 3 + ib];
-        dX[ib * 3 + 0] += d0 * xb;
-        dX[ib * 3 + 1] += d1 * xb;
-        dX[ib * 3 + 2] += d2 * xb;
+        const double xb = s_x[slot][(t * LPQ + sub) * 3 + ib];
+#pragma unroll
+        for (int ic = 0; ic < 3; ++ic) dX[ib * 3 + ic] += d[t][ic] * xb;
       }
-    }
 #pragma unroll
     for (int i = 0; i < 9; ++i) dX[i] = group_sum<LPQ>(dX[i]);
     const double J0 = det3(dX);
@@ -497,11 +513,13 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
     double Fr[9];  // sum of u_n (x) dN_n/dX over the lane's nodes, then over the QP's lanes
 #pragma unroll
     for (int i = 0; i < 9; ++i) Fr[i] = 0.0;
-    for (int n = sub; n < NNE; n += LPQ) {
-      const double d0 = hq[n * 3 + 0], d1 = hq[n * 3 + 1], d2 = hq[n * 3 + 2];
+#pragma unroll
+    for (int t = 0; t < NPL; ++t) {
+      const int n = t * LPQ + sub;
       double g[3];
 #pragma unroll
-      for (int ib = 0; ib < 3; ++ib) g[ib] = rJ0 * (d0 * cof[0 * 3 + ib] + d1 * cof[1 * 3 + ib] + d2 * cof[2 * 3 + ib]);
+      for (int ib = 0; ib < 3; ++ib)
+        g[ib] = rJ0 * (d[t][0] * cof[0 * 3 + ib] + d[t][1] * cof[1 * 3 + ib] + d[t][2] * cof[2 * 3 + ib]);
 #pragma unroll
       for (int ib = 0; ib < 3; ++ib) {
         hq[n * 3 + ib] = g[ib];  // dN/dX
@@ -633,10 +651,12 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
           if ((i * 3 + j) % LPQ == sub)
             s_g[slot][ip][i * 3 + j] = Fr[i * 3 + 0] * Fi[0 * 3 + j] + Fr[i * 3 + 1] * Fi[1 * 3 + j] + Fr[i * 3 + 2] * Fi[2 * 3 + j];
     }
-    for (int n = sub; n < NNE; n += LPQ) {
-      const double d0 = hq[n * 3 + 0], d1 = hq[n * 3 + 1], d2 = hq[n * 3 + 2];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) hq[n * 3 + i] = Fi[0 * 3 + i] * d0 + Fi[1 * 3 + i] * d1 + Fi[2 * 3 + i] * d2;
+    for (int t = 0; t < NPL; ++t) {
+      double *hn = hq + (t * LPQ + sub) * 3;
+      const double d0 = hn[0], d1 = hn[1], d2 = hn[2];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) hn[i] = Fi[0 * 3 + i] * d0 + Fi[1 * 3 + i] * d1 + Fi[2 * 3 + i] * d2;
     }
   }
   lds_barrier();
@@ -760,40 +780,39 @@ __global__ __launch_bounds__(256, STG ? (VAR != 0 ? 3 : 4) : 1) void elem_kernel
     }
   }
   if constexpr (WK && STG) {
-    // Gather mode: RE elements at a time, the rows go to LDS laid out as the staging blocks
-    // ([node a][row b][K row, residual]); then the whole workgroup copies each node block
-    // (3 (NDE+1) doubles, zero-padded to whole lines) to its staging offset, consecutive
-    // threads on consecutive doubles.  Rows of prescribed DOFs are copied too (nothing reads
-    // them; it keeps every line whole); nodes without free DOFs have no block.
+    // Gather mode: each wave lays RE of its elements' rows out in LDS as the staging blocks
+    // ([node a][row b][K row, residual]) and copies each node block (3 (NDE+1) doubles,
+    // zero-padded to whole lines) to its staging offset, consecutive lanes on consecutive doubles.
+    // Rows of prescribed DOFs are copied too (nothing reads them; it keeps every line whole);
+    // nodes without free DOFs have no block.  No wave waits for another's rows.
     constexpr int PB = stage_block(NNE);
+    constexpr int PB2 = PB / 2;  // two doubles per lane (blocks are whole 128-byte lines)
     lds_barrier();  // every lane is done with s_h / s_c
-    const int64_t e_blk = e_begin + blk * EPB;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), wl = threadIdx.x % 64;
+    double *st = s_work + wave * (RE * NDE * LD);
 #pragma unroll 1
-    for (int r0 = 0; r0 < EPB; r0 += RE) {
+    for (int r0 = wave * EPW; r0 < (wave + 1) * EPW; r0 += RE) {
       if (rowlane && slot >= r0 && slot < r0 + RE) {
-        double *row = s_work + ((slot - r0) * NDE + lane) * LD;
+        double *row = st + ((slot - r0) * NDE + lane) * LD;
 #pragma unroll
         for (int i = 0; i < NDE; ++i) row[i] = K[i];
         row[NDE] = fe;
       }
-      lds_barrier();
-      // two doubles per thread (blocks are whole 128-byte lines, so pairs are 16-byte aligned)
-      constexpr int PB2 = PB / 2;
-      for (int idx = threadIdx.x; idx < RE * NNE * PB2; idx += 256) {
+      __builtin_amdgcn_wave_barrier();
+      for (int idx = wl; idx < RE * NNE * PB2; idx += 64) {
         const int el = idx / (NNE * PB2), o = idx - el * (NNE * PB2);
         const int na = o / PB2, ob = 2 * (o - na * PB2);
-        const int64_t ee = e_blk + r0 + el;
-        if (ee >= e_end) continue;
-        const int64_t so = a.soff[ee * NNE + na];
+        if (e_begin + blk * EPB + r0 + el >= e_end) continue;
+        const int64_t so = s_so[r0 + el][na];
         if (so < 0) continue;
-        const double *src = s_work + (el * NDE + na * 3) * LD + ob;
+        const double *src = st + (el * NDE + na * 3) * LD + ob;
         dbl2 v;
         v.x = (ob < 3 * LD) ? src[0] : 0.0;
         v.y = (ob + 1 < 3 * LD) ? src[1] : 0.0;
         // streamed past L2: the gather reads it in a later launch
         __builtin_nontemporal_store(v, reinterpret_cast<dbl2 *>(a.stage + so + ob));
       }
-      lds_barrier();
+      __builtin_amdgcn_wave_barrier();
     }
     return;
   }
