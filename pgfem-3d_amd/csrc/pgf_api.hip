@@ -213,11 +213,10 @@ struct pgf_handle_s {
   int32_t cp_law = 0;  // elastic law of the crystal-plasticity material (pgf_material.cp_elastic)
   int32_t cp_flow = 0;  // what its flow and hardening rule need pow for (pgf::CPArgs::flow)
   int64_t cp_nq = 0;         // crystal-plasticity QPs: device QPs [0, cp_nq)
-  // QPs per wave range of the local Newton (autotuned; 1: every wave draws from one global queue).
-  // A wave's own batch of 64 spreads a mesh over the most SIMDs, and nothing is carried from one
-  // batch to the next: cp_newton on 10,368 QPs 184 us at 256, 99 at 128, 55 at 64, 57 at 1; on
-  // 998,250 QPs 774, 769, 755, 735.
-  int64_t cp_chunk = 64;
+  // QPs per wave range of the local Newton (autotuned; 1: one global queue, or where that has nothing
+  // to balance a batch of 64 per wave).  cp_newton on 10,368 QPs 184 us at 256, 99 at 128, 55 at
+  // 64 and 1; on 998,250 QPs 774, 769, 755, 735.
+  int64_t cp_chunk = 1;
   unsigned long long *d_qnext = nullptr;  // the global queue's counter
   int32_t gather_waves = 4;  // nodes per gather workgroup (autotuned; capped by LDS)
   int32_t gather_batch = 4;  // staging blocks each gather half-wave keeps in flight (autotuned)

@@ -606,8 +606,9 @@ __device__ __forceinline__ bool eliminate(double (&A)[N * N], double (&B)[NR][N]
     }
   return lmax <= max_mult && fabs(rd[N - 1]) < __builtin_huge_val();
 }
-// The same with partial pivoting, in scratch memory: rare, and kept from costing the common path
-// registers (the system is stored before the common path consumes it, and solved after it).
+// The same with partial pivoting, in LDS, for one lane: rare, and kept from costing the common path
+// registers (the system is stored before the common path consumes it, and solved after it).  In a
+// lane's scratch memory every step waited for it: 100 us for a wave that met such a point.
 // The solutions take the right-hand sides' places; false for a singular matrix.
 template <int N, int NR>
 __device__ __forceinline__ void store_system(const double (&A)[N * N], const double (&B)[NR][N], double *a) {
@@ -852,16 +853,17 @@ __global__ __launch_bounds__(64) void cp_start_kernel(CPArgs a) {
 }
 
 // ------------------------------------------------------------------- Newton kernel
-// One wave per workgroup, one QP per lane, 64 QPs at a time: wave w works through QPs
-// [w*chunk, (w+1)*chunk) of the block, or, with a.qnext set, draws its batches from one global
-// queue.  Which lane takes a QP does not change its result.  A batch ends when its last QP has
-// converged (mean 5.1 iterations, largest 8): handing a free lane the next QP instead gained
-// nothing, since the wave then reads and writes that QP's state alone.  The starting points come
-// from cp_start_kernel (qpbuf).
+// One wave per workgroup, one QP per lane: wave w works through QPs [w*chunk, (w+1)*chunk) of the
+// block, or, with a.qnext set, draws them from one global queue.  Which lane takes a QP does not
+// change its result.  A wave hands out new QPs when kRefill of its lanes are idle: at each idle lane it
+// would wait for that QP's state too often (no gain over whole batches), and in whole batches it
+// waits for the batch's last QP: with up to 25 iterations (178,752 QPs) the pass took 1000 us at 64,
+// 900 at 48, 32 and 16; with a mean of 5 and at most 8 (998,250 QPs) all are within 2%.  The starting
+// points come from cp_start_kernel (qpbuf).
 //
 // Bound by FP64 issue: a turn is about 3300 instructions for 64 QPs.  A turn has no divergent
 // branch around its stages (values would be kept across it), and each stage is closed by pin, so
-// the widest stretch, the 9 x 9 elimination, fits 306 registers with nothing spilled.  One wave
+// the widest stretch, the 9 x 9 elimination, fits 298 registers with nothing spilled.  One wave
 // per SIMD: at two, 256 registers spill and it takes 800 us instead of 740 (998,250 QPs; 2743 us
 // in the sample frame, with the pivoting and the slip systems' tensors in registers).
 template <bool HE, int FLOW>
@@ -871,264 +873,276 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
   // The lane's QP data that lives across turns sits in LDS (lane-fastest; each lane touches
   // only its own slots), read where used, rather than in registers held through the material
   // point and the elimination: A (9), x (11), dx (11), det pF(n), g(n), gscale.  17 KB per wave.
-  __shared__ double sPk[34 * 64];
+  __shared__ double sPk[34 * 64], sSystem[9 * 11];
   double *pk = sPk + lane;  // field i at pk[i * 64]
   constexpr int kA = 0, kX = 9, kDX = 20, kDet = 31, kGn = 32, kGs = 33;
+  constexpr int kRefill = 48;
   const double dt = a.dt;
   const CPMaterial cm = a.cpmats[0];  // one material for every CP point: wave-uniform, loaded once
   // the lane's phase: evaluate the start, a line-search trial x + alpha dx, the full step after 40
   // halvings without a decrease, or x once more, for a step with a pivoting elimination
   constexpr int kPhStart = 0, kPhTrial = 1, kPhFull = 2, kPhAgain = 3, kPhDone = 4;
-  int64_t q0 = int64_t(blockIdx.x) * chunk;
-  const int64_t q_hi = a.qnext ? a.nq : (q0 + chunk < a.nq ? q0 + chunk : a.nq);
-  for (;; q0 += 64) {
-    if (a.qnext) {
-      unsigned long long base = 0;
-      if (lane == 0) base = atomicAdd(a.qnext, 64ull);
-      q0 = int64_t(__shfl((long long)base, 0));
-    }
-    if (q0 >= q_hi) break;
-    const int64_t qg = a.qp_base + q0 + lane;
-    const bool live = q0 + lane < q_hi;
-    int kind = 0;  // the QP's start: 0 plain, 1 the caller's (learned), 2 the caller's, then the plain fallback
-    int phase = kPhDone, it = 0, it_att = 0, ls = 0;
-    bool bad_start = false, failed = false;
-    double f0 = 0.0, alpha = 1.0;
-    if (live) {
-      double F[9], pFn[9], pFi[9], T[9], A[9], det = 0.0;
+  int64_t next = int64_t(blockIdx.x) * chunk;  // the range's first point that no lane has taken
+  const int64_t q_hi = a.qnext ? a.nq : (next + chunk < a.nq ? next + chunk : a.nq);
+  bool more = true;
+  int64_t q = -1;  // the lane's point
+  int kind = 0;    // its start: 0 plain, 1 the caller's (learned), 2 the caller's, then the plain fallback
+  int phase = kPhDone, it = 0, it_att = 0, ls = 0;
+  bool bad_start = false, failed = false;
+  double f0 = 0.0, alpha = 1.0;
+  for (;;) {
+    const uint64_t idle = __ballot(phase == kPhDone);
+    const int n_idle = __popcll(idle);
+    if (n_idle == 64 || (more && n_idle >= kRefill)) {
+      if (phase == kPhDone && q >= 0) {
+        const int64_t qg = a.qp_base + q;
+        a.iters[qg] = it | (kind << 24);  // iterations, and the start in the high byte
+        if (failed) {
+          atomicAdd(a.err, 1);
+        } else {
+          // pF(n+1) = M^-1 pF(n)
+          double x[11], Mc[9], Mi[9] = {}, pFn[9], pF1[9], det;
 #pragma unroll
-      for (int i = 0; i < 9; ++i) {
-        F[i] = a.F_np1[i * NQ + qg];
-        pFn[i] = a.pF_n[i * NQ + qg];
-        pFi[i] = 0.0;
+          for (int i = 0; i < 11; ++i) x[i] = pk[(kX + i) * 64];
+          rot_out_1(a.grains[a.qgrain[q]].R, x, Mc);
+          inv_det(Mc, Mi, det);
+#pragma unroll
+          for (int i = 0; i < 9; ++i) pFn[i] = a.pF_n[i * NQ + qg];
+          mul_ab(Mi, pFn, pF1);
+#pragma unroll
+          for (int i = 0; i < 9; ++i) a.pF_np1[i * NQ + qg] = pF1[i];
+          a.Sc_np1[qg] = x[10];
+          a.Sc_np1[NQ + qg] = x[9];
+        }
       }
-      const double *R = a.grains[a.qgrain[q0 + lane]].R;
-      inv_det(pFn, pFi, det);
-      mul_ab(F, pFi, T);
-      rot_in_1(R, T, A);
+      if (phase == kPhDone) q = -1;
+      if (more) {
+        if (a.qnext) {
+          unsigned long long base = 0;
+          if (lane == 0) base = atomicAdd(a.qnext, (unsigned long long)n_idle);
+          next = int64_t(__shfl((long long)base, 0));
+        }
+        const int64_t mine = next + __popcll(idle & ((1ull << lane) - 1));
+        next += n_idle;
+        more = next < q_hi;
+        if (phase == kPhDone && mine < q_hi) {
+          q = mine;
+          const int64_t qg = a.qp_base + q;
+          kind = it = it_att = ls = 0;
+          failed = false;
+          double F[9], pFn[9], pFi[9], T[9], A[9], det = 0.0;
 #pragma unroll
-      for (int i = 0; i < 9; ++i) pk[(kA + i) * 64] = A[i];
-      pk[kDet * 64] = det;
-      const double g_n = a.g_n[qg];
-      pk[kGn * 64] = g_n;
-      pk[kGs * 64] = 1.0 / (fabs(cm.gs0 - cm.g0) * g_n + 1e-300);
-      phase = kPhStart;
-      // start: the caller's warm start where cp_start_kernel chose it, else the plain start
-      const double *row = a.qpbuf + qrec(qg);
-      const int flag = int(row[kStartFlag * kRecStride]);
-      bad_start = (flag & 1) != 0;
-      if (flag & 2) {
+          for (int i = 0; i < 9; ++i) {
+            F[i] = a.F_np1[i * NQ + qg];
+            pFn[i] = a.pF_n[i * NQ + qg];
+            pFi[i] = 0.0;
+          }
+          const double *R = a.grains[a.qgrain[q]].R;
+          inv_det(pFn, pFi, det);
+          mul_ab(F, pFi, T);
+          rot_in_1(R, T, A);
 #pragma unroll
-        for (int i = 0; i < 9; ++i) T[i] = a.warm[i * NQ + qg];
-        rot_in_1(R, T, A);
+          for (int i = 0; i < 9; ++i) pk[(kA + i) * 64] = A[i];
+          pk[kDet * 64] = det;
+          const double g_n = a.g_n[qg];
+          pk[kGn * 64] = g_n;
+          pk[kGs * 64] = 1.0 / (fabs(cm.gs0 - cm.g0) * g_n + 1e-300);
+          phase = kPhStart;
+          // start: the caller's warm start where cp_start_kernel chose it, else the plain start
+          const double *row = a.qpbuf + qrec(qg);
+          const int flag = int(row[kStartFlag * kRecStride]);
+          bad_start = (flag & 1) != 0;
+          if (flag & 2) {
 #pragma unroll
-        for (int i = 0; i < 9; ++i) pk[(kX + i) * 64] = A[i];
-        pk[(kX + 9) * 64] = a.warm[9 * NQ + qg];
-        pk[(kX + 10) * 64] = a.warm[10 * NQ + qg];
-        kind = 1;
-        bad_start = false;
-      } else {
+            for (int i = 0; i < 9; ++i) T[i] = a.warm[i * NQ + qg];
+            rot_in_1(R, T, A);
 #pragma unroll
-        for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
+            for (int i = 0; i < 9; ++i) pk[(kX + i) * 64] = A[i];
+            pk[(kX + 9) * 64] = a.warm[9 * NQ + qg];
+            pk[(kX + 10) * 64] = a.warm[10 * NQ + qg];
+            kind = 1;
+            bad_start = false;
+          } else {
+#pragma unroll
+            for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
+          }
+        }
       }
+      if (!__any(phase != kPhDone)) break;
     }
     // One turn: every live lane evaluates the material point once, at its start or at its
     // line-search trial x + alpha dx; a lane whose start or accepted trial this is then takes a
     // Newton step from it.  A trial's evaluation is thus also the point of the next iteration.
-    while (__any(phase != kPhDone)) {
-      // A step that asked for pivoting is taken in a turn of its own, in which the wave's other
-      // lanes wait: the choice of elimination is then the wave's, not the lane's.
-      const bool pivots = __builtin_amdgcn_readfirstlane(__any(phase == kPhAgain)) != 0;
-      const bool turn = pivots ? phase == kPhAgain : phase != kPhDone;
-      const bool moved = phase == kPhTrial || phase == kPhFull;
-      const double len = phase == kPhTrial ? alpha : (phase == kPhFull ? 1.0 : 0.0);
-      double xc[11], A[9];
+    // A step that asked for pivoting is taken in a turn of its own, in which the wave's other
+    // lanes wait: the choice of elimination is then the wave's, not the lane's, and the system's
+    // copy is one lane's, in LDS.
+    const uint64_t again = __ballot(phase == kPhAgain);
+    const bool pivots = again != 0;
+    const bool pivot_lane = pivots && lane == __builtin_ctzll(again);
+    const bool turn = pivots ? pivot_lane : phase != kPhDone;
+    const bool moved = phase == kPhTrial || phase == kPhFull;
+    const double len = phase == kPhTrial ? alpha : (phase == kPhFull ? 1.0 : 0.0);
+    double xc[11], A[9];
 #pragma unroll
-      for (int i = 0; i < 11; ++i) {
-        const double x = pk[(kX + i) * 64], xm = x + len * pk[(kDX + i) * 64];
-        xc[i] = moved ? xm : x;
-      }
+    for (int i = 0; i < 11; ++i) {
+      const double x = pk[(kX + i) * 64], xm = x + len * pk[(kDX + i) * 64];
+      xc[i] = moved ? xm : x;
+    }
 #pragma unroll
-      for (int i = 0; i < 9; ++i) A[i] = pk[(kA + i) * 64];
-      CPPoint p;
-      bool valid = cp_point<HE, FLOW>(cm, A, pk[kDet * 64], pk[kGn * 64], dt, xc, p);
-      valid = valid && !(phase == kPhStart && bad_start);
-      const double merit = cp_merit(p, pk[kGs * 64]);
-      const bool accept = turn && moved && valid && (phase == kPhFull || merit <= (1.0 - 1e-4 * alpha) * f0);
-      bool fail = turn && !valid && phase != kPhTrial;
-      if (turn && phase == kPhTrial && !accept) {
-        alpha *= 0.5;
-        if (++ls == 40) phase = kPhFull;  // no decrease found: the full step, if it is valid
-      }
-      if (accept) {
+    for (int i = 0; i < 9; ++i) A[i] = pk[(kA + i) * 64];
+    CPPoint p;
+    bool valid = cp_point<HE, FLOW>(cm, A, pk[kDet * 64], pk[kGn * 64], dt, xc, p);
+    valid = valid && !(phase == kPhStart && bad_start);
+    const double merit = cp_merit(p, pk[kGs * 64]);
+    const bool accept = turn && moved && valid && (phase == kPhFull || merit <= (1.0 - 1e-4 * alpha) * f0);
+    bool fail = turn && !valid && phase != kPhTrial;
+    if (turn && phase == kPhTrial && !accept) {
+      alpha *= 0.5;
+      if (++ls == 40) phase = kPhFull;  // no decrease found: the full step, if it is valid
+    }
+    if (accept) {
 #pragma unroll
-        for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = xc[i];
-      }
-      // the iteration that took this step may have been the last
-      fail = fail || (accept && it_att >= cm.maxit);
-      const bool step = turn && !fail && (accept || (!moved && valid));
-      if (phase == kPhStart ? turn : (accept && step)) {
-        ++it;
-        ++it_att;
-      }
-      if (__builtin_amdgcn_readfirstlane(__any(step))) {
-        // The point of this step (the start, or the accepted trial) is x in LDS.  The slip sums are
-        // the widest stretch, so the residual waits in dx's slots and the frames are formed again
-        // from A and x afterwards; e then takes those slots over the elimination.
-        double Ah[81], u[2][9], f;
-        const double lam = pk[(kX + 9) * 64], rhs_s = -p.R[9], rhs_t = -p.R[10];
-        if (step) {
-          f0 = merit;
+      for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = xc[i];
+    }
+    // the iteration that took this step may have been the last
+    fail = fail || (accept && it_att >= cm.maxit);
+    const bool step = turn && !fail && (accept || (!moved && valid));
+    if (phase == kPhStart ? turn : (accept && step)) {
+      ++it;
+      ++it_att;
+    }
+    if (__builtin_amdgcn_readfirstlane(__any(step))) {
+      // The point of this step (the start, or the accepted trial) is x in LDS.  The slip sums are
+      // the widest stretch, so the residual waits in dx's slots and the frames are formed again
+      // from A and x afterwards; e then takes those slots over the elimination.
+      double Ah[81], u[2][9], f;
+      const double lam = pk[(kX + 9) * 64], rhs_s = -p.R[9], rhs_t = -p.R[10];
+      if (step) {
+        f0 = merit;
 #pragma unroll
-          for (int i = 0; i < 9; ++i) pk[(kDX + i) * 64] = p.R[i];
+        for (int i = 0; i < 9; ++i) pk[(kDX + i) * 64] = p.R[i];
+      }
+      pin(p.S);
+      pin(p.sd);
+      LocalLin L;
+      end_stage();
+      cp_slip_sums<HE>(cm, p, p.sd, L);
+#pragma unroll
+      for (int r = 0; r < 9; ++r) pin(L.G[r]);
+      pin(L.eq);
+      end_stage();
+      pk = reload(sPk, lane);
+      {
+        double M[9], Mi[9], eF[9], AtE[9], T[9], E9[9], E9e[9], c[9], dM;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+          M[i] = pk[(kX + i) * 64];
+          A[i] = pk[(kA + i) * 64];
         }
-        pin(p.S);
-        pin(p.sd);
-        LocalLin L;
-        end_stage();
-        cp_slip_sums<HE>(cm, p, p.sd, L);
-#pragma unroll
-        for (int r = 0; r < 9; ++r) pin(L.G[r]);
-        pin(L.eq);
-        end_stage();
-        pk = reload(sPk, lane);
-        {
-          double M[9], Mi[9], eF[9], AtE[9], T[9], E9[9], E9e[9], c[9], dM;
-#pragma unroll
-          for (int i = 0; i < 9; ++i) {
-            M[i] = pk[(kX + i) * 64];
-            A[i] = pk[(kA + i) * 64];
-          }
-          inv_det(M, Mi, dM);
-          const double pJ = pk[kDet * 64] / dM, g = pk[(kX + 10) * 64], dl = dt * lam * pJ, mg = -1.0 / (cm.m * g);
-          mm3(A, M, eF);
-          mtm3(A, eF, AtE);
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-              const int r = i * 3 + j;
-              T[r] = Mi[j * 3 + i];
-              u[0][r] = pk[(kDX + r) * 64];
-              c[r] = mg * (u[0][r] - (M[r] - ((i == j) ? 1.0 : 0.0)) + dl * T[r]);  // N from the residual
-            }
-          cp_fold(cm, dt, g, pk[kGn * 64], p.gsum, p.gs, p.dgs, c, L);
-          f = L.f;
-          const double tf = rhs_t / f;
-          v6_to_9(L.eq, E9);
-          mm3(AtE, E9, E9e);
-#pragma unroll
-          for (int r = 0; r < 9; ++r) {
-            u[0][r] = -u[0][r] - c[r] * tf;
-            u[1][r] = -pJ * T[r];  // d
-          }
-          if (step) {
-#pragma unroll
-            for (int r = 0; r < 9; ++r) pk[(kDX + r) * 64] = L.es * E9e[r];
-          }
-          pin(u[0]);
-          pin(u[1]);
-#pragma unroll
-          for (int r = 0; r < 9; ++r) pin(L.G[r]);
-          end_stage();
-          cp_matrix(L, AtE, T, dl, Ah);
-        }
-        pin(Ah);
-        end_stage();
-        pk = reload(sPk, lane);
-        double system[9 * 11];
-        if (pivots) store_system<9, 2>(Ah, u, system);
-        bool solved = eliminate<9, 2>(Ah, u, kMaxMultStep);
-        if (pivots) {
-          solved = eliminate_pivot<9, 2>(system);
-#pragma unroll
-          for (int i = 0; i < 9; ++i) {
-            u[0][i] = system[i * 11 + 9];
-            u[1][i] = system[i * 11 + 10];
-          }
-        }
-        double M[9], Mi[9], dM, du = 0.0, dv = 0.0, ex = 0.0, dx[11];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) M[i] = pk[(kX + i) * 64];
         inv_det(M, Mi, dM);
-        const double pJ = pk[kDet * 64] / dM;
+        const double pJ = pk[kDet * 64] / dM, g = pk[(kX + 10) * 64], dl = dt * lam * pJ, mg = -1.0 / (cm.m * g);
+        mm3(A, M, eF);
+        mtm3(A, eF, AtE);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
-            const double d = -pJ * Mi[j * 3 + i];
-            du += d * u[0][i * 3 + j];
-            dv += d * u[1][i * 3 + j];
+            const int r = i * 3 + j;
+            T[r] = Mi[j * 3 + i];
+            u[0][r] = pk[(kDX + r) * 64];
+            c[r] = mg * (u[0][r] - (M[r] - ((i == j) ? 1.0 : 0.0)) + dl * T[r]);  // N from the residual
           }
-        const double yd = (du - rhs_s) / dv;  // dt times the step's multiplier of b
+        cp_fold(cm, dt, g, pk[kGn * 64], p.gsum, p.gs, p.dgs, c, L);
+        f = L.f;
+        const double tf = rhs_t / f;
+        v6_to_9(L.eq, E9);
+        mm3(AtE, E9, E9e);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+          u[0][r] = -u[0][r] - c[r] * tf;
+          u[1][r] = -pJ * T[r];  // d
+        }
+        if (step) {
+#pragma unroll
+          for (int r = 0; r < 9; ++r) pk[(kDX + r) * 64] = L.es * E9e[r];
+        }
+        pin(u[0]);
+        pin(u[1]);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) pin(L.G[r]);
+        end_stage();
+        cp_matrix(L, AtE, T, dl, Ah);
+      }
+      pin(Ah);
+      end_stage();
+      pk = reload(sPk, lane);
+      if (pivot_lane) store_system<9, 2>(Ah, u, sSystem);
+      bool solved = eliminate<9, 2>(Ah, u, kMaxMultStep);
+      if (pivot_lane) {
+        solved = eliminate_pivot<9, 2>(sSystem);
 #pragma unroll
         for (int i = 0; i < 9; ++i) {
-          dx[i] = u[0][i] - yd * u[1][i];
-          ex += pk[(kDX + i) * 64] * dx[i];
-        }
-        dx[9] = yd / dt - lam / pJ * rhs_s;
-        dx[10] = (rhs_t - ex) / f;
-        double size = 0.0;
-#pragma unroll
-        for (int i = 0; i < 9; ++i) size = fmax(size, fabs(dx[i]));
-        size = fmax(size, fabs(dx[9]) * dt);
-        size = fmax(size, fabs(dx[10]) / pk[kGn * 64]);
-        if (step) {
-          if (!solved) {
-            fail = pivots;  // singular
-            phase = kPhAgain;
-          } else if (size < cm.tol) {
-#pragma unroll
-            for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = pk[(kX + i) * 64] + dx[i];
-            phase = kPhDone;
-          } else {  // backtracking on half the squared residual norm, from the full step
-#pragma unroll
-            for (int i = 0; i < 11; ++i) pk[(kDX + i) * 64] = dx[i];
-            alpha = 1.0;
-            ls = 0;
-            phase = kPhTrial;
-          }
+          u[0][i] = sSystem[i * 11 + 9];
+          u[1][i] = sSystem[i * 11 + 10];
         }
       }
-      if (fail) {
-        if (kind == 1) {
-          // the warm start did not converge: fall back to the plain start with a fresh budget
-          // (iterations keep counting)
-          kind = 2;
-          it_att = 0;
-          const double *row = a.qpbuf + qrec(qg);
+      double M[9], Mi[9], dM, du = 0.0, dv = 0.0, ex = 0.0, dx[11];
 #pragma unroll
-          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
-          bad_start = (int(row[kStartFlag * kRecStride]) & 1) != 0;
-          phase = kPhStart;
-        } else {
-          failed = true;
+      for (int i = 0; i < 9; ++i) M[i] = pk[(kX + i) * 64];
+      inv_det(M, Mi, dM);
+      const double pJ = pk[kDet * 64] / dM;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const double d = -pJ * Mi[j * 3 + i];
+          du += d * u[0][i * 3 + j];
+          dv += d * u[1][i * 3 + j];
+        }
+      const double yd = (du - rhs_s) / dv;  // dt times the step's multiplier of b
+#pragma unroll
+      for (int i = 0; i < 9; ++i) {
+        dx[i] = u[0][i] - yd * u[1][i];
+        ex += pk[(kDX + i) * 64] * dx[i];
+      }
+      dx[9] = yd / dt - lam / pJ * rhs_s;
+      dx[10] = (rhs_t - ex) / f;
+      double size = 0.0;
+#pragma unroll
+      for (int i = 0; i < 9; ++i) size = fmax(size, fabs(dx[i]));
+      size = fmax(size, fabs(dx[9]) * dt);
+      size = fmax(size, fabs(dx[10]) / pk[kGn * 64]);
+      if (step) {
+        if (!solved) {
+          fail = pivots;  // singular
+          phase = kPhAgain;
+        } else if (size < cm.tol) {
+#pragma unroll
+          for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = pk[(kX + i) * 64] + dx[i];
           phase = kPhDone;
+        } else {  // backtracking on half the squared residual norm, from the full step
+#pragma unroll
+          for (int i = 0; i < 11; ++i) pk[(kDX + i) * 64] = dx[i];
+          alpha = 1.0;
+          ls = 0;
+          phase = kPhTrial;
         }
       }
     }
-    if (live) {
-      // read R and pF(n) again rather than keep them from the batch's start
-      int again = lane;
-      asm volatile("" : "+v"(again));
-      const int64_t q = q0 + again, qg = a.qp_base + q;
-      a.iters[qg] = it | (kind << 24);  // iterations, and the start in the high byte
-      if (failed) {
-        atomicAdd(a.err, 1);
+    if (fail) {
+      if (kind == 1) {
+        // the warm start did not converge: fall back to the plain start with a fresh budget
+        // (iterations keep counting)
+        kind = 2;
+        it_att = 0;
+        const double *row = a.qpbuf + qrec(a.qp_base + q);
+#pragma unroll
+        for (int i = 0; i < 11; ++i) pk[(kX + i) * 64] = row[i * kRecStride];
+        bad_start = (int(row[kStartFlag * kRecStride]) & 1) != 0;
+        phase = kPhStart;
       } else {
-        // pF(n+1) = M^-1 pF(n)
-        double x[11], Mc[9], Mi[9] = {}, pFn[9], pF1[9], det;
-#pragma unroll
-        for (int i = 0; i < 11; ++i) x[i] = pk[(kX + i) * 64];
-        rot_out_1(a.grains[a.qgrain[q]].R, x, Mc);
-        inv_det(Mc, Mi, det);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) pFn[i] = a.pF_n[i * NQ + qg];
-        mul_ab(Mi, pFn, pF1);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) a.pF_np1[i * NQ + qg] = pF1[i];
-        a.Sc_np1[qg] = x[10];
-        a.Sc_np1[NQ + qg] = x[9];
+        failed = true;
+        phase = kPhDone;
       }
     }
   }
@@ -1327,15 +1341,16 @@ __device__ __forceinline__ void store_moduli(const CPMaterial &cm, const PointFr
 // three-field element, Me, S, pJ and dMe/dF.
 enum : int { kOutPoint = 0, kOutModuli = 1, kOutMe = 2 };
 
-// The nine columns by the 9 x 9 system with pivoting.  A function of its own, so that the common
-// path keeps nothing in registers for it.
+// The nine columns by the 9 x 9 system with pivoting, for one lane at a time (the system is in
+// LDS).  A function of its own, so that the common path keeps nothing in registers for it.
 template <bool HE, int FLOW, int OUT>
 __device__ __attribute__((noinline)) void tangent_pivot(CPArgs a, int64_t t) {
   const CPMaterial cm = a.cpmats[0];
   double *out = a.qpbuf + qrec(a.qp_base + t);
   TangentPoint q;
   tangent_point<HE, FLOW>(a, cm, t, q);
-  double U[9], W[9], RpFi[9], system[9 * 19];
+  __shared__ double system[9 * 19];
+  double U[9], W[9], RpFi[9];
   tangent_frames(q, U, W, RpFi);
   {
     double Ah[81], AtE[9], Y[10][9];
@@ -1507,7 +1522,8 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
         for (int I = 0; I < 6; ++I) v[r] -= L.G[r][I] * Y[9][I];
     }
     if (!ok) {
-      tangent_pivot<HE, FLOW, OUT>(a, t);
+      for (uint64_t rest = __ballot(1); rest; rest &= rest - 1)
+        if (int(threadIdx.x) == __builtin_ctzll(rest)) tangent_pivot<HE, FLOW, OUT>(a, t);
       return;
     }
     double dv = 0.0;
@@ -2494,22 +2510,26 @@ void by_law(const CPArgs &a, F run) {
 void launch_cp_newton(const CPArgs &a, int64_t chunk, hipStream_t s) {
   const int64_t nq = a.nq;
   if (nq <= 0) return;
-  if (a.qnext) {
+  CPArgs b = a;
+  // Up to two batches per wave the queue has nothing to balance (380 us against 373 for a pass over
+  // 100,736 QPs); above, it keeps the waves filled (178,752 QPs, up to 25 iterations: 1000 -> 900).
+  if (nq <= 2 * 64 * kQueueWaves) b.qnext = nullptr;
+  if (b.qnext) {
     // one persistent wave per SIMD of the chip (the kernel holds all 512 registers of a lane),
     // draining the global queue; the counter is reset by a kernel, so a captured pass replays it
-    cp_queue_reset<<<1, 1, 0, s>>>(a.qnext);
+    cp_queue_reset<<<1, 1, 0, s>>>(b.qnext);
     chunk = 64;
   } else if (chunk < 64) {
     chunk = 64;
   }
-  const unsigned grid = a.qnext ? unsigned(std::min<int64_t>((nq + 63) / 64, kQueueWaves))
+  const unsigned grid = b.qnext ? unsigned(std::min<int64_t>((nq + 63) / 64, kQueueWaves))
                                 : unsigned((nq + chunk - 1) / chunk);
   const unsigned sgrid = unsigned((nq + 63) / 64);
   const auto run = [&](auto he, auto fl) {
     constexpr bool HE = decltype(he)::value;
     constexpr int FLOW = decltype(fl)::value;
     cp_start_kernel<HE, FLOW><<<sgrid, 64, 0, s>>>(a);
-    cp_newton<HE, FLOW><<<grid, 64, 0, s>>>(a, chunk);
+    cp_newton<HE, FLOW><<<grid, 64, 0, s>>>(b, chunk);
   };
   by_law(a, run);
 }

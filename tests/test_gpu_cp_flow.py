@@ -93,3 +93,26 @@ def test_three_field_initial_gradients(device, etype, n):
         assert np.abs(h3.get_state(fld) - ref).max() < 1e-15
     h3.close()
     h.close()
+
+
+def test_work_queue_gives_the_ranges_results(device):
+    """146,334 points, enough for the local Newton's global queue: which wave and lane solves a point,
+    and beside which others, leaves no trace in its state."""
+    prob = CPBoxProblem(29, P.PGF_TET4, P.fcc_crystal(), n_grains=3, seed=5)
+    out = []
+    for chunk in (1, 64, 192):
+        h = P.Handle(prob.mesh, prob.ids, prob.ndof, prob.Ap, prob.Ai, prob.mats)
+        h.set_orientations(prob.R, prob.grain)
+        h.set_tuning(cp_chunk=chunk)
+        f = torch.empty(prob.ndof, dtype=torch.float64, device=device)
+        for s in (1, 2):
+            r, defl = prob.displacement(6e-4 * s, 2e-5, seed=s)
+            rd, dd = (torch.from_numpy(np.ascontiguousarray(x)).to(device) for x in (r, defl))
+            assert h.residual(f, rd, defl=dd, dt=1.0) == 0
+            h.commit_step()
+        out.append([h.get_state(k) for k in (P.STATE_PLASTIC_N, P.STATE_SCALAR_N, P.STATE_ITERS)])
+        h.close()
+    assert out[0][2].max() > 3
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            assert np.array_equal(a, b)
