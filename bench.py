@@ -64,19 +64,18 @@ def cp_flops_per_qp(mean_iters, nne=4):
     """FP64 operations per QP of the crystal-plasticity pass, counted from the kernels (FMA = 2,
     divide, pow and cbrt as one each; the flow rule's |tau/g|^19 is eight multiplies of binary
     powering, counted as one, which the ~1e4 totals absorb):
-      material-point evaluation (cp_point) ~1.4e3: eF, C_e, S = L:E, Mandel stress, 12 tau_a,
-        12 power-law rates, R_M;
-      Jacobian ~6.2e3: 12 x (d tau_a/dM 260 + rank-1 update of the 9x9 block 162 + borders
-        36), lambda terms 400, Schur complement 162;
-      9x9 LU 500 and two solves 324;
-      => Newton iteration ~8.4e3 (one evaluation: a line-search trial's evaluation is the next
+      material-point evaluation (cp_point, in the crystal frame) ~4.5e2: eF, C_e, S, Mandel stress,
+        12 tau_a, 12 power-law rates, R_M;
+      Jacobian ~1.4e3: 12 x 60 slip-system sums, the 9x9 block 7e2;
+      9x9 elimination with two right-hand sides 8e2, line search and border 3e2;
+      => Newton iteration ~3.0e3 (one evaluation: a line-search trial's evaluation is the next
       iteration's point);
-      start ~3.5e3 (up to 10 tau-ratio evaluations of ~350);
-      tangent pass ~1.2e4 (evaluation, Jacobian, LU, nine bordered solves, d tau/dF);
-      element rows: nine row-basis vectors per QP x ~650 (B, Y = L:B, Z, z = Z:D, W, Fr W),
-        then 3*nne rows x 2 (50 + 9 nne) (S g_a, residual, the three-basis combination, the
-        geometric term and the row of K)."""
-    return 8.4e3 * mean_iters + 3.5e3 + 1.2e4 + 9 * 650 + 3 * nne * 2 * (50 + 9 * nne)
+      start ~2.0e3 (up to 10 tau-ratio evaluations of ~200);
+      tangent pass ~7.3e3 (evaluation, slip sums, the 6x6 system and its ten right-hand sides, nine
+      columns of moduli x 460);
+      element rows: 3*nne rows x 2 (30 + 9 nne) (the gradient's combination of the moduli, the
+        residual, the row of K)."""
+    return 3.0e3 * mean_iters + 2.0e3 + 7.3e3 + 3 * nne * 2 * (30 + 9 * nne)
 
 
 def measured_traffic(key):
