@@ -200,6 +200,7 @@ struct pgf_handle_s {
   int32_t *d_err = nullptr;        // failure counter of the pass, zero between passes
   int32_t *err_host = nullptr;     // pinned: where a pass leaves its count (-1 until then)
   bool err_dirty = true;           // d_err may hold something else (new, or an aborted pass)
+  hipStream_t pass_stream = nullptr;  // the stream that the last pass was launched on
   double *d_red = nullptr;  // one scalar of a device reduction (pgf_subdivision_param)
   // crystal plasticity
   bool has_cp = false;
@@ -616,11 +617,26 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
   return launches;
 }
 
-// Before a pass is launched.
-void begin_pass(pgf_handle h) {
-  if (h->err_dirty) pgf::launch_fill_i32(h->d_err, 1, 0, h->stream);
+// Wait for whatever the handle has launched.  The last pass may have been launched on a stream that
+// pgf_set_stream has replaced since, and that its owner may have destroyed: then on the device.
+int finish_work(pgf_handle h) {
+  const bool moved = h->pass_stream && h->pass_stream != h->stream;
+  if ((moved ? hipDeviceSynchronize() : hipStreamSynchronize(h->stream)) != hipSuccess) return PGF_EHIP;
+  h->pass_stream = nullptr;
+  return PGF_OK;
+}
+
+// Before a pass is launched.  A pass that was given up after its launches were queued has its count
+// still to come, which end_pass could not tell from the new pass's own: it is waited for first.
+int begin_pass(pgf_handle h) {
+  if (h->err_dirty) {
+    if (int rc = finish_work(h)) return rc;
+    pgf::launch_fill_i32(h->d_err, 1, 0, h->stream);
+  }
   h->err_dirty = true;
+  h->pass_stream = h->stream;
   *static_cast<volatile int32_t *>(h->err_host) = -1;
+  return PGF_OK;
 }
 
 // Wait for the pass and return its failure count.  Its last kernel runs when all of its results
@@ -688,7 +704,7 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
     }
     h->gkey = key;
   }
-  begin_pass(h);
+  if (int rc = begin_pass(h)) return rc;
   if (h->profiling) hipEventRecord(h->ev0, h->stream);
   if (graph) {
     if (hipGraphLaunch(h->gexec, h->stream) != hipSuccess) return PGF_EHIP;
@@ -1316,7 +1332,7 @@ int pgf_residual_tangent_static(pgf_handle h, const pgf_nodal_input *in, double 
   if (dt > 0.0) h->dt = dt;
   // eager launches only: instantiating a graph may allocate.  Every staging block the pass
   // reads is written earlier in the same pass, so what an earlier call left is never read.
-  begin_pass(h);
+  if (int rc = begin_pass(h)) return rc;
   if (h->profiling) hipEventRecord(h->ev0, h->stream);
   h->last_launches = enqueue_pass(h, in, pgf::MODE_INTEGRATE | pgf::MODE_RESIDUAL | pgf::MODE_TANGENT, f, vals,
                                   h->stage_size ? stage : nullptr);
