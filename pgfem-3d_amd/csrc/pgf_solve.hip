@@ -11,6 +11,9 @@
 //   step_s    alpha; r <- s = r - alpha v, sh = D s
 //   spmv T    t = A sh                        partials t.t, t.s
 //   step_x    omega; x += alpha ph + omega sh, r <- s - omega t   partials rh.r, r.r
+// A launch reads no scalar that it writes.  The stop is kept as the number of the launch that decided
+// it, and only later launches return for it: the deciding launch's blocks, which may see the word
+// written or not, all reach the decision by themselves.
 // The host enqueues a few iterations at a time and looks, one batch behind, at a status word in
 // pinned memory; once the stop is decided, the launches already enqueued return at their first
 // load.
@@ -18,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 
 #include "pgf_device.h"
 
@@ -39,8 +43,16 @@ inline int dot_blocks(int64_t n) { return int(std::min<int64_t>(kMaxPart, (n + k
 
 struct Scalars {
   double rho[2], alpha, omega, bnorm, res;
-  int32_t done, stop_after;
+  int64_t stop;  // the launch that decided the stop, kRunning before
+  int32_t stop_after;
 };
+constexpr int64_t kRunning = INT64_MAX;
+// launches are numbered over the solve, five an iteration in the order above
+__host__ __device__ constexpr int64_t launch_number(int it, int k) { return 5 * int64_t(it) + k; }
+// an earlier launch has decided the stop
+__device__ __forceinline__ bool stopped(const Scalars *sc, int64_t launch) {
+  return __hip_atomic_load(&sc->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < launch;
+}
 
 template <int ROR>
 __device__ __forceinline__ double row_rotate(double v) {  // lane i of a DPP row reads lane i - ROR mod 16
@@ -101,6 +113,7 @@ struct SpmvArgs {
   double *r, *rh, *p, *v, *dinv;  // kInit
   double *pa, *pb;           // partials
   const Scalars *sc;
+  int64_t launch;
 };
 
 __device__ __forceinline__ double pick3(int b, double v0, double v1, double v2) {
@@ -116,7 +129,7 @@ __device__ __forceinline__ double pick3(int b, double v0, double v1, double v2) 
 // entries of x (13 us at 1.46 million entries, 75 workgroups).
 template <int MODE>
 __global__ __launch_bounds__(kSpmvBlock) void spmv(SpmvArgs g) {
-  if (MODE != kInit && g.sc->done) return;
+  if (MODE != kInit && stopped(g.sc, g.launch)) return;
   const int lane = threadIdx.x % kLanes;
   for (int rg = blockIdx.x; rg < g.rows.n_ranges; rg += gridDim.x) {
     const int hi = g.rows.range[rg + 1];
@@ -212,10 +225,11 @@ struct StepArgs {
   SolveStatus *status;    // pinned host memory
   double tol;
   int it, maxit;
+  int64_t launch;
 };
 
 __device__ __forceinline__ void finish(const StepArgs &g, int it, double res) {
-  g.sc->done = 1;
+  __hip_atomic_store(&g.sc->stop, g.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   g.status->it = it;
   g.status->res = res;
   __threadfence_system();
@@ -224,7 +238,7 @@ __device__ __forceinline__ void finish(const StepArgs &g, int it, double res) {
 
 // Iteration g.it: the state after iteration g.it - 1 decides whether it runs.
 __global__ __launch_bounds__(kBlock) void step_p(StepArgs g) {
-  if (g.sc->done) return;
+  if (stopped(g.sc, g.launch)) return;
   const bool first = g.it == 1, lead = blockIdx.x == 0 && threadIdx.x == 0;
   double a, b;
   close_dots(g.pa, g.pb, g.m, a, b);  // first: b.b and r.r (= rh.r); later: rh.r and r.r
@@ -249,7 +263,7 @@ __global__ __launch_bounds__(kBlock) void step_p(StepArgs g) {
     return;
   }
   if (lead) {
-    g.sc->bnorm = bnorm;
+    if (first) g.sc->bnorm = bnorm;
     g.sc->res = res;
     g.sc->rho[g.it & 1] = a;
   }
@@ -262,7 +276,7 @@ __global__ __launch_bounds__(kBlock) void step_p(StepArgs g) {
 }
 
 __global__ __launch_bounds__(kBlock) void step_s(StepArgs g) {
-  if (g.sc->done) return;
+  if (stopped(g.sc, g.launch)) return;
   double rv, unused;
   close_dots(g.pa, g.pa, g.m, rv, unused);
   if (rv == 0.0 || !isfinite(rv)) {
@@ -279,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void step_s(StepArgs g) {
 }
 
 __global__ __launch_bounds__(kBlock) void step_x(StepArgs g) {
-  if (g.sc->done) return;
+  if (stopped(g.sc, g.launch)) return;
   double tt, ts;
   close_dots(g.pa, g.pb, g.m, tt, ts);
   const double omega = tt > 0.0 ? ts / tt : 0.0, alpha = g.sc->alpha;
@@ -302,7 +316,10 @@ __global__ __launch_bounds__(kBlock) void step_x(StepArgs g) {
   }
 }
 
-__global__ void clear_scalars(Scalars *sc) { sc->done = sc->stop_after = 0; }
+__global__ void clear_scalars(Scalars *sc) {
+  sc->stop = kRunning;
+  sc->stop_after = 0;
+}
 
 }  // namespace
 
@@ -323,8 +340,8 @@ int bicgstab(hipStream_t s, const RowGroups &rows, const int32_t *Ai, const doub
   status->it = 0;
   status->res = std::nan("");
   const unsigned nb = unsigned(dot_blocks(n));
-  SpmvArgs m{rows, n, Ai, vals, x, nullptr, b, r, rh, p, v, dinv, p_bb, p_rr, sc};
-  StepArgs e{n, dinv, r, rh, p, v, ph, sh, t, x, p_bb, p_rr, int(nb), p_rho, p_rr, sc, status, tol, 0, maxit};
+  SpmvArgs m{rows, n, Ai, vals, x, nullptr, b, r, rh, p, v, dinv, p_bb, p_rr, sc, 0};
+  StepArgs e{n, dinv, r, rh, p, v, ph, sh, t, x, p_bb, p_rr, int(nb), p_rho, p_rr, sc, status, tol, 0, maxit, 0};
   clear_scalars<<<1, 1, 0, s>>>(sc);
   spmv<kInit><<<nb, kSpmvBlock, 0, s>>>(m);
   hipError_t err = hipSuccess;
@@ -337,6 +354,7 @@ int bicgstab(hipStream_t s, const RowGroups &rows, const int32_t *Ai, const doub
     bool last = false;
     for (int k = 0; k < kBatch && !last; ++k, ++it) {
       e.it = it;
+      e.launch = launch_number(it, 0);
       e.pa = it == 1 ? p_bb : p_rho;
       e.pb = p_rr;
       step_p<<<nb, kBlock, 0, s>>>(e);
@@ -346,17 +364,21 @@ int bicgstab(hipStream_t s, const RowGroups &rows, const int32_t *Ai, const doub
       m.y = v;
       m.w = rh;
       m.pa = p_rv;
+      m.launch = launch_number(it, 1);
       spmv<kV><<<nb, kSpmvBlock, 0, s>>>(m);
       e.pa = p_rv;
+      e.launch = launch_number(it, 2);
       step_s<<<nb, kBlock, 0, s>>>(e);
       m.x = sh;
       m.y = t;
       m.w = r;
       m.pa = p_tt;
       m.pb = p_ts;
+      m.launch = launch_number(it, 3);
       spmv<kT><<<nb, kSpmvBlock, 0, s>>>(m);
       e.pa = p_tt;
       e.pb = p_ts;
+      e.launch = launch_number(it, 4);
       step_x<<<nb, kBlock, 0, s>>>(e);
     }
     if (!chk(hipGetLastError()) || !chk(hipEventRecord(ev[batch & 1], s))) break;
