@@ -200,7 +200,8 @@ struct pgf_handle_s {
   int32_t *d_err = nullptr;        // failure counter of the pass, zero between passes
   int32_t *err_host = nullptr;     // pinned: where a pass leaves its count (-1 until then)
   bool err_dirty = true;           // d_err may hold something else (new, or an aborted pass)
-  hipStream_t pass_stream = nullptr;  // the stream that the last pass was launched on
+  hipStream_t pass_stream = nullptr;    // the stream that the last pass was launched on
+  hipStream_t replay_stream = nullptr;  // and the last replay of a captured one
   double *d_red = nullptr;  // one scalar of a device reduction (pgf_subdivision_param)
   // crystal plasticity
   bool has_cp = false;
@@ -617,12 +618,14 @@ int32_t enqueue_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *
   return launches;
 }
 
-// Wait for whatever the handle has launched.  The last pass may have been launched on a stream that
-// pgf_set_stream has replaced since, and that its owner may have destroyed: then on the device.
+// Wait for whatever the handle has launched.  The last pass or replay may have been launched on a
+// stream that pgf_set_stream has replaced since, and that its owner may have destroyed: then on the
+// device.
 int finish_work(pgf_handle h) {
-  const bool moved = h->pass_stream && h->pass_stream != h->stream;
+  const bool moved = (h->pass_stream && h->pass_stream != h->stream) ||
+                     (h->replay_stream && h->replay_stream != h->stream);
   if ((moved ? hipDeviceSynchronize() : hipStreamSynchronize(h->stream)) != hipSuccess) return PGF_EHIP;
-  h->pass_stream = nullptr;
+  h->pass_stream = h->replay_stream = nullptr;
   return PGF_OK;
 }
 
@@ -662,10 +665,11 @@ int end_pass(pgf_handle h) {
   return *count;
 }
 
-// Finish the handle's work and forget its captured pass: for setters that free or replace a
-// buffer whose address the graph's kernels hold.
+// Finish the handle's work and forget its captured pass (its last kernel may still be retiring when
+// a replay has returned): before a new capture, and for setters that free or replace a buffer whose
+// address the graph's kernels hold.
 int drop_graph(pgf_handle h) {
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
+  if (int rc = finish_work(h)) return rc;
   if (h->gexec) {
     hipGraphExecDestroy(h->gexec);
     h->gexec = nullptr;
@@ -686,12 +690,8 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
   GraphKey key{mode, in->r, in->d_r, in->defl, in->defl_d, f, vals, h->warm, h->dt, h->cp_chunk, h->gather_waves,
                h->gather_batch};
   if (graph && !(h->gexec && key == h->gkey)) {
-    if (h->gexec) {
-      // its last kernel may still be retiring (end_pass)
-      if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
-      hipGraphExecDestroy(h->gexec);
-      h->gexec = nullptr;
-    }
+    if (h->gexec)
+      if (int rc = drop_graph(h)) return rc;
     hipGraph_t g = nullptr;
     if (hipStreamBeginCapture(h->stream, hipStreamCaptureModeRelaxed) != hipSuccess) return PGF_EHIP;
     h->glaunches = enqueue_pass(h, in, mode, f, vals, pass_stage(h));
@@ -707,6 +707,7 @@ int run_pass(pgf_handle h, const pgf_nodal_input *in, int mode, double *f, doubl
   if (int rc = begin_pass(h)) return rc;
   if (h->profiling) hipEventRecord(h->ev0, h->stream);
   if (graph) {
+    h->replay_stream = h->stream;
     if (hipGraphLaunch(h->gexec, h->stream) != hipSuccess) return PGF_EHIP;
     h->last_launches = h->glaunches;
   } else {
@@ -1190,7 +1191,7 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
 
 int pgf_destroy(pgf_handle h) {
   if (!h) return PGF_OK;
-  if (h->stream) hipStreamSynchronize(h->stream);
+  if (h->stream) finish_work(h);
   hipFree(h->d_X);
   hipFree(h->d_dofid);
   hipFree(h->d_row_start);
@@ -1883,22 +1884,14 @@ int pgf_solve(pgf_handle h, const double *vals, const double *b, double *x, doub
 int pgf_set_graph(pgf_handle h, int on) {
   if (!h) return PGF_EINVAL;
   h->use_graph = on != 0;
-  if (!h->use_graph && h->gexec) {
-    hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-  }
-  return PGF_OK;
+  return !h->use_graph && h->gexec ? drop_graph(h) : PGF_OK;
 }
 
 int pgf_set_assembly(pgf_handle h, int32_t mode) {
   if (!h || (mode != PGF_ASSEMBLY_GATHER && mode != PGF_ASSEMBLY_COLOURED)) return PGF_EINVAL;
   if (mode == PGF_ASSEMBLY_GATHER && (pgf::gather_waves(h->maxlen) < 1 || !h->gather_fits)) return PGF_ENOTSUP;
   if (mode == h->assembly) return PGF_OK;
-  if (hipStreamSynchronize(h->stream) != hipSuccess) return PGF_EHIP;
-  if (h->gexec) {  // a captured pass holds the old schedule
-    hipGraphExecDestroy(h->gexec);
-    h->gexec = nullptr;
-  }
+  if (int rc = drop_graph(h)) return rc;  // a captured pass holds the old schedule
   if (mode == PGF_ASSEMBLY_COLOURED && h->d_stage) {  // release the staging memory
     hipFree(h->d_stage);
     h->d_stage = nullptr;

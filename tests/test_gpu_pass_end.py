@@ -45,3 +45,33 @@ def test_pass_after_one_given_up(device, mode):
         assert torch.equal(a, b)
     assert call(*lost, bad, defl=defl) > 0
     h.close()
+
+
+def test_captured_pass_dropped_after_a_change_of_stream(device):
+    """Passes replayed on one stream, the graph then dropped or captured anew from another."""
+    prob, h, good, _, defl = _problem(device)
+    ref, out = (_vectors(h, prob, device) for _ in range(2))
+    assert h.residual_tangent(*ref, good, defl=defl) == 0
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for k in range(6):
+        h.set_stream(streams[k % 2].cuda_stream)
+        h.set_graph(True)
+        for x in out:
+            x.fill_(np.nan)
+        torch.cuda.synchronize()
+        for _ in range(3):
+            assert h.residual_tangent(*out, good, defl=defl) == 0
+            for a, b in zip(out, ref):
+                assert torch.equal(a, b)
+        h.set_stream(streams[(k + 1) % 2].cuda_stream)
+        if k % 3 == 0:
+            h.set_graph(False)
+        elif k % 3 == 1:
+            h.set_assembly(P.ASSEMBLY_COLOURED)
+            h.set_assembly(P.ASSEMBLY_GATHER)
+        else:
+            other = _vectors(h, prob, device)
+            assert h.residual_tangent(*other, good, defl=defl) == 0
+            assert torch.equal(other[1], ref[1])
+    h.set_stream(streams[0].cuda_stream)
+    h.close()
