@@ -297,8 +297,8 @@ int gather_waves(int32_t maxlen);
 // waves: nodes per workgroup (capped by the LDS each node needs); batch: staging blocks each
 // half-wave keeps in flight (2, 4 or 8)
 void launch_gather(int mode, const GatherArgs &g, int waves, int batch, hipStream_t s);
-// The CSR rows in groups of up to three with the same columns (a node's free DOFs), cut at
-// multiples of 256 rows: group g is rows [x, x + y) from entry z on, w columns each; rows
+// The CSR rows in groups of up to three (a node's free DOFs, where their columns are the same, which
+// pgf_create looks at), cut at multiples of 256 rows: group g is rows [x, x + y) from entry z on, w columns each; rows
 // [256 k, 256 (k + 1)) are groups [range[k], range[k + 1]).
 struct RowGroups {
   const int4 *groups;
