@@ -164,8 +164,9 @@ int pgf_get_sizes(pgf_handle h, int64_t *n_qp, int64_t *nnz, int64_t *ndof,
  * [n_grains*9], host) and the grain of every element ([n_elem], host).  Replaces
  * plasticity_model_set_orientations / plasticity_model_construct_rotation
  * (src/plasticity_model.cc:1226-1258,1455), which store R per QP (TENSOR_R); here R is stored
- * per grain and slip systems and stiffness are rotated once per grain.  Without this call
- * every element uses the crystal frame. */
+ * per grain, and the local solve rotates a point's state into the crystal frame.  A matrix that
+ * is not orthonormal (rounded, scaled, or improper) stands for the nearest rotation.  Without
+ * this call every element uses the crystal frame. */
 int pgf_set_orientations(pgf_handle h, int32_t n_grains, const double *R, const int32_t *elem_grain);
 
 /* Interface element properties: n_props records and the property index of every interface

@@ -106,6 +106,39 @@ void rot_to_quat(const double *R, float *q) {
   q[3] = float(sg * z);
 }
 
+// The rotation nearest to R (its orthogonal polar factor by Newton's iteration, and -R for an improper
+// one, whose slip systems are the same).  The kernels rotate by R^T and back by R, so what R lacks to
+// R^T R = I, 1e-7 in single precision, would come into the elastic strain.  An R that is orthonormal to
+// rounding is kept as it is; so is one without an inverse.
+void nearest_rotation(const double *R, double *Q) {
+  std::copy(R, R + 9, Q);
+  double det = 1.0, step = 1.0;
+  for (int it = 0; it < 100 && step > 1.0e-15; ++it) {
+    double C[9], N[9];  // cofactors: Q^-T = C / det
+    for (int i = 0; i < 3; ++i)
+      for (int j = 0; j < 3; ++j) {
+        const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+        C[i * 3 + j] = Q[i1 * 3 + j1] * Q[i2 * 3 + j2] - Q[i1 * 3 + j2] * Q[i2 * 3 + j1];
+      }
+    det = Q[0] * C[0] + Q[1] * C[1] + Q[2] * C[2];
+    step = 0.0;
+    bool finite = true;
+    for (int i = 0; i < 9; ++i) {
+      const double d = 0.5 * (C[i] / det - Q[i]);
+      N[i] = Q[i] + d;
+      step = std::max(step, std::fabs(d));
+      finite = finite && std::isfinite(N[i]);
+    }
+    if (!finite) {
+      std::copy(R, R + 9, Q);
+      return;
+    }
+    if (step > 1.0e-15) std::copy(N, N + 9, Q);
+  }
+  if (det < 0.0)
+    for (int i = 0; i < 9; ++i) Q[i] = -Q[i];
+}
+
 // Host tables of one grain: the 12 FCC {111}<110> systems (unit slip direction s and plane
 // normal m, Schmid tensor s (x) m) rotated by R (crystal -> sample frame).
 void make_grain(const double *R, DevGrain &g) {
@@ -1758,8 +1791,10 @@ int pgf_set_orientations(pgf_handle h, int32_t n_grains, const double *R, const 
   std::vector<pgf::DevGrain> g(n_grains);
   std::vector<float> q(size_t(n_grains) * 4);
   for (int32_t k = 0; k < n_grains; ++k) {
-    pgf::make_grain(R + 9 * k, g[k]);
-    pgf::rot_to_quat(R + 9 * k, q.data() + 4 * k);
+    double Q[9];
+    pgf::nearest_rotation(R + 9 * k, Q);
+    pgf::make_grain(Q, g[k]);
+    pgf::rot_to_quat(Q, q.data() + 4 * k);
   }
   std::vector<std::vector<int32_t>> egs(h->blocks.size()), qgs(h->blocks.size());
   if (elem_grain)
