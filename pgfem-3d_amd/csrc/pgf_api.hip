@@ -253,6 +253,7 @@ struct pgf_handle_s {
   // 64 and 1; on 998,250 QPs 774, 769, 755, 735.
   int64_t cp_chunk = 1;
   unsigned long long *d_qnext = nullptr;  // the global queue's counter
+  unsigned long long *d_pivots = nullptr;  // [cp_nq / 64], zero between passes (pgf::CPArgs::pivots)
   int32_t gather_waves = 4;  // nodes per gather workgroup (autotuned; capped by LDS)
   int32_t gather_batch = 4;  // staging blocks each gather half-wave keeps in flight (autotuned)
   int32_t *d_qgrain_all = nullptr;  // [n_qp] grain of every device QP
@@ -357,6 +358,7 @@ pgf::CPArgs cp_args(pgf_handle h, const Block &b, const pgf_nodal_input *in) {
   c.gdot = h->d_gdot[0];
   c.iters = h->d_iters;
   c.qnext = h->cp_chunk == 1 ? h->d_qnext : nullptr;
+  c.pivots = h->d_pivots;
   c.warm = h->warm;
   c.qpbuf = h->d_qpbuf;  // indexed by device QP (pgf::qrec)
   c.err = h->d_err;
@@ -1205,6 +1207,9 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     }
     if ((rc = pgf::dalloc(&h->d_iters, size_t(h->n_qp)))) return fail(rc);
     if ((rc = pgf::dalloc(&h->d_qnext, 1))) return fail(rc);
+    const size_t n_masks = size_t((h->cp_nq + 63) / 64);
+    if ((rc = pgf::dalloc(&h->d_pivots, n_masks))) return fail(rc);
+    if (hipMemset(h->d_pivots, 0, n_masks * sizeof(*h->d_pivots)) != hipSuccess) return fail(PGF_EHIP);
     if ((rc = pgf::dalloc(&h->d_qpbuf, size_t((h->n_qp + pgf::kRecStride - 1) / pgf::kRecStride) *
                                              pgf::kCPBuf * pgf::kRecStride)))
       return fail(rc);
@@ -1283,6 +1288,7 @@ int pgf_destroy(pgf_handle h) {
   }
   hipFree(h->d_iters);
   hipFree(h->d_qnext);
+  hipFree(h->d_pivots);
   hipFree(h->d_qpbuf);
   for (int t = 0; t < 3; ++t) {
     hipFree(h->d_F[t]);

@@ -29,6 +29,7 @@
 //   cp_tangent     at the converged state: tau, gdot, and per point the stress and the moduli that
 //                  the element kernel contracts (qpbuf); for the three-field element Me, S, pJ
 //                  and dMe/dF (Me = pF(n+1)^-1)
+//   cp_tangent_pivot  the same for the points whose system needs pivoting
 //   cp_elem        element rows: the reference contraction (compute_stiffness_matrix,
 //                  src/constitutive_model.cc:1520-1616) is linear in the two gradients, so it is
 //                  f_ab = sum_j T_bj dN_a,j, K_ab,wg = sum_jl dN_a,j A[b j][g l] dN_w,l with the
@@ -654,6 +655,64 @@ __device__ __forceinline__ bool eliminate_pivot(double *a) {
   return ok;
 }
 
+// The same with partial pivoting, as factors and solutions: every lane that needs it takes part, its
+// rows exchanged by selects, so that no index is known at run time only.  False for a singular matrix.
+template <int N>
+__device__ __forceinline__ bool factor_pivot(double (&A)[N * N], int (&piv)[N]) {
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    int p = k;
+    double amax = fabs(A[k * N + k]);
+#pragma unroll
+    for (int i = k + 1; i < N; ++i) {
+      const double v = fabs(A[i * N + k]);
+      p = v > amax ? i : p;
+      amax = v > amax ? v : amax;
+    }
+    ok = ok && amax > 0.0;
+    piv[k] = p;
+#pragma unroll
+    for (int i = k + 1; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const double x = A[k * N + j], y = A[i * N + j];
+        A[k * N + j] = p == i ? y : x;
+        A[i * N + j] = p == i ? x : y;
+      }
+    const double r = 1.0 / A[k * N + k];
+    A[k * N + k] = r;
+#pragma unroll
+    for (int i = k + 1; i < N; ++i) {
+      A[i * N + k] *= r;
+#pragma unroll
+      for (int j = k + 1; j < N; ++j) A[i * N + j] -= A[i * N + k] * A[k * N + j];
+    }
+  }
+  return ok;
+}
+template <int N>
+__device__ __forceinline__ void solve_pivot(const double (&A)[N * N], const int (&piv)[N], double (&b)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int i = k + 1; i < N; ++i) {
+      const double x = b[k], y = b[i];
+      b[k] = piv[k] == i ? y : x;
+      b[i] = piv[k] == i ? x : y;
+    }
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int i = k + 1; i < N; ++i) b[i] -= A[i * N + k] * b[k];
+#pragma unroll
+  for (int i = N - 1; i >= 0; --i) {
+#pragma unroll
+    for (int j = i + 1; j < N; ++j) b[i] -= A[i * N + j] * b[j];
+    b[i] *= A[i * N + i];
+  }
+}
+
 __device__ __forceinline__ double cp_merit(const CPPoint &p, double gscale) {
   double r = 0.0;
 #pragma unroll
@@ -1161,9 +1220,10 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
 // a 6 x 6 system serves the nine columns and the border's b, with no sum over slip systems and
 // no 9 x 9 factor.  lp is of the order of the squared strain increment (1e-7 at 1e-3), so H
 // comes by the series in lp, to the last bit.  A point where lp is not small, or where the
-// 6 x 6 elimination meets a multiplier above kMaxMultTangent, takes the 9 x 9 system with
-// pivoting.  998,250 QPs in 571 us, of them 130 for the moduli, instead of the 1066 us of the
-// sample-frame kernel with its pivoted 9 x 9 and without the moduli (25 instead of 61 us for 10,368).
+// 6 x 6 elimination meets a multiplier above kMaxMultTangent, is left to cp_tangent_pivot, which takes
+// the 9 x 9 system with pivoting.  998,250 QPs in 575 us, of them 130 for the moduli, instead of the
+// 1066 us of the sample-frame kernel with its pivoted 9 x 9 and without the moduli (25 instead of 61
+// us for 10,368).
 // Bound by FP64 issue and latency at one wave per SIMD: G, the columns and the frames are 512
 // registers.  The columns run in a rolled loop with what is indexed by the column in LDS.
 constexpr double kMaxLp = 0.01;
@@ -1341,81 +1401,54 @@ __device__ __forceinline__ void store_moduli(const CPMaterial &cm, const PointFr
 // three-field element, Me, S, pJ and dMe/dF.
 enum : int { kOutPoint = 0, kOutModuli = 1, kOutMe = 2 };
 
-// The nine columns by the 9 x 9 system with pivoting, for one lane at a time (the system is in
-// LDS).  A function of its own, so that the common path keeps nothing in registers for it.
+// The lanes' LDS of the tangent kernel, field i of a lane at [i * 64]: the columns' kappa -- then their
+// solutions -- and the U, W of the moduli, by a run-time column.  36 KB per wave.
+constexpr int kColY = 0, kColU = 54, kColW = 63;
 template <bool HE, int FLOW, int OUT>
-__device__ __attribute__((noinline)) void tangent_pivot(CPArgs a, int64_t t) {
-  const CPMaterial cm = a.cpmats[0];
-  double *out = a.qpbuf + qrec(a.qp_base + t);
-  TangentPoint q;
-  tangent_point<HE, FLOW>(a, cm, t, q);
-  __shared__ double system[9 * 19];
-  double U[9], W[9], RpFi[9];
-  tangent_frames(q, U, W, RpFi);
-  {
-    double Ah[81], AtE[9], Y[10][9];
-    LocalLin L;
-    tangent_lin<HE>(cm, a.dt, q, AtE, L);
-    cp_matrix(L, AtE, q.p.T, a.dt * q.x[9] * q.p.pJ, Ah);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) {
-      double kp[6];
-      kappa(U + (c / 3) * 3, W + (c % 3) * 3, kp);
-#pragma unroll
-      for (int r = 0; r < 9; ++r) {
-        double s = 0.0;
-#pragma unroll
-        for (int I = 0; I < 6; ++I) s -= L.G[r][I] * kp[I];
-        Y[c][r] = s;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 9; ++r) Y[9][r] = q.p.T[r];
-    store_system<9, 10>(Ah, Y, system);
-  }
-  if (!eliminate_pivot<9, 10>(system)) {
-    atomicAdd(a.err, 1);
-    return;
-  }
-  PointFrame<HE> f;
-  // (T may take the place of Fr in the record: stored last)
-  double T[9];
-  if constexpr (OUT == kOutModuli) point_frame<HE>(a, cm, t, q, true, f, T);
-  double dv = 0.0;
-#pragma unroll
-  for (int r = 0; r < 9; ++r) dv += q.p.T[r] * system[r * 19 + 18];
-#pragma unroll 1
-  for (int c = 0; c < 9; ++c) {
-    double du = 0.0, dM[9];
-#pragma unroll
-    for (int r = 0; r < 9; ++r) du += q.p.T[r] * system[r * 19 + 9 + c];
-    du /= dv;
-#pragma unroll
-    for (int r = 0; r < 9; ++r) dM[r] = system[r * 19 + 9 + c] - du * system[r * 19 + 18];
-    if constexpr (OUT == kOutModuli) {
-      const int g = c / 3, l = c % 3;
-      double u[3], w[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        u[i] = g == 0 ? f.U[i] : (g == 1 ? f.U[3 + i] : f.U[6 + i]);
-        w[i] = l == 0 ? f.W[i] : (l == 1 ? f.W[3 + i] : f.W[6 + i]);
-      }
-      store_moduli<HE>(cm, f, u, w, dM, g, l, out);
-    } else {
-      store_dMe(q, RpFi, dM, c, out);
-    }
-  }
+__device__ __forceinline__ double *tangent_slots() {
+  __shared__ double sCol[(OUT == kOutPoint ? 1 : 72) * 64];
+  return sCol + threadIdx.x;
+}
+// Column c of the tangent from its dM, in a rolled loop over the columns: U and W in the lane's LDS.
+template <bool HE, int OUT>
+__device__ __forceinline__ void store_column(const CPMaterial &cm, const TangentPoint &q, const PointFrame<HE> &f,
+                                             const double *RpFi, const double *col, const double *dM, int c,
+                                             double *out) {
   if constexpr (OUT == kOutModuli) {
+    const int g = c / 3, l = c - 3 * g;
+    double u[3], w[3];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];
+    for (int i = 0; i < 3; ++i) {
+      u[i] = col[(kColU + g * 3 + i) * 64];
+      w[i] = col[(kColW + l * 3 + i) * 64];
+    }
+    store_moduli<HE>(cm, f, u, w, dM, g, l, out);
+  } else {
+    store_dMe(q, RpFi, dM, c, out);
+  }
+}
+// What store_column needs: the point's T to the record and its frame, with U and W to the lane's LDS, or
+// R pF(n)^-1.
+template <bool HE, int OUT>
+__device__ __forceinline__ void open_columns(const CPArgs &a, const CPMaterial &cm, int64_t t, const TangentPoint &q,
+                                             PointFrame<HE> &f, double *RpFi, double *col, double *out) {
+  if constexpr (OUT == kOutModuli) {
+    double T[9];
+    point_frame<HE>(a, cm, t, q, true, f, T);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];  // where Fr was
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      col[(kColU + i) * 64] = f.U[i];
+      col[(kColW + i) * 64] = f.W[i];
+    }
+  } else {
+    mul_ab(q.pFi, q.R, RpFi);
   }
 }
 
 template <bool HE, int FLOW, int OUT>
 __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
-  // The columns' kappa -- then their solutions -- and U, W, by a run-time column.  36 KB per wave.
-  __shared__ double sCol[(OUT == kOutPoint ? 1 : 72) * 64];
-  constexpr int kY = 0, kU = 54, kW = 63;
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= nqb) return;
   const int64_t NQ = a.n_qp;
@@ -1495,7 +1528,7 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
         for (int r = 0; r < 9; ++r) L.G[r][I] = h[r];
       }
     }
-    double *col = sCol + threadIdx.x;  // field i at col[i * 64]
+    double *col = tangent_slots<HE, FLOW, OUT>();
     {
       double U[9], W[9], RpFi[9], S6[36], Y[10][6];
       tangent_frames(q, U, W, RpFi);
@@ -1515,15 +1548,15 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
 #pragma unroll
       for (int c = 0; c < 9; ++c)
 #pragma unroll
-        for (int I = 0; I < 6; ++I) col[(kY + c * 6 + I) * 64] = Y[c][I];
+        for (int I = 0; I < 6; ++I) col[(kColY + c * 6 + I) * 64] = Y[c][I];
 #pragma unroll
       for (int r = 0; r < 9; ++r)
 #pragma unroll
         for (int I = 0; I < 6; ++I) v[r] -= L.G[r][I] * Y[9][I];
     }
     if (!ok) {
-      for (uint64_t rest = __ballot(1); rest; rest &= rest - 1)
-        if (int(threadIdx.x) == __builtin_ctzll(rest)) tangent_pivot<HE, FLOW, OUT>(a, t);
+      const uint64_t m = __ballot(1);
+      if (int(threadIdx.x) == __builtin_ctzll(m)) a.pivots[blockIdx.x] = m;
       return;
     }
     double dv = 0.0;
@@ -1532,24 +1565,12 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
     const double rdv = 1.0 / dv;
     PointFrame<HE> f;
     double RpFi[9];
-    if constexpr (OUT == kOutModuli) {
-      double T[9];
-      point_frame<HE>(a, cm, t, q, true, f, T);
-#pragma unroll
-      for (int i = 0; i < 9; ++i) out[i * kRecStride] = T[i];
-#pragma unroll
-      for (int i = 0; i < 9; ++i) {
-        col[(kU + i) * 64] = f.U[i];
-        col[(kW + i) * 64] = f.W[i];
-      }
-    } else {
-      mul_ab(q.pFi, q.R, RpFi);
-    }
+    open_columns<HE, OUT>(a, cm, t, q, f, RpFi, col, out);
 #pragma unroll 1
     for (int c = 0; c < 9; ++c) {
       double dM[9], du = 0.0, y[6];
 #pragma unroll
-      for (int I = 0; I < 6; ++I) y[I] = col[(kY + c * 6 + I) * 64];
+      for (int I = 0; I < 6; ++I) y[I] = col[(kColY + c * 6 + I) * 64];
 #pragma unroll
       for (int r = 0; r < 9; ++r) {
         double z = 0.0;
@@ -1561,19 +1582,83 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
       du *= rdv;
 #pragma unroll
       for (int r = 0; r < 9; ++r) dM[r] -= du * v[r];
-      if constexpr (OUT == kOutModuli) {
-        const int g = c / 3, l = c - 3 * g;
-        double u[3], w[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          u[i] = col[(kU + g * 3 + i) * 64];
-          w[i] = col[(kW + l * 3 + i) * 64];
-        }
-        store_moduli<HE>(cm, f, u, w, dM, g, l, out);
-      } else {
-        store_dMe(q, RpFi, dM, c, out);
-      }
+      store_column<HE, OUT>(cm, q, f, RpFi, col, dM, c, out);
     }
+  }
+}
+
+// The points that cp_tangent has left to the 9 x 9 system with pivoting, by the masks of its waves: a
+// wave looks through `waves` of them, takes a mask's points together and clears it.  A launch of its
+// own: beside the common path, in one kernel, it costs that path registers (cp_tangent 705 us instead of
+// 575 on 998,250 points), and as a function called there the compiler lost the other lanes' values.
+// A tangent pass over 82,944 points that all come here takes 214 us, beside 151 where none does (with
+// the points one after another, each lane's system in LDS, 8.2 ms; in the sample frame, where every point
+// pivoted, 337).  With nothing to do it takes 5 us, as long as any short launch.
+template <bool HE, int FLOW, int OUT>
+__device__ __forceinline__ void tangent_pivot(const CPArgs &a, const CPMaterial &cm, int64_t t) {
+  double *out = a.qpbuf + qrec(a.qp_base + t), *col = tangent_slots<HE, FLOW, OUT>();
+  TangentPoint q;
+  if (!tangent_point<HE, FLOW>(a, cm, t, q)) return;  // counted by cp_tangent
+  LocalLin L;
+  double Ah[81], v[9];
+  int piv[9];
+  {
+    double U[9], W[9], RpFi[9], AtE[9];
+    tangent_frames(q, U, W, RpFi);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+      double kp[6];
+      kappa(U + (c / 3) * 3, W + (c % 3) * 3, kp);
+#pragma unroll
+      for (int I = 0; I < 6; ++I) col[(kColY + c * 6 + I) * 64] = kp[I];
+    }
+    tangent_lin<HE>(cm, a.dt, q, AtE, L);
+    cp_matrix(L, AtE, q.p.T, a.dt * q.x[9] * q.p.pJ, Ah);
+  }
+  if (!factor_pivot<9>(Ah, piv)) {
+    atomicAdd(a.err, 1);
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 9; ++r) v[r] = q.p.T[r];
+  solve_pivot<9>(Ah, piv, v);
+  double dv = 0.0;
+#pragma unroll
+  for (int r = 0; r < 9; ++r) dv += q.p.T[r] * v[r];
+  const double rdv = 1.0 / dv;
+  PointFrame<HE> f;
+  double RpFi[9];
+  open_columns<HE, OUT>(a, cm, t, q, f, RpFi, col, out);
+#pragma unroll 1
+  for (int c = 0; c < 9; ++c) {
+    double dM[9], du = 0.0, y[6];
+#pragma unroll
+    for (int I = 0; I < 6; ++I) y[I] = col[(kColY + c * 6 + I) * 64];
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+      dM[r] = 0.0;
+#pragma unroll
+      for (int I = 0; I < 6; ++I) dM[r] -= L.G[r][I] * y[I];
+    }
+    solve_pivot<9>(Ah, piv, dM);
+#pragma unroll
+    for (int r = 0; r < 9; ++r) du += q.p.T[r] * dM[r];
+    du *= rdv;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) dM[r] -= du * v[r];
+    store_column<HE, OUT>(cm, q, f, RpFi, col, dM, c, out);
+  }
+}
+template <bool HE, int FLOW, int OUT>
+__global__ __launch_bounds__(64) void cp_tangent_pivot(CPArgs a, int64_t n_waves, int waves) {
+  const CPMaterial cm = a.cpmats[0];
+  const int64_t w0 = int64_t(blockIdx.x) * waves, w1 = w0 + waves < n_waves ? w0 + waves : n_waves;
+#pragma unroll 1
+  for (int64_t w = w0; w < w1; ++w) {
+    const uint64_t m = a.pivots[w];
+    if (!m) continue;
+    if ((m >> threadIdx.x) & 1) tangent_pivot<HE, FLOW, OUT>(a, cm, w * 64 + threadIdx.x);
+    if (threadIdx.x == 0) a.pivots[w] = 0;
   }
 }
 
@@ -2538,11 +2623,19 @@ void launch_cp_tangent(const CPArgs &a, bool with_D, hipStream_t s) {
   const int64_t nq = a.nq;
   if (nq <= 0) return;
   const unsigned grid = unsigned((nq + 63) / 64);
+  // masks per wave of cp_tangent_pivot: one until the chip's 1024 waves are busy twice over, few
+  // enough waves beyond that a launch that finds nothing stays short
+  const unsigned waves = (grid + 2 * kQueueWaves - 1) / (2 * kQueueWaves);
   by_law(a, [&](auto he, auto fl) {
     constexpr bool HE = decltype(he)::value;
     constexpr int FLOW = decltype(fl)::value;
-    if (a.tf) cp_tangent<HE, FLOW, kOutMe><<<grid, 64, 0, s>>>(a, nq);
-    else if (with_D) cp_tangent<HE, FLOW, kOutModuli><<<grid, 64, 0, s>>>(a, nq);
+    const auto columns = [&](auto out) {
+      constexpr int OUT = decltype(out)::value;
+      cp_tangent<HE, FLOW, OUT><<<grid, 64, 0, s>>>(a, nq);
+      cp_tangent_pivot<HE, FLOW, OUT><<<(grid + waves - 1) / waves, 64, 0, s>>>(a, grid, int(waves));
+    };
+    if (a.tf) columns(std::integral_constant<int, kOutMe>{});
+    else if (with_D) columns(std::integral_constant<int, kOutModuli>{});
     else cp_tangent<HE, FLOW, kOutPoint><<<grid, 64, 0, s>>>(a, nq);
   });
 }

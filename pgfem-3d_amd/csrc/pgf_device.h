@@ -156,6 +156,7 @@ struct CPArgs {
   // Me 9, S 6, pJ 1, D = dMe/dF 81 by columns, field 16 + 9 c + r holding D[r][c])
   double *qpbuf;
   int32_t *err;
+  unsigned long long *pivots;  // per wave of the tangent kernel, its points left to cp_tangent_pivot
   unsigned long long *qnext;  // global work queue of the local Newton (cp_chunk = 1), else null
   int32_t law;                // cpmats[0].law, read on the host to pick the kernels
   int32_t flow;               // likewise: 2 cpmats[0].ipow >= 0 and w = 0, 1 ipow >= 0, 0 neither
