@@ -312,6 +312,13 @@ int pgf_get_tuning(pgf_handle h, int64_t *cp_chunk, int32_t *gather_waves, int32
  * {1, 2, 4}, gather_batch in {2, 4, 8}; a value <= 0 keeps the current one. */
 int pgf_set_tuning(pgf_handle h, int64_t cp_chunk, int32_t gather_waves, int32_t gather_batch);
 
+/* Crystal plasticity: a point's local systems are eliminated without pivoting while no multiplier
+ * exceeds these bounds, and with partial pivoting otherwise: step for a Newton step of the local
+ * solve (default 1e6; the residual, not the matrix, fixes the point that it ends at), tangent for
+ * the consistent tangent (default 1e4).  0 pivots wherever there is something to eliminate.  (No
+ * reference counterpart.) */
+int pgf_set_pivoting(pgf_handle h, double step, double tangent);
+
 /* Assembly of element rows into f and the CSR values (the role of fd_res_assemble and
  * PLoc_Sparse, src/fd_residuals.cc:58-73, src/PLoc_Sparse.cc:15-175).  Both modes are
  * deterministic, use no atomics, and give the same sums up to the order of the additions:

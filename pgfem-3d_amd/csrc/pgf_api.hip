@@ -252,6 +252,7 @@ struct pgf_handle_s {
   // to balance a batch of 64 per wave).  cp_newton on 10,368 QPs 184 us at 256, 99 at 128, 55 at
   // 64 and 1; on 998,250 QPs 774, 769, 755, 735.
   int64_t cp_chunk = 1;
+  double max_step = pgf::kMaxMultStep, max_tangent = pgf::kMaxMultTangent;  // pgf_set_pivoting
   unsigned long long *d_qnext = nullptr;  // the global queue's counter
   unsigned long long *d_pivots = nullptr;  // [cp_nq / 64], zero between passes (pgf::CPArgs::pivots)
   int32_t gather_waves = 4;  // nodes per gather workgroup (autotuned; capped by LDS)
@@ -359,6 +360,8 @@ pgf::CPArgs cp_args(pgf_handle h, const Block &b, const pgf_nodal_input *in) {
   c.iters = h->d_iters;
   c.qnext = h->cp_chunk == 1 ? h->d_qnext : nullptr;
   c.pivots = h->d_pivots;
+  c.max_step = h->max_step;
+  c.max_tangent = h->max_tangent;
   c.warm = h->warm;
   c.qpbuf = h->d_qpbuf;  // indexed by device QP (pgf::qrec)
   c.err = h->d_err;
@@ -2031,6 +2034,14 @@ int pgf_get_tuning(pgf_handle h, int64_t *cp_chunk, int32_t *gather_waves, int32
   if (cp_chunk) *cp_chunk = h->cp_chunk;
   if (gather_waves) *gather_waves = std::min(h->gather_waves, std::max(pgf::gather_waves(h->maxlen), 1));
   if (gather_batch) *gather_batch = h->gather_batch;
+  return PGF_OK;
+}
+
+int pgf_set_pivoting(pgf_handle h, double step, double tangent) {
+  if (!h || !(step >= 0.0) || !(tangent >= 0.0)) return PGF_EINVAL;
+  if (int rc = drop_graph(h)) return rc;  // a captured pass holds the bounds
+  h->max_step = step;
+  h->max_tangent = tangent;
   return PGF_OK;
 }
 

@@ -19,7 +19,7 @@
 // solved through the Schur complement of its (M, M) block: with the bordered structure
 //   [A b c; d^T 0 0; e^T 0 f]
 // one 9x9 elimination (in registers, unpivoted; the rare matrix that needs pivoting is solved
-// again in scratch memory) serves the two right-hand sides of a Newton step, and a 6x6 one the
+// again with it) serves the two right-hand sides of a Newton step, and a 6x6 one the
 // nine columns of the tangent.  All of it runs in the crystal frame (see below).
 //
 // Kernels:
@@ -571,14 +571,14 @@ __device__ __forceinline__ void cp_matrix(const LocalLin &L, const double *AtE, 
 
 // Gaussian elimination of A with NR right-hand sides, solutions in B, without pivoting; false
 // where a multiplier exceeds max_mult or a pivot is no number, and the caller takes
-// eliminate_pivot.  The local system is the identity plus the slip systems' positive part, so
+// factor_pivot.  The local system is the identity plus the slip systems' positive part, so
 // large multipliers are rare (above 1000 in 0.1% of the matrices of a plastic step), and partial
 // pivoting by predicated swaps is more instructions than the elimination.  A Newton step only has
 // to be a good direction: the residual, not the matrix, fixes the point that the iteration ends
-// at, and at 1e6 its relative error stays near 1e-10.  At 1e3 one turn of the wave in ten waited
-// for a lane's pivoting, and cp_newton took 2295 us instead of 740 (998,250 QPs).  The tangent is
-// a result, and its bound lower.
-constexpr double kMaxMultStep = 1.0e6, kMaxMultTangent = 1.0e4;
+// at, and at 1e6 its relative error stays near 1e-10.  A step that pivots is taken twice: with a bound
+// of 1e3 a pass over 998,250 points takes 2333 us instead of 2277, and 3476 where every step pivots.
+// The tangent is a result, and its bound lower; where every point's pivots, the pass takes 2564 us.
+// (kMaxMultStep and kMaxMultTangent, unless the caller sets others.)
 template <int N, int NR>
 __device__ __forceinline__ bool eliminate(double (&A)[N * N], double (&B)[NR][N], double max_mult) {
   double lmax = 0.0, rd[N];
@@ -607,54 +607,6 @@ __device__ __forceinline__ bool eliminate(double (&A)[N * N], double (&B)[NR][N]
     }
   return lmax <= max_mult && fabs(rd[N - 1]) < __builtin_huge_val();
 }
-// The same with partial pivoting, in LDS, for one lane: rare, and kept from costing the common path
-// registers (the system is stored before the common path consumes it, and solved after it).  In a
-// lane's scratch memory every step waited for it: 100 us for a wave that met such a point.
-// The solutions take the right-hand sides' places; false for a singular matrix.
-template <int N, int NR>
-__device__ __forceinline__ void store_system(const double (&A)[N * N], const double (&B)[NR][N], double *a) {
-  constexpr int W = N + NR;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) a[i * W + j] = A[i * N + j];
-#pragma unroll
-    for (int q = 0; q < NR; ++q) a[i * W + N + q] = B[q][i];
-  }
-}
-template <int N, int NR>
-__device__ __forceinline__ bool eliminate_pivot(double *a) {
-  constexpr int W = N + NR;
-  bool ok = true;
-#pragma unroll 1
-  for (int k = 0; k < N; ++k) {
-    int p = k;
-    double amax = fabs(a[k * W + k]);
-#pragma unroll 1
-    for (int i = k + 1; i < N; ++i) {
-      const double v = fabs(a[i * W + k]);
-      p = v > amax ? i : p;
-      amax = v > amax ? v : amax;
-    }
-    ok = ok && amax > 0.0;
-    double row[W];
-    const double r = 1.0 / a[p * W + k];
-#pragma unroll
-    for (int j = 0; j < W; ++j) row[j] = a[p * W + j] * r;
-#pragma unroll
-    for (int j = 0; j < W; ++j) a[p * W + j] = a[k * W + j];
-#pragma unroll
-    for (int j = 0; j < W; ++j) a[k * W + j] = row[j];
-#pragma unroll 1
-    for (int i = 0; i < N; ++i) {  // to the diagonal: the rows above take part
-      const double l = i == k ? 0.0 : a[i * W + k];
-#pragma unroll
-      for (int j = 0; j < W; ++j) a[i * W + j] -= l * row[j];
-    }
-  }
-  return ok;
-}
-
 // The same with partial pivoting, as factors and solutions: every lane that needs it takes part, its
 // rows exchanged by selects, so that no index is known at run time only.  False for a singular matrix.
 template <int N>
@@ -912,6 +864,42 @@ __global__ __launch_bounds__(64) void cp_start_kernel(CPArgs a) {
 }
 
 // ------------------------------------------------------------------- Newton kernel
+// The lane's slots of the Newton kernel's LDS: A (9), x (11), dx (11), det pF(n), g(n), gscale.
+constexpr int kA = 0, kX = 9, kDX = 20, kDet = 31, kGn = 32, kGs = 33;
+// A step's system with pivoting, formed again from G and the residual's right-hand side (rec) and from
+// A and x (pk): as a copy of the matrix, in registers or scratch memory, it cost the steps that do not
+// pivot 2 us of a pass over 10,368 points.
+__device__ __forceinline__ bool step_pivot(const double *rec, const double *pk, double dt, double (&Ah)[81],
+                                           double (&u)[2][9]) {
+  LocalLin L;
+  double M[9], Mi[9], A[9], eF[9], AtE[9], T[9], dM;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    M[i] = pk[(kX + i) * 64];
+    A[i] = pk[(kA + i) * 64];
+  }
+  inv_det(M, Mi, dM);
+  const double pJ = pk[kDet * 64] / dM;
+  mm3(A, M, eF);
+  mtm3(A, eF, AtE);
+#pragma unroll
+  for (int i = 0; i < 54; ++i) L.G[i / 6][i % 6] = rec[i * kRecStride];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int r = i * 3 + j;
+      T[r] = Mi[j * 3 + i];
+      u[0][r] = rec[(54 + r) * kRecStride];
+      u[1][r] = -pJ * T[r];
+    }
+  cp_matrix(L, AtE, T, dt * pk[(kX + 9) * 64] * pJ, Ah);
+  int piv[9];
+  const bool ok = factor_pivot<9>(Ah, piv);
+  solve_pivot<9>(Ah, piv, u[0]);
+  solve_pivot<9>(Ah, piv, u[1]);
+  return ok;
+}
 // One wave per workgroup, one QP per lane: wave w works through QPs [w*chunk, (w+1)*chunk) of the
 // block, or, with a.qnext set, draws them from one global queue.  Which lane takes a QP does not
 // change its result.  A wave hands out new QPs when kRefill of its lanes are idle: at each idle lane it
@@ -922,7 +910,7 @@ __global__ __launch_bounds__(64) void cp_start_kernel(CPArgs a) {
 //
 // Bound by FP64 issue: a turn is about 3300 instructions for 64 QPs.  A turn has no divergent
 // branch around its stages (values would be kept across it), and each stage is closed by pin, so
-// the widest stretch, the 9 x 9 elimination, fits 298 registers with nothing spilled.  One wave
+// the widest stretch, the 9 x 9 elimination, fits 300 registers with nothing spilled.  One wave
 // per SIMD: at two, 256 registers spill and it takes 800 us instead of 740 (998,250 QPs; 2743 us
 // in the sample frame, with the pivoting and the slip systems' tensors in registers).
 template <bool HE, int FLOW>
@@ -932,9 +920,8 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
   // The lane's QP data that lives across turns sits in LDS (lane-fastest; each lane touches
   // only its own slots), read where used, rather than in registers held through the material
   // point and the elimination: A (9), x (11), dx (11), det pF(n), g(n), gscale.  17 KB per wave.
-  __shared__ double sPk[34 * 64], sSystem[9 * 11];
+  __shared__ double sPk[34 * 64];
   double *pk = sPk + lane;  // field i at pk[i * 64]
-  constexpr int kA = 0, kX = 9, kDX = 20, kDet = 31, kGn = 32, kGs = 33;
   constexpr int kRefill = 48;
   const double dt = a.dt;
   const CPMaterial cm = a.cpmats[0];  // one material for every CP point: wave-uniform, loaded once
@@ -1032,13 +1019,9 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
     // One turn: every live lane evaluates the material point once, at its start or at its
     // line-search trial x + alpha dx; a lane whose start or accepted trial this is then takes a
     // Newton step from it.  A trial's evaluation is thus also the point of the next iteration.
-    // A step that asked for pivoting is taken in a turn of its own, in which the wave's other
-    // lanes wait: the choice of elimination is then the wave's, not the lane's, and the system's
-    // copy is one lane's, in LDS.
-    const uint64_t again = __ballot(phase == kPhAgain);
-    const bool pivots = again != 0;
-    const bool pivot_lane = pivots && lane == __builtin_ctzll(again);
-    const bool turn = pivots ? pivot_lane : phase != kPhDone;
+    // A lane whose elimination asked for pivoting takes the same step once more in the next turn, beside
+    // the wave's other lanes, with a copy of what its system is made of in the point's record.
+    const bool again = phase == kPhAgain, turn = phase != kPhDone;
     const bool moved = phase == kPhTrial || phase == kPhFull;
     const double len = phase == kPhTrial ? alpha : (phase == kPhFull ? 1.0 : 0.0);
     double xc[11], A[9];
@@ -1129,22 +1112,21 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
         pin(u[1]);
 #pragma unroll
         for (int r = 0; r < 9; ++r) pin(L.G[r]);
+        if (again) {
+          double *rec = a.qpbuf + qrec(a.qp_base + q) + kRecStep * kRecStride;
+#pragma unroll
+          for (int i = 0; i < 54; ++i) rec[i * kRecStride] = L.G[i / 6][i % 6];
+#pragma unroll
+          for (int i = 0; i < 9; ++i) rec[(54 + i) * kRecStride] = u[0][i];
+        }
         end_stage();
         cp_matrix(L, AtE, T, dl, Ah);
       }
       pin(Ah);
       end_stage();
       pk = reload(sPk, lane);
-      if (pivot_lane) store_system<9, 2>(Ah, u, sSystem);
-      bool solved = eliminate<9, 2>(Ah, u, kMaxMultStep);
-      if (pivot_lane) {
-        solved = eliminate_pivot<9, 2>(sSystem);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) {
-          u[0][i] = sSystem[i * 11 + 9];
-          u[1][i] = sSystem[i * 11 + 10];
-        }
-      }
+      bool solved = eliminate<9, 2>(Ah, u, a.max_step);
+      if (again) solved = step_pivot(a.qpbuf + qrec(a.qp_base + q) + kRecStep * kRecStride, pk, dt, Ah, u);
       double M[9], Mi[9], dM, du = 0.0, dv = 0.0, ex = 0.0, dx[11];
 #pragma unroll
       for (int i = 0; i < 9; ++i) M[i] = pk[(kX + i) * 64];
@@ -1173,7 +1155,7 @@ __global__ __launch_bounds__(64) void cp_newton(CPArgs a, int64_t chunk) {
       size = fmax(size, fabs(dx[10]) / pk[kGn * 64]);
       if (step) {
         if (!solved) {
-          fail = pivots;  // singular
+          fail = again;  // singular
           phase = kPhAgain;
         } else if (size < cm.tol) {
 #pragma unroll
@@ -1544,7 +1526,7 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
 #pragma unroll
       for (int c = 0; c < 9; ++c) kappa(U + (c / 3) * 3, W + (c % 3) * 3, Y[c]);
       k_of(AtE, v, Y[9]);
-      ok = eliminate<6, 10>(S6, Y, kMaxMultTangent) && ok;
+      ok = eliminate<6, 10>(S6, Y, a.max_tangent) && ok;
 #pragma unroll
       for (int c = 0; c < 9; ++c)
 #pragma unroll
@@ -2600,7 +2582,7 @@ void launch_cp_newton(const CPArgs &a, int64_t chunk, hipStream_t s) {
   // 100,736 QPs); above, it keeps the waves filled (178,752 QPs, up to 25 iterations: 1000 -> 900).
   if (nq <= 2 * 64 * kQueueWaves) b.qnext = nullptr;
   if (b.qnext) {
-    // one persistent wave per SIMD of the chip (the kernel holds all 512 registers of a lane),
+    // one persistent wave per SIMD of the chip (the kernel takes more than 256 registers of a lane),
     // draining the global queue; the counter is reset by a kernel, so a captured pass replays it
     cp_queue_reset<<<1, 1, 0, s>>>(b.qnext);
     chunk = 64;

@@ -156,6 +156,7 @@ struct CPArgs {
   // Me 9, S 6, pJ 1, D = dMe/dF 81 by columns, field 16 + 9 c + r holding D[r][c])
   double *qpbuf;
   int32_t *err;
+  double max_step, max_tangent;  // largest multipliers of an elimination without pivoting
   unsigned long long *pivots;  // per wave of the tangent kernel, its points left to cp_tangent_pivot
   unsigned long long *qnext;  // global work queue of the local Newton (cp_chunk = 1), else null
   int32_t law;                // cpmats[0].law, read on the host to pick the kernels
@@ -172,8 +173,11 @@ struct CPArgs {
 enum : int { kKinState = 1, kKinRec = 2, kKinDefl = 4 };
 // A displacement element's record: fields 0..8 the pass's F where it is not the state's, or the plain
 // start x(0..10) and its flag, then T; kRecXi the inverse of dX/dxi; kRecA the moduli, column
-// (g, l) at kRecA + 9 (3 g + l); kRecW, until the last of them is stored, detJ w.
-constexpr int kRecXi = 12, kRecA = 21, kRecW = kRecA + 80;
+// (g, l) at kRecA + 9 (3 g + l); kRecW, until the last of them is stored, detJ w; kRecStep, within the
+// local solve, 63 numbers of a step that pivots.
+constexpr int kRecXi = 12, kRecA = 21, kRecStep = kRecA, kRecW = kRecA + 80;
+static_assert(kRecStep + 63 <= kRecW, "a step's numbers beside detJ w");
+constexpr double kMaxMultStep = 1.0e6, kMaxMultTangent = 1.0e4;  // CPArgs::max_step, max_tangent
 constexpr int kCPBuf = 102;  // doubles per QP in qpbuf
 // qpbuf holds the records of 8 QPs at a time with the field outermost: field f of device QP q
 // is at qpbuf[qrec(q) + f * kRecStride].  A wave's store of one field over its 64 QPs then

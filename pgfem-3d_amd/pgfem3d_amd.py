@@ -134,6 +134,7 @@ def lib() -> C.CDLL:
             "pgf_autotune": [P, P, D, P],
             "pgf_get_tuning": [P, P, P, P],
             "pgf_set_tuning": [P, I64, I32, I32],
+            "pgf_set_pivoting": [P, D, D],
             "pgf_set_surrogate": [P, P, P, P, P],
             "pgf_set_three_field": [P, I32],
             "pgf_tf_initial": [P, P, P],
@@ -164,7 +165,7 @@ def exported_symbols():
         "pgf_set_three_field", "pgf_tf_initial", "pgf_tf_update", "pgf_tf_accept", "pgf_tf_get", "pgf_tf_set",
         "pgf_autotune", "pgf_residual_tangent_static", "pgf_stage_doubles",
         "pgf_subdivision_param", "pgf_cp_start_stats", "pgf_output_variables", "pgf_mlp_infer",
-        "pgf_get_tuning", "pgf_set_tuning",
+        "pgf_get_tuning", "pgf_set_tuning", "pgf_set_pivoting",
     ]
 
 
@@ -378,6 +379,10 @@ class Handle:
     def set_tuning(self, cp_chunk=0, gather_waves=0, gather_batch=0):
         _check(self._lib.pgf_set_tuning(self.h, int(cp_chunk), int(gather_waves), int(gather_batch)),
                "pgf_set_tuning")
+
+    def set_pivoting(self, step=1e6, tangent=1e4):
+        """Largest multipliers of the crystal-plasticity eliminations without pivoting."""
+        _check(self._lib.pgf_set_pivoting(self.h, float(step), float(tangent)), "pgf_set_pivoting")
 
     def set_stream(self, stream_ptr: int | None):
         _check(self._lib.pgf_set_stream(self.h, stream_ptr), "pgf_set_stream")
