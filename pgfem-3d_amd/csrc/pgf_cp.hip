@@ -1383,6 +1383,22 @@ __device__ __forceinline__ void store_moduli(const CPMaterial &cm, const PointFr
 // three-field element, Me, S, pJ and dMe/dF.
 enum : int { kOutPoint = 0, kOutModuli = 1, kOutMe = 2 };
 
+// The record of a point without a tangent: nothing of an earlier pass reaches the element.
+template <int OUT>
+__device__ __forceinline__ void zero_record(double *out) {
+  if constexpr (OUT == kOutMe) {
+#pragma unroll
+    for (int i = 0; i < 97; ++i) out[i * kRecStride] = 0.0;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) out[i * kRecStride] = 0.0;
+    if constexpr (OUT == kOutModuli) {
+#pragma unroll
+      for (int i = 0; i < 81; ++i) out[(kRecA + i) * kRecStride] = 0.0;
+    }
+  }
+}
+
 // The lanes' LDS of the tangent kernel, field i of a lane at [i * 64]: the columns' kappa -- then their
 // solutions -- and the U, W of the moduli, by a run-time column.  36 KB per wave.
 constexpr int kColY = 0, kColU = 54, kColW = 63;
@@ -1440,17 +1456,7 @@ __global__ __launch_bounds__(64) void cp_tangent(CPArgs a, int64_t nqb) {
   TangentPoint q;
   if (!tangent_point<HE, FLOW>(a, cm, t, q)) {
     atomicAdd(a.err, 1);
-    if constexpr (OUT == kOutMe) {
-#pragma unroll
-      for (int i = 0; i < 97; ++i) out[i * kRecStride] = 0.0;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 9; ++i) out[i * kRecStride] = 0.0;
-      if constexpr (OUT == kOutModuli) {
-#pragma unroll
-        for (int i = 0; i < 81; ++i) out[(kRecA + i) * kRecStride] = 0.0;
-      }
-    }
+    zero_record<OUT>(out);
     return;
   }
   const CPPoint &p = q.p;
@@ -1599,6 +1605,7 @@ __device__ __forceinline__ void tangent_pivot(const CPArgs &a, const CPMaterial 
   }
   if (!factor_pivot<9>(Ah, piv)) {
     atomicAdd(a.err, 1);
+    zero_record<OUT>(out);
     return;
   }
 #pragma unroll
