@@ -39,8 +39,7 @@ struct Block {
   int64_t *d_soff = nullptr;       // gather mode: [ne*nne] staging offsets
   int32_t *d_rslot = nullptr;      // and block numbers
   int32_t *d_mat = nullptr;
-  int32_t *d_egrain = nullptr;  // crystal plasticity: grain per element / per QP (device order)
-  int32_t *d_qgrain = nullptr;
+  int32_t *d_qgrain = nullptr;  // crystal plasticity: grain per QP (device order)
 };
 
 // Interface elements of one kind (nn nodes per side), in mesh order; colour lists as Block.
@@ -1221,8 +1220,6 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
     if (hipMemset(h->d_qgrain_all, 0, sizeof(int32_t) * h->n_qp) != hipSuccess) return fail(PGF_EHIP);
     for (auto &b : h->blocks) {
       if (b.model != PGF_MODEL_CRYSTAL_PLASTICITY) continue;
-      if ((rc = pgf::dalloc(&b.d_egrain, size_t(b.ne)))) return fail(rc);
-      if (hipMemset(b.d_egrain, 0, sizeof(int32_t) * b.ne) != hipSuccess) return fail(PGF_EHIP);
       b.d_qgrain = h->d_qgrain_all + b.qp_base;  // view into the handle's array
     }
     const double I9[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
@@ -1252,7 +1249,6 @@ int pgf_destroy(pgf_handle h) {
     hipFree(b.d_rslot);
     hipFree(b.d_clist);
     hipFree(b.d_mat);
-    hipFree(b.d_egrain);
   }
   for (auto &cb : h->cblocks) {
     hipFree(cb.d_conn);
@@ -1805,17 +1801,15 @@ int pgf_set_orientations(pgf_handle h, int32_t n_grains, const double *R, const 
     pgf::make_grain(Q, g[k]);
     pgf::rot_to_quat(Q, q.data() + 4 * k);
   }
-  std::vector<std::vector<int32_t>> egs(h->blocks.size()), qgs(h->blocks.size());
+  std::vector<std::vector<int32_t>> qgs(h->blocks.size());
   if (elem_grain)
     for (size_t bi = 0; bi < h->blocks.size(); ++bi) {
       const Block &b = h->blocks[bi];
       if (b.model != PGF_MODEL_CRYSTAL_PLASTICITY) continue;
-      egs[bi].resize(b.ne);
       qgs[bi].resize(b.ne * b.nqp);
       for (int64_t k = 0; k < b.ne; ++k) {
         const int32_t gk = elem_grain[b.elems[k]];
         if (gk < 0 || gk >= n_grains) return PGF_EINVAL;
-        egs[bi][k] = gk;
         for (int ip = 0; ip < b.nqp; ++ip) qgs[bi][k * b.nqp + ip] = gk;
       }
     }
@@ -1828,10 +1822,9 @@ int pgf_set_orientations(pgf_handle h, int32_t n_grains, const double *R, const 
   if ((rc = pgf::upload(&h->d_grains, g.data(), g.size()))) return rc;
   if ((rc = pgf::upload(&h->d_gquat, q.data(), q.size()))) return rc;
   for (size_t bi = 0; bi < h->blocks.size(); ++bi) {
-    if (egs[bi].empty()) continue;
-    const Block &b = h->blocks[bi];
-    if (hipMemcpy(b.d_egrain, egs[bi].data(), egs[bi].size() * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(b.d_qgrain, qgs[bi].data(), qgs[bi].size() * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess)
+    if (qgs[bi].empty()) continue;
+    if (hipMemcpy(h->blocks[bi].d_qgrain, qgs[bi].data(), qgs[bi].size() * sizeof(int32_t), hipMemcpyHostToDevice) !=
+        hipSuccess)
       return PGF_EHIP;
   }
   return PGF_OK;

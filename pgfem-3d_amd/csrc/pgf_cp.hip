@@ -48,7 +48,6 @@ namespace {
 
 using namespace dev;
 
-constexpr int kWave = 64;
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 
 // Voigt helpers: index I -> (i,j) in xx,yy,zz,xy,yz,xz
