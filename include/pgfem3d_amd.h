@@ -271,8 +271,8 @@ int pgf_subdivision_param(pgf_handle h, double dt, double *alpha);
  * fixed device array of PGF_STATIC_STAGE_DOUBLES doubles (64 MiB) that the library holds on
  * each GPU it runs on until the process ends, instead of the buffer pgf_residual_tangent
  * allocates at its first gather pass.  The call makes no hipMalloc, hipFree or other
- * allocating call; it launches eagerly (even with pgf_set_graph on) and synchronises the
- * handle's stream to read the failure count, like pgf_residual_tangent.
+ * allocating call; it launches eagerly (even with pgf_set_graph on) and waits for the pass to
+ * end and its failure count, like pgf_residual_tangent.
  * No counterpart in the reference: it is for callers that cannot allocate device memory
  * (serving loops, harnesses that forbid allocation).
  * Returns PGF_ESCRATCH when the mesh's staging blocks exceed the array (pgf_stage_doubles
@@ -298,8 +298,9 @@ int pgf_set_graph(pgf_handle h, int on);
 /* Autotune the launch configuration by timing passes at the given input (no reference
  * counterpart: the reference's element loop has no launch shape):
  *   - points per wavefront of the crystal-plasticity local-Newton work queue (QPs per wave
- *     range, 64..2048, or 1: every wave draws its QPs from one global queue as its lanes free
- *     up), on integrating residual passes;
+ *     range, 64..2048, or 1: above 131,072 QPs every wave draws its QPs from one global queue as
+ *     its lanes free up, up to there, where a queue has nothing to balance, 64 per wave), on
+ *     integrating residual passes;
  *   - the gather assembly's tile (gather mode): nodes per workgroup (1, 2, 4; capped by the
  *     LDS a node's rows take) x staging blocks each half-wave keeps in flight (2, 4, 8), on
  *     residual + tangent passes.
@@ -308,7 +309,7 @@ int pgf_set_graph(pgf_handle h, int on);
 int pgf_autotune(pgf_handle h, const pgf_nodal_input *in, double dt, int64_t *chunk);
 /* The launch configuration in use (pgf_autotune's choice or pgf_set_tuning's). */
 int pgf_get_tuning(pgf_handle h, int64_t *cp_chunk, int32_t *gather_waves, int32_t *gather_batch);
-/* Set the launch configuration: cp_chunk = 1 (one global queue) or >= 64, gather_waves in
+/* Set the launch configuration: cp_chunk = 1 (one global queue, as above) or >= 64, gather_waves in
  * {1, 2, 4}, gather_batch in {2, 4, 8}; a value <= 0 keeps the current one. */
 int pgf_set_tuning(pgf_handle h, int64_t cp_chunk, int32_t gather_waves, int32_t gather_batch);
 

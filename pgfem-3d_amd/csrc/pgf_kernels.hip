@@ -327,10 +327,10 @@ __device__ __forceinline__ void j2_point(const DevMaterial &m, bool plastic, con
 // variable per element, condensed): F(n+1) is always Fr (the model stores (theta/J)^1/3 Fr),
 // tau and c take the element pressure, and the rows get the condensation terms.  Its staged
 // variant runs at three waves per SIMD: at four (128 registers) the extra element terms spill.
-// Bound, on large tet10 meshes, by FP64 issue (half of the cycles) and by the rate at which the
-// staged rows are written (2.9 TB/s), which overlap as far as four workgroups per CU let them: 1.80 ms on
-// 663,552 J2 tet10 (1.75 without the stores, 1.79 with the stores alone).  The staging offsets are
-// loaded with the nodes (a load ahead of every store was 2.20 ms -> 2.00), each wave stages its own
+// Bound, on large tet10 meshes, by FP64 issue (half of the cycles) and by the staged rows' stores,
+// which overlap only as far as four workgroups per CU let them: 1.73 to 1.80 ms on 663,552 J2 tet10, 1.43
+// without the stores, 1.25 without the QP phase, 1.00 with the stores alone (5.1 TB/s).  The staging
+// offsets are loaded with the nodes (a load ahead of every store was 2.20 ms -> 2.00), each wave stages its own
 // rows (no barriers in the transpose: 2.00 -> 1.90), and the QP phase, one wave's, has its node
 // loops unrolled over registers (1.90 -> 1.80; three-field tet10, 93,750: 295 -> 249 us in all).
 // VAR: 0 the displacement element, 1 the three-field element (TF), 2 the displacement
