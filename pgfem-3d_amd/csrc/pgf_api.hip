@@ -1126,10 +1126,8 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
         }
       if (first >= 0) cnt[first] = k;
     }
-    // the columns are the caller's: only rows that share them are read together
-    auto same_columns = [&](int64_t a, int64_t b) {
-      return Ap[b + 1] - Ap[b] == Ap[a + 1] - Ap[a] && std::equal(Ai + Ap[a], Ai + Ap[a + 1], Ai + Ap[b]);
-    };
+    std::vector<uint8_t> like_previous;  // the columns are the caller's: only rows that share them are read together
+    pgf::compare_rows(ndof, Ap, Ai, like_previous);
     std::vector<int4> rows;
     std::vector<int32_t> range;
     rows.reserve(size_t(m.n_nodes));
@@ -1138,7 +1136,7 @@ int pgf_create(const pgf_mesh *mesh, const int64_t *id, int64_t ndof, const int3
       while (d < end) {  // a node's rows; a range's end cuts them
         const int64_t stop = std::min(end, (d / pgf::kRowRange + 1) * pgf::kRowRange);
         int64_t cut = d + 1;
-        while (cut < stop && same_columns(d, cut)) ++cut;
+        while (cut < stop && like_previous[cut]) ++cut;
         if (d % pgf::kRowRange == 0) range.push_back(int32_t(rows.size()));
         rows.push_back(make_int4(int(d), int(cut - d), Ap[d], Ap[d + 1] - Ap[d]));
         d = cut;

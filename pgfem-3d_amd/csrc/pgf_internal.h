@@ -31,6 +31,10 @@ int build_scatter_offsets(const pgf_mesh &m, const int64_t *id, int64_t ndof,
 int build_coel_offsets(const pgf_mesh &m, const int64_t *id, const int32_t *Ap, const int32_t *Ai,
                        std::vector<int64_t> &pair_ptr, std::vector<int16_t> &off);
 
+// like_previous[r] = 1 where CSR row r has the columns of row r - 1, in the same order (pgf_solve reads
+// such rows of a node together).
+void compare_rows(int64_t ndof, const int32_t *Ap, const int32_t *Ai, std::vector<uint8_t> &like_previous);
+
 // Greedy colouring of the interface elements among themselves (they are launched after all
 // volume colours, so they never race with volume elements).
 int color_coels(const pgf_mesh &m, std::vector<int32_t> &color);

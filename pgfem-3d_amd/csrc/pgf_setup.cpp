@@ -171,6 +171,13 @@ int build_coel_offsets(const pgf_mesh &m, const int64_t *id, const int32_t *Ap, 
   return pair_offsets(m.n_coel, m.coel_ptr, m.coel_conn, id, Ap, Ai, pair_ptr, off);
 }
 
+void compare_rows(int64_t ndof, const int32_t *Ap, const int32_t *Ai, std::vector<uint8_t> &like_previous) {
+  like_previous.assign(ndof, 0);
+#pragma omp parallel for schedule(static)
+  for (int64_t r = 1; r < ndof; ++r)
+    like_previous[r] = Ap[r + 1] - Ap[r] == Ap[r] - Ap[r - 1] && std::equal(Ai + Ap[r], Ai + Ap[r + 1], Ai + Ap[r - 1]);
+}
+
 int color_coels(const pgf_mesh &m, std::vector<int32_t> &color) {
   constexpr int kWords = 4;
   std::vector<uint64_t> used(size_t(m.n_nodes) * kWords, 0);
